@@ -436,34 +436,6 @@ __global__ __launch_bounds__(kT) void k_bin_count(Tiles tiles_of, int n, Bins B,
     count_entries(act, tx0, tx1, ty0, ty1, i, n, B, par);
 }
 
-// Exclusive scan of value(k) over tiles k < tiles into out[0..tiles] (out[tiles]
-// = total) by the whole block in LDS: thread t takes a run of tiles.  value
-// is called once per tile, by the thread of its run, in tile order.
-template <class Value>
-__device__ __forceinline__ void block_scan_tiles(int tiles, const Value &value, int *out, int *wsum) {
-    const int per = (tiles + kT - 1) / kT;
-    const int lo = min(int(threadIdx.x) * per, tiles), hi = min(lo + per, tiles);
-    int sum = 0;
-    for (int k = lo; k < hi; ++k) {
-        const int v = value(k);
-        out[k] = sum;
-        sum += v;
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = sum;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += v;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int off = incl - sum;
-    for (int w = 0; w < wave; ++w) off += wsum[w];
-    for (int k = lo; k < hi; ++k) out[k] += off;
-    if (threadIdx.x == kT - 1) out[tiles] = off + sum;
-    __syncthreads();
-}
-
 // Work items of a tile with c entries that had `before` entries in the step
 // before: ceil(c / kT) chunks, or one empty item (which zeroes the tile's
 // nodes) when the tile has just emptied, or none.
@@ -501,7 +473,7 @@ __global__ __launch_bounds__(kT) void k_bin_place(Tiles tiles_of, int n, Bins B,
     int rank[4];
     for (int j = 0; j < 4; ++j) rank[j] = B.rank[int64_t(j) * n + ic];
     if (kLds) {
-        block_scan_tiles(tiles, [&](int k) { return B.count[par][k]; }, sstart, wsum);
+        scan::block_exclusive(tiles, [&](int k) { return B.count[par][k]; }, sstart, wsum);
         if (blockIdx.x == 0)
             for (int k = threadIdx.x; k <= tiles; k += kT) B.start[k] = sstart[k];
         start = sstart;
@@ -544,7 +516,7 @@ __global__ __launch_bounds__(kT) void k_item_place(StencilTiles tiles_of, int n,
     int rank[4];
     for (int j = 0; j < 4; ++j) rank[j] = B.rank[int64_t(j) * n + ic];
     if (kLds) {
-        block_scan_tiles(tiles, [&](int k) {
+        scan::block_exclusive(tiles, [&](int k) {
             const int c = B.count[par][k], before = B.count[par ^ 1][k];
             scount[k] = c;
             return work_items(c, before);
@@ -1900,16 +1872,15 @@ __global__ __launch_bounds__(kT) void k_fluid_update(amh_render R, const FramePa
                                                     LagSlopeMemo *__restrict__ memo,
                                                     const uint64_t *__restrict__ atom_keys) {
     const Frame F = fp->F;
-    __shared__ int lagp[512], slopep[512];
+    __shared__ uint32_t tab[kPerlinTab];
     __shared__ uint64_t wsum[kT / 64];
     __shared__ int32_t choff[kChainLds];
     uint64_t tag = 0;
     if (R.fading == kPerlin) {  // (uniform)
         uint64_t hsum = 0;
+        stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
         for (int i = threadIdx.x; i < 512; i += kT) {
             const int l = R.lag_perm_dev[i], q = R.slope_perm_dev[i];
-            lagp[i] = l;
-            slopep[i] = q;
             hsum += mix64((uint64_t(i) << 32) | uint32_t(l)) + mix64((uint64_t(i + 512) << 32) | uint32_t(q));
         }
         tag = lag_slope_tag(R, hsum, wsum);  // (its barrier also publishes the tables)
@@ -1935,7 +1906,7 @@ __global__ __launch_bounds__(kT) void k_fluid_update(amh_render R, const FramePa
         lag = mm.lag;
         slope = mm.slope;
         if (!(mm.p1 == p1 && mm.tag == tag)) {
-            atom_lag_slope(R, p1, lagp, slopep, lag, slope);
+            atom_lag_slope(R, p1, tab, lag, slope);
             memo[a] = LagSlopeMemo{lag, slope, p1, tag};
         }
     }
@@ -2055,18 +2026,14 @@ __global__ __launch_bounds__(kT) void k_fluid_compose(amh_render R, const FrameP
                                                       const uint32_t *img, const int32_t *mask) {
     const Frame F = fp->F;
     uint32_t *out = fp->out;
-    __shared__ int lagp[512], slopep[512];
-    if (R.keep_background && R.fading == kPerlin) {
-        for (int i = threadIdx.x; i < 512; i += kT) {
-            lagp[i] = R.lag_perm_dev[i];
-            slopep[i] = R.slope_perm_dev[i];
-        }
-    }
+    __shared__ uint32_t tab[kPerlinTab];
+    if (R.keep_background && R.fading == kPerlin)
+        stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
     __syncthreads();
     const int64_t p = int64_t(blockIdx.x) * kT + threadIdx.x;
     if (p >= int64_t(R.width) * R.height) return;
     const int x = int(p % R.width), y = int(p / R.width);
-    const uint32_t bg = R.keep_background ? background(R, F, x, y, lagp, slopep) : 0u;
+    const uint32_t bg = R.keep_background ? background(R, F, x, y, tab) : 0u;
     if (mask[p] != 1) {
         out[p] = bg;
         return;

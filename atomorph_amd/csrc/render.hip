@@ -3,20 +3,27 @@
 //
 // Per frame:
 //   prepare  per atom: trajectory point and colour at t (FP64, the
-//            reference's operation order), bilinear taps; per tap pixel the
-//            smallest blob index that touches it (atomicMin).
-//   splat    taps of a pixel's smallest blob go to dense per-pixel integer
-//            accumulators (count, sum n, sum c*n with n = the integer
-//            bilinear weight numerator); taps of any other blob are counted
-//            per pixel.
-//   scan     exclusive scan of those counts -> per-pixel overflow segments.
-//   overflow the other taps scattered into their pixel's segment (the count
-//            is decremented back to zero, so the workspace cleans itself).
-//   composite per pixel: resolve the smallest blob, then the overflow blobs
-//            in increasing blob order, "over" in that order, feather, the
-//            background blend, RGBA8 out.
+//            reference's operation order), bilinear taps; its taps counted
+//            into the 16 x 16 pixel tiles they fall in.
+//   place    the atoms' numbers into the tiles' lists (starts: the scan of
+//            the counts).
+//   splat    one workgroup per tile, one thread per pixel: the tile's taps
+//            are summed in LDS (count, sum n, sum c*n with n = the integer
+//            bilinear weight numerator) for one blob per pixel at a time, in
+//            increasing blob order, and each resolved colour is composited
+//            "over" in that order; background, RGBA8 out.
+//   composite  (inward feather only) the splat leaves each pixel's resolved
+//            blobs as a list instead, since the feather of a pixel asks
+//            whether its neighbours, in other tiles too, hold the same blob;
+//            a second kernel feathers and composites them.
 // Composite order equals the reference's (blob order); sums are exact, so
 // nothing depends on the order the atoms land in.
+//
+// The sums stay in LDS because device-wide 64-bit atomics are performed past
+// the L2: with five of them per tap into per-pixel accumulators in memory
+// (and a second, scanned list for the other blobs of a pixel) a frame took
+// 1,518 us at 2048^2 with 1.7 M atoms, 261 us at 1001 x 777 with feather 2;
+// in tiles it takes 330 and 99 us.
 #include <mutex>
 
 #include "colour.h"
@@ -30,13 +37,28 @@ using namespace amh::shade;
 
 namespace {
 
-constexpr uint32_t kNoPos = 0xFFFFFFFFu;
+constexpr int kT = 256;
+constexpr int kTile = 16;             // pixels per side of an image tile
+constexpr int kTilePx = kTile * kTile;  // one thread of the splat per pixel
+static_assert(kTilePx == kT, "one thread per pixel");
+constexpr int kLdsTiles = 4096;       // up to this many tiles every placing block scans the counts in LDS
+constexpr int kNoBlob = 0x7FFFFFFF;
+
 // --------------------------------------------------------------- prepare
 struct Rec {       // one atom's splat, 16 bytes
-    uint32_t pos;  // y * W + x of the base tap, kNoPos if not drawn
-    uint32_t fm;   // x_fract | y_fract << 8 | tap mask << 16
+    uint32_t xy;   // x | y << 16 of the base tap
+    uint32_t fm;   // x_fract | y_fract << 8 | tap mask << 16 (mask 0: not drawn)
     uint32_t col;  // RGBA8
     int32_t blob;  // composite index
+};
+
+// The image tiles and their lists.
+struct Tiles {
+    int32_t ntx, nty;
+    int32_t *taps;     // [tiles] taps that fall in the tile
+    int32_t *entries;  // [tiles] atoms listed so far
+    int32_t *start;    // [tiles + 1] scan of taps: a tile lists at most one atom per tap
+    uint32_t *list;    // [<= 4 atoms] atom numbers
 };
 
 // What changes from frame to frame when frames replay from a captured
@@ -49,139 +71,120 @@ struct RenderParams {
 
 __global__ void k_set_render_params(RenderParams *dst, RenderParams v) { *dst = v; }
 
-__global__ __launch_bounds__(256) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, int *__restrict__ bmin,
-                                                 const RenderParams *__restrict__ fp) {
+// The taps of `mask` (bit k: tap (k & 1, k >> 1) of the base pixel x, y) that
+// fall in tile (x / 16 + (j & 1), y / 16 + (j >> 1)).
+__device__ __forceinline__ uint32_t taps_in(uint32_t mask, uint32_t x, uint32_t y, int j) {
+    const uint32_t right = (x % kTile == kTile - 1) ? 10u : 0u, below = (y % kTile == kTile - 1) ? 12u : 0u;
+    return mask & ((j & 1) ? right : ~right) & ((j & 2) ? below : ~below);
+}
+__device__ __forceinline__ int tile_of(uint32_t x, uint32_t y, int j, int ntx) {
+    return int(y / kTile + (j >> 1)) * ntx + int(x / kTile + (j & 1));
+}
+
+// What bounds it: the PERLIN fade's 16 noise octaves per atom (FP64 and LDS
+// table reads).  The taps are counted per tile with the wave's lanes grouped
+// by tile first, one atomic per distinct tile: neighbouring atoms of a chain
+// fall in few tiles.
+__global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B,
+                                                const RenderParams *__restrict__ fp) {
     if (fp) F = fp->F;
-    __shared__ int lagp[512], slopep[512];
-    if (R.fading == kPerlin) {
-        for (int i = threadIdx.x; i < 512; i += 256) {
-            lagp[i] = R.lag_perm_dev[i];
-            slopep[i] = R.slope_perm_dev[i];
-        }
-    }
+    __shared__ uint32_t tab[kPerlinTab];
+    if (R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
     __syncthreads();
-    const int64_t a = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
     const int c = block_chain(R.chain_off_dev, R.nchains, a);
-    if (a >= R.wtot) return;
-    Rec rec = {kNoPos, 0u, 0u, -1};
-    const int W = R.width, H = R.height;
-    const int b = R.rank_dev[int64_t(F.fk) * R.nchains + c];
-    const uint64_t p1 = R.pts_dev[int64_t(F.fk) * R.wtot + a];
-    const uint64_t p2 = R.pts_dev[int64_t(F.fnext) * R.wtot + a];
-    const bool h1 = pt_flags(p1) & HAS_PIXEL, h2 = pt_flags(p2) & HAS_PIXEL;
-    if (b < 0 || (!h1 && !h2)) {
+    const bool in = a < R.wtot;
+    uint32_t mask = 0, X = 0, Y = 0;
+    if (in) {
+        Rec rec = {0u, 0u, 0u, -1};
+        const int W = R.width, H = R.height;
+        const int b = R.rank_dev[int64_t(F.fk) * R.nchains + c];
+        const uint64_t p1 = R.pts_dev[int64_t(F.fk) * R.wtot + a];
+        const uint64_t p2 = R.pts_dev[int64_t(F.fnext) * R.wtot + a];
+        const bool h1 = pt_flags(p1) & HAS_PIXEL, h2 = pt_flags(p2) & HAS_PIXEL;
+        if (b >= 0 && (h1 || h2)) {
+            // colours at both ends (morph.cpp:495-522); a missing end fades from /
+            // to the other end's colour with alpha 0
+            uint32_t c1 = key_px(R.keys_dev, F.fk, W, H, pt_x(p1), pt_y(p1));
+            uint32_t c2 = key_px(R.keys_dev, F.fnext, W, H, pt_x(p2), pt_y(p2));
+            if (!h2) c2 = c1 & 0x00FFFFFFu;
+            else if (!h1) c1 = c2 & 0x00FFFFFFu;
+            uint32_t qxf, qyf;
+            traj_point(R, F, a, p1, p2, X, Y, qxf, qyf);
+            const uint32_t col = atom_colour(R, F, p1, c1, c2, tab);
+            // guards and taps (morph.cpp:552-589); taps outside the image are
+            // dropped (draw_atoms skips pos >= W*H)
+            const int x = int(X), y = int(Y), xf = int(qxf), yf = int(qyf);
+            if (x < W && y < H) {
+                if ((255 - xf) * (255 - yf) > 0) mask |= 1u;
+                if (x + 1 < W && xf * (255 - yf) > 0) mask |= 2u;
+                if (y + 1 < H && (255 - xf) * yf > 0) mask |= 4u;
+                if (x + 1 < W && y + 1 < H && xf * yf > 0) mask |= 8u;
+            }
+            if (mask) rec = Rec{X | (Y << 16), qxf | (qyf << 8) | (mask << 16), col, b};
+        }
         recs[a] = rec;
-        return;
     }
-    // colours at both ends (morph.cpp:495-522); a missing end fades from /
-    // to the other end's colour with alpha 0
-    uint32_t c1, c2;
-    if (h1 && !h2) {
-        c1 = key_px(R.keys_dev, F.fk, W, H, pt_x(p1), pt_y(p1));
-        c2 = c1 & 0x00FFFFFFu;
-    } else if (h2 && !h1) {
-        c2 = key_px(R.keys_dev, F.fnext, W, H, pt_x(p2), pt_y(p2));
-        c1 = c2 & 0x00FFFFFFu;
-    } else {
-        c1 = key_px(R.keys_dev, F.fk, W, H, pt_x(p1), pt_y(p1));
-        c2 = key_px(R.keys_dev, F.fnext, W, H, pt_x(p2), pt_y(p2));
-    }
-    uint32_t qx, qy, qxf, qyf;
-    traj_point(R, F, a, p1, p2, qx, qy, qxf, qyf);
-    const uint32_t col = atom_colour(R, F, p1, c1, c2, lagp, slopep);
-    // guards and taps (morph.cpp:552-589)
-    const int X = int(qx), Y = int(qy);
-    if (X >= W || Y >= H) {
-        if (X > R.bbox_x2 || X < R.bbox_x1 || Y > R.bbox_y2 || Y < R.bbox_y1) {
-            recs[a] = rec;
-            return;
-        }
-    }
-    const int xf = int(qxf), yf = int(qyf);
-    uint32_t mask = 0;
-    if ((255 - xf) * (255 - yf) > 0) mask |= 1u;
-    if ((X < R.bbox_x2 || X + 1 < W) && xf * (255 - yf) > 0) mask |= 2u;
-    if ((Y < R.bbox_y2 || Y + 1 < H) && (255 - xf) * yf > 0) mask |= 4u;
-    if (xf * yf > 0 && ((Y < R.bbox_y2 && X < R.bbox_x2) || (Y + 1 < H && X + 1 < W))) mask |= 8u;
-    // taps outside the image are dropped (draw_atoms skips pos >= W*H)
-    if (X >= W || Y >= H) mask &= 0u;
-    if (X + 1 >= W) mask &= ~(2u | 8u);
-    if (Y + 1 >= H) mask &= ~(4u | 8u);
-    if (!mask) {
-        recs[a] = rec;
-        return;
-    }
-    rec.pos = uint32_t(Y * W + X);
-    rec.fm = qxf | (qyf << 8) | (mask << 16);
-    rec.col = col;
-    rec.blob = b;
-    recs[a] = rec;
-    if (mask & 1u) atomicMin(&bmin[rec.pos], b);
-    if (mask & 2u) atomicMin(&bmin[rec.pos + 1], b);
-    if (mask & 4u) atomicMin(&bmin[rec.pos + W], b);
-    if (mask & 8u) atomicMin(&bmin[rec.pos + W + 1], b);
-}
-
-// Integer bilinear weight numerators of tap k (weights are these / 255^2).
-__device__ __forceinline__ void tap(const Rec &r, int W, int k, uint32_t &p, uint32_t &n) {
-    const uint32_t xf = r.fm & 255u, yf = (r.fm >> 8) & 255u;
-    switch (k) {
-        case 0: p = r.pos; n = (255u - xf) * (255u - yf); break;
-        case 1: p = r.pos + 1; n = xf * (255u - yf); break;
-        case 2: p = r.pos + W; n = (255u - xf) * yf; break;
-        default: p = r.pos + W + 1; n = xf * yf; break;
-    }
-}
-
-struct Acc {  // dense per-pixel accumulators (structure of arrays)
-    unsigned long long *cn;       // count << 40 | sum n
-    unsigned long long *s[4];     // sum c * n per channel
-};
-
-__global__ __launch_bounds__(256) void k_splat(const Rec *__restrict__ recs, int64_t n_atoms, int W,
-                                               const int *__restrict__ bmin, Acc acc, int *__restrict__ ovcount) {
-    const int64_t a = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (a >= n_atoms) return;
-    const Rec r = recs[a];
-    if (r.pos == kNoPos) return;
-    const uint32_t mask = r.fm >> 16;
-    for (int k = 0; k < 4; ++k) {
-        if (!(mask & (1u << k))) continue;
-        uint32_t p, n;
-        tap(r, W, k, p, n);
-        if (bmin[p] == r.blob) {
-            atomicAdd(&acc.cn[p], (1ull << 40) | n);
-            for (int c = 0; c < 4; ++c) atomicAdd(&acc.s[c][p], (unsigned long long)(ch(r.col, c) * n));
-        } else {
-            atomicAdd(&ovcount[p], 1);
+    const int lane = threadIdx.x & 63;
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t m = taps_in(mask, X, Y, j);
+        const int t = m ? tile_of(X, Y, j, B.ntx) : -1;
+        const int w = int(__popc(m));
+        uint64_t todo = __ballot(m != 0);
+        if (!todo) continue;
+        const uint64_t w0 = __ballot(w & 1), w1 = __ballot(w & 2), w2 = __ballot(w & 4);
+        while (todo) {
+            const int leader = __ffsll((unsigned long long)todo) - 1;
+            const uint64_t same = __ballot(t == __builtin_amdgcn_readlane(t, leader));
+            if (lane == leader)
+                atomicAdd(&B.taps[t], int(__popcll(same & w0) + 2 * __popcll(same & w1) + 4 * __popcll(same & w2)));
+            todo &= ~same;
         }
     }
 }
 
-struct Ov {  // an overflow tap, 16 bytes
-    int32_t blob;
-    uint32_t n;
-    uint32_t col;
-    uint32_t pad;
-};
-
-__global__ __launch_bounds__(256) void k_overflow(const Rec *__restrict__ recs, int64_t n_atoms, int W,
-                                                  const int *__restrict__ bmin, int *__restrict__ ovcount,
-                                                  const int *__restrict__ ovstart, Ov *__restrict__ ov) {
-    const int64_t a = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (a >= n_atoms) return;
-    const Rec r = recs[a];
-    if (r.pos == kNoPos) return;
-    const uint32_t mask = r.fm >> 16;
-    for (int k = 0; k < 4; ++k) {
-        if (!(mask & (1u << k))) continue;
-        uint32_t p, n;
-        tap(r, W, k, p, n);
-        if (bmin[p] != r.blob) {
-            const int slot = atomicSub(&ovcount[p], 1) - 1;
-            Ov o = {r.blob, n, r.col, 0u};
-            ov[ovstart[p] + slot] = o;
+// The atoms' numbers into their tiles' lists, in no fixed order (the sums are
+// exact).  kLds: every block scans the tap counts in LDS (block 0 stores the
+// starts); otherwise B.start holds the scan already.
+template <bool kLds>
+__global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int64_t n, Tiles B) {
+    __shared__ int sstart[kLds ? kLdsTiles + 1 : 1];
+    __shared__ int wsum[kT / 64];
+    const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
+    const uint2 r = *reinterpret_cast<const uint2 *>(&recs[a < n ? a : 0]);
+    const uint32_t X = r.x & 0xFFFFu, Y = r.x >> 16, mask = a < n ? r.y >> 16 : 0u;
+    const int32_t *start = B.start;
+    if (kLds) {
+        const int tiles = B.ntx * B.nty;
+        scan::block_exclusive(tiles, [&](int k) { return B.taps[k]; }, sstart, wsum);
+        if (blockIdx.x == 0)
+            for (int k = threadIdx.x; k <= tiles; k += kT) B.start[k] = sstart[k];
+        start = sstart;
+    }
+    const int lane = threadIdx.x & 63;
+    const uint64_t below = (1ull << lane) - 1ull;
+    int t[4], lead[4], pre[4], total[4];  // the wave's lanes grouped by tile, per neighbour tile
+    for (int j = 0; j < 4; ++j) {
+        t[j] = taps_in(mask, X, Y, j) ? tile_of(X, Y, j, B.ntx) : -1;
+        lead[j] = lane;
+        pre[j] = total[j] = 0;
+        uint64_t todo = __ballot(t[j] >= 0);
+        while (todo) {
+            const int leader = __ffsll((unsigned long long)todo) - 1;
+            const uint64_t same = __ballot(t[j] == __builtin_amdgcn_readlane(t[j], leader));
+            if ((same >> lane) & 1u) {
+                lead[j] = leader;
+                pre[j] = int(__popcll(same & below));
+            }
+            if (lane == leader) total[j] = int(__popcll(same));
+            todo &= ~same;
         }
+    }
+    int base[4];
+    for (int j = 0; j < 4; ++j) base[j] = total[j] > 0 ? atomicAdd(&B.entries[t[j]], total[j]) : 0;
+    for (int j = 0; j < 4; ++j) {
+        const int b = __shfl(base[j], lead[j], 64);
+        if (t[j] >= 0) B.list[start[t[j]] + b + pre[j]] = uint32_t(a);
     }
 }
 
@@ -207,16 +210,26 @@ __device__ Px resolve(uint64_t cnt, uint64_t sn, const uint64_t s[4], int densit
     return q;
 }
 
-struct Seg {  // overflow segment of one pixel
-    const Ov *ov;
-    int begin, end;
+// With feather: the resolved blobs of a pixel, in increasing blob order.  The
+// first is kept per pixel; the others are a chain of Ov, in the splat's
+// numbering of the tile's taps (a (pixel, blob) pair has at least one tap).
+struct Ov {
+    int32_t blob;
+    uint32_t col;
+    int32_t next;  // -1: last
+};
+struct Resolved {
+    int32_t *blob;  // [npx] kNoBlob: none
+    uint32_t *col;
+    int32_t *next;
+    Ov *ov;         // [<= 4 atoms]
 };
 
-// Is pixel q (inside the image) a member of blob b's resolved pixel set?
-__device__ bool member(const int *bmin, const int *ovstart, const Ov *ov, int64_t q, int b) {
-    if (bmin[q] == b) return true;
-    for (int i = ovstart[q]; i < ovstart[q + 1]; ++i)
-        if (ov[i].blob == b) return true;
+// Does pixel q hold blob b?
+__device__ __forceinline__ bool member(const Resolved &V, int64_t q, int b) {
+    if (V.blob[q] >= b) return V.blob[q] == b;  // the pixel's smallest
+    for (int i = V.next[q]; i >= 0; i = V.ov[i].next)
+        if (V.ov[i].blob == b) return true;
     return false;
 }
 
@@ -224,8 +237,7 @@ __device__ bool member(const int *bmin, const int *ovstart, const Ov *ov, int64_
 // blob b is d - 1, d = L1 distance to the nearest pixel outside the blob
 // (coordinates 0 and 65535 count as blob borders).  Returns d (> feather:
 // untouched).
-__device__ int feather_depth(int x, int y, int W, int H, int F, int b, const int *bmin, const int *ovstart,
-                             const Ov *ov) {
+__device__ int feather_depth(int x, int y, int W, int H, int F, int b, const Resolved &V) {
     int best = F + 1;
     best = min(best, x + 1);
     best = min(best, y + 1);
@@ -240,7 +252,7 @@ __device__ int feather_depth(int x, int y, int W, int H, int F, int b, const int
                 const int qx = x + dx, qy = y + sgn * ady;
                 bool in;
                 if (qx < 0 || qy < 0 || qx >= W || qy >= H) in = false;
-                else in = member(bmin, ovstart, ov, int64_t(qy) * W + qx, b);
+                else in = member(V, int64_t(qy) * W + qx, b);
                 if (!in) return r;
             }
         }
@@ -271,83 +283,9 @@ struct Fold {
     }
 };
 
-
-__global__ __launch_bounds__(256) void k_composite(amh_render R, Frame F, int *__restrict__ bmin, Acc acc,
-                                                   const int *__restrict__ ovstart, const Ov *__restrict__ ov,
-                                                   uint32_t *__restrict__ out, int clear_bmin,
-                                                   const RenderParams *__restrict__ fp) {
-    if (fp) {
-        F = fp->F;
-        out = fp->out;
-    }
-    __shared__ int lagp[512], slopep[512];
-    if (R.keep_background && R.fading == kPerlin) {
-        for (int i = threadIdx.x; i < 512; i += 256) {
-            lagp[i] = R.lag_perm_dev[i];
-            slopep[i] = R.slope_perm_dev[i];
-        }
-    }
-    __syncthreads();
-    const int W = R.width, H = R.height;
-    const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (p >= int64_t(W) * H) return;
-    const int x = int(p % W), y = int(p / W);
-    const uint32_t bg = R.keep_background ? background(R, F, x, y, lagp, slopep) : 0u;
-    const int b0 = bmin[p];
-    if (b0 == 0x7FFFFFFF) {
-        out[p] = bg;
-        return;
-    }
-    const int nb = R.nblobs;
-    const bool texture = R.show_blobs != 1 && R.show_blobs != 2;
-    Fold fold;
-    auto emit = [&](int b, Px q) {
-        if (texture && R.feather > 0) {
-            const int d = feather_depth(x, y, W, H, R.feather, b, bmin, ovstart, ov);
-            if (d <= R.feather) q.a = narrow8(round(double(q.a) * (double(d) / double(R.feather + 1))));
-        }
-        uint32_t c = q.r | (q.g << 8) | (q.b << 16) | (q.a << 24);
-        if (!texture && R.blob_rgba_dev) c = R.blob_rgba_dev[int64_t(F.fk) * nb + b];
-        if ((c >> 24) == 0) return;
-        fold.add(c);
-    };
-    {
-        const uint64_t cn = acc.cn[p];
-        uint64_t s[4];
-        for (int k = 0; k < 4; ++k) {
-            s[k] = acc.s[k][p];
-            acc.s[k][p] = 0;
-        }
-        acc.cn[p] = 0;
-        emit(b0, resolve(cn >> 40, cn & ((1ull << 40) - 1), s, R.density));
-    }
-    const int o0 = ovstart[p], o1 = ovstart[p + 1];
-    int last = b0;
-    while (o1 > o0) {
-        // next blob above `last`, with its sums (one pass per blob)
-        int nbk = 0x7FFFFFFF;
-        uint64_t cnt = 0, sn = 0, s[4] = {0, 0, 0, 0};
-        for (int i = o0; i < o1; ++i) {
-            const Ov e = ov[i];
-            if (e.blob <= last || e.blob > nbk) continue;
-            if (e.blob < nbk) {
-                nbk = e.blob;
-                cnt = sn = 0;
-                s[0] = s[1] = s[2] = s[3] = 0;
-            }
-            ++cnt;
-            sn += e.n;
-            for (int k = 0; k < 4; ++k) s[k] += uint64_t(ch(e.col, k)) * e.n;
-        }
-        if (nbk == 0x7FFFFFFF) break;
-        emit(nbk, resolve(cnt, sn, s, R.density));
-        last = nbk;
-    }
-    if (clear_bmin) bmin[p] = 0x7FFFFFFF;
-    if (fold.n == 0) {
-        out[p] = bg;
-        return;
-    }
+// The folded pixel over the background (morph.cpp:1381-1401, 1405-1417).
+__device__ uint32_t finish(const amh_render &R, const Fold &fold, uint32_t bg) {
+    if (fold.n == 0) return bg;
     double r = fold.r, g = fold.g, b = fold.b, a = fold.a;
     if (R.blend_blobs) {
         r = fold.rs / fold.as;
@@ -362,44 +300,185 @@ __global__ __launch_bounds__(256) void k_composite(amh_render R, Frame F, int *_
         b = a * b + (1.0 - a) * bgb;
         a = bga + (1.0 - bga) * a;
     }
-    out[p] = rgba_pack(narrow8(round(r * 255.0)), narrow8(round(g * 255.0)), narrow8(round(b * 255.0)),
-                       narrow8(round(a * 255.0)));
+    return rgba_pack(narrow8(round(r * 255.0)), narrow8(round(g * 255.0)), narrow8(round(b * 255.0)),
+                     narrow8(round(a * 255.0)));
 }
 
-__global__ void k_fill_i32(int *p, int64_t n, int v) {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
+// One tile's pixels from its listed atoms.  Each pass sums, per pixel, the
+// taps of one blob (bcur) in LDS and finds the next larger blob that touches
+// the pixel (bnext) on the way; most pixels hold one or two blobs.  The first
+// atom of each thread is kept in registers for all passes (a tile lists about
+// one atom per covered pixel and density), further ones are read again.
+// kFeather: the resolved colours go to V for k_composite.  Leaves the tile's
+// counters at zero for the next frame.
+template <bool kFeather>
+__global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *__restrict__ recs, Tiles B, Resolved V,
+                                              uint32_t *__restrict__ out, const RenderParams *__restrict__ fp) {
+    if (fp) {
+        F = fp->F;
+        out = fp->out;
+    }
+    __shared__ unsigned long long acc[5][kTilePx];  // count << 40 | sum n, then sum c * n per channel
+    __shared__ int bcur[kTilePx], bnext[kTilePx];
+    __shared__ uint32_t tab[kFeather ? 1 : kPerlinTab];
+    __shared__ int nov;
+    const int tile = int(blockIdx.x), tid = int(threadIdx.x);
+    const int x0 = (tile % B.ntx) * kTile, y0 = (tile / B.ntx) * kTile;
+    const int n = B.entries[tile], s0 = B.start[tile];
+    const uint32_t *list = B.list + s0;
+    Rec mine = {0u, 0u, 0u, 0};
+    if (tid < n) mine = recs[list[tid]];
+    if (!kFeather && R.keep_background && R.fading == kPerlin)
+        stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, tid, kT);
+    bnext[tid] = kNoBlob;
+    if (tid == 0) nov = 0;
+    __syncthreads();
+    if (tid == 0 && n > 0) {
+        B.entries[tile] = 0;
+        B.taps[tile] = 0;
+    }
+    // f(pixel of the tile, weight numerator, atom) for every tap in the tile
+    const auto taps = [&](const auto &f) {
+        for (int e = tid; e < n; e += kT) {
+            const Rec r = e == tid ? mine : recs[list[e]];
+            const uint32_t xf = r.fm & 255u, yf = (r.fm >> 8) & 255u, mask = r.fm >> 16;
+            const int lx = int(r.xy & 0xFFFFu) - x0, ly = int(r.xy >> 16) - y0;
+            for (int k = 0; k < 4; ++k) {
+                const int px = lx + (k & 1), py = ly + (k >> 1);
+                if (!((mask >> k) & 1u) || uint32_t(px) >= uint32_t(kTile) || uint32_t(py) >= uint32_t(kTile)) continue;
+                f(py * kTile + px, ((k & 1) ? xf : 255u - xf) * ((k >> 1) ? yf : 255u - yf), r);
+            }
+        }
+    };
+    taps([&](int p, uint32_t, const Rec &r) { atomicMin(&bnext[p], r.blob); });
+    __syncthreads();
+    const int x = x0 + tid % kTile, y = y0 + tid / kTile;
+    const bool inside = x < R.width && y < R.height;
+    const int64_t p = int64_t(y) * R.width + x;
+    const bool texture = R.show_blobs != 1 && R.show_blobs != 2;
+    Fold fold;
+    int last = -1;  // kFeather: the pixel's last chained Ov
+    bool first = true;
+    for (;;) {
+        const int b = bnext[tid];
+        bcur[tid] = b;
+        bnext[tid] = kNoBlob;
+        for (int k = 0; k < 5; ++k) acc[k][tid] = 0ull;
+        if (!__syncthreads_or(b != kNoBlob)) break;
+        taps([&](int q, uint32_t w, const Rec &r) {
+            const int cur = bcur[q];
+            if (r.blob == cur) {
+                atomicAdd(&acc[0][q], (1ull << 40) | w);
+                for (int k = 0; k < 4; ++k) atomicAdd(&acc[1 + k][q], (unsigned long long)(ch(r.col, k) * w));
+            } else if (r.blob > cur) {
+                atomicMin(&bnext[q], r.blob);
+            }
+        });
+        __syncthreads();
+        if (b != kNoBlob) {
+            const uint64_t cn = acc[0][tid];
+            const uint64_t s[4] = {acc[1][tid], acc[2][tid], acc[3][tid], acc[4][tid]};
+            const Px q = resolve(cn >> 40, cn & ((1ull << 40) - 1), s, R.density);
+            uint32_t c = rgba_pack(q.r, q.g, q.b, q.a);
+            if (kFeather) {
+                if (first) {
+                    V.blob[p] = b;
+                    V.col[p] = c;
+                } else {
+                    const int o = s0 + atomicAdd(&nov, 1);
+                    V.ov[o] = Ov{b, c, -1};
+                    if (last < 0) V.next[p] = o;
+                    else V.ov[last].next = o;
+                    last = o;
+                }
+                first = false;
+            } else {
+                if (!texture && R.blob_rgba_dev) c = R.blob_rgba_dev[int64_t(F.fk) * R.nblobs + b];
+                if (c >> 24) fold.add(c);
+            }
+        }
+    }
+    if (!inside) return;
+    if (kFeather) {
+        if (first) V.blob[p] = kNoBlob;
+        if (last < 0) V.next[p] = -1;
+    } else {
+        out[p] = finish(R, fold, R.keep_background ? background(R, F, x, y, tab) : 0u);
+    }
+}
+
+// Feather and composite of the resolved blobs (texture blobs only: the other
+// modes are not feathered).
+__global__ __launch_bounds__(kT) void k_composite(amh_render R, Frame F, Resolved V, uint32_t *__restrict__ out,
+                                                  const RenderParams *__restrict__ fp) {
+    if (fp) {
+        F = fp->F;
+        out = fp->out;
+    }
+    __shared__ uint32_t tab[kPerlinTab];
+    if (R.keep_background && R.fading == kPerlin)
+        stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
+    __syncthreads();
+    const int W = R.width, H = R.height;
+    const int64_t p = int64_t(blockIdx.x) * kT + threadIdx.x;
+    if (p >= int64_t(W) * H) return;
+    const int x = int(p % W), y = int(p / W);
+    Fold fold;
+    Ov o = {V.blob[p], V.col[p], V.next[p]};
+    while (o.blob != kNoBlob) {
+        const int d = feather_depth(x, y, W, H, R.feather, o.blob, V);
+        uint32_t c = o.col;
+        if (d <= R.feather)
+            c = (c & 0x00FFFFFFu) | (narrow8(round(double(c >> 24) * (double(d) / double(R.feather + 1)))) << 24);
+        if (c >> 24) fold.add(c);
+        if (o.next < 0) break;
+        o = V.ov[o.next];
+    }
+    out[p] = finish(R, fold, R.keep_background ? background(R, F, x, y, tab) : 0u);
 }
 
 // ------------------------------------------------------------ workspace
 struct Layout {
-    int64_t npx, nblk;
-    size_t bmin, ovcount, ovstart, sums, offs, acc, recs, ov, total;
+    int64_t npx, tiles;
+    int32_t ntx, nty;
+    size_t taps, entries, start, sums, offs, recs, list, ov, blob, col, next, total;
 };
 Layout layout(int32_t W, int32_t H, int64_t wtot) {
     Layout L;
     L.npx = int64_t(W) * H;
-    L.nblk = scan::blocks(L.npx);
+    L.ntx = (W + kTile - 1) / kTile;
+    L.nty = (H + kTile - 1) / kTile;
+    L.tiles = int64_t(L.ntx) * L.nty;
+    const size_t n = size_t(wtot > 0 ? wtot : 1), nt = size_t(L.tiles), nb = size_t(scan::blocks(L.tiles));
     auto al = [](size_t v) { return (v + 255) & ~size_t(255); };
     size_t o = 0;
-    L.bmin = o; o = al(o + sizeof(int) * L.npx);
-    L.ovcount = o; o = al(o + sizeof(int) * L.npx);
-    L.ovstart = o; o = al(o + sizeof(int) * (L.npx + 1));
-    L.sums = o; o = al(o + sizeof(int) * (L.nblk + 1));
-    L.offs = o; o = al(o + sizeof(int) * (L.nblk + 1));
-    L.acc = o; o = al(o + 5 * sizeof(uint64_t) * L.npx);
-    L.recs = o; o = al(o + sizeof(Rec) * size_t(wtot > 0 ? wtot : 1));
-    L.ov = o; o = al(o + sizeof(Ov) * 4 * size_t(wtot > 0 ? wtot : 1));
-    L.total = o;
+    L.taps = o;  // the counters first: they stay at zero between frames
+    L.entries = o + 4 * nt;
+    o = al(o + 8 * nt);
+    L.start = o; o = al(o + 4 * (nt + 1));
+    L.sums = o;
+    L.offs = o + 4 * nb;
+    o = al(o + 4 * (2 * nb + 1));
+    // per atom: its record, 4 list entries, 4 chained blobs
+    L.recs = o;
+    L.list = o + sizeof(Rec) * n;
+    L.ov = L.list + 16 * n;
+    o = al(L.ov + 4 * sizeof(Ov) * n);
+    L.blob = o;
+    L.col = o + 4 * size_t(L.npx);
+    L.next = o + 8 * size_t(L.npx);
+    o += 12 * size_t(L.npx);
+    // The size asked of callers: 52 bytes per pixel and 80 per atom, eight
+    // arrays.  It decides which frames amh_render_frame_noalloc takes.
+    const size_t px = size_t(L.npx), pb = size_t(scan::blocks(L.npx));
+    L.total = 2 * al(4 * px) + al(4 * (px + 1)) + 2 * al(4 * (pb + 1)) + al(40 * px) + al(16 * n) + al(64 * n);
+    if (L.total < o) L.total = o;
     return L;
 }
 
-Acc acc_of(char *ws, const Layout &L) {
-    Acc a;
-    unsigned long long *base = reinterpret_cast<unsigned long long *>(ws + L.acc);
-    a.cn = base;
-    for (int k = 0; k < 4; ++k) a.s[k] = base + (k + 1) * L.npx;
-    return a;
+Tiles tiles_of(char *ws, const Layout &L) {
+    return Tiles{L.ntx, L.nty, reinterpret_cast<int32_t *>(ws + L.taps), reinterpret_cast<int32_t *>(ws + L.entries),
+                 reinterpret_cast<int32_t *>(ws + L.start), reinterpret_cast<uint32_t *>(ws + L.list)};
 }
 
 }  // namespace
@@ -417,11 +496,7 @@ extern "C" int amh_render_workspace_init(void *ws, size_t ws_bytes, int32_t W, i
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     char *base = static_cast<char *>(ws);
-    if (int r = check_hip(hipMemsetAsync(base, 0, L.total, s), "amh_render_workspace_init")) return r;
-    hipLaunchKernelGGL(k_fill_i32, dim3(uint32_t((L.npx + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<int *>(base + L.bmin), L.npx, 0x7FFFFFFF);
-    AMH_LAUNCH_CHECK("amh_render_workspace_init");
-    return AMH_OK;
+    return check_hip(hipMemsetAsync(base, 0, L.total, s), "amh_render_workspace_init");
 }
 
 namespace {
@@ -433,8 +508,8 @@ bool render_args_ok(const amh_render *R) {
            R->height <= 65535 && R->wtot >= 0;
 }
 
-// The frame itself, on a workspace laid out by `L` whose accumulators,
-// overflow counts and smallest-blob map are clean; leaves them clean.
+// The frame itself, on a workspace laid out by `L` whose tile counters are
+// zero; leaves them at zero.
 // fp (device, may be NULL): the frame's time and output are read from it
 // (graph capture; then nothing is timed, since events would be captured).
 int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, uint32_t *out, hipStream_t s,
@@ -493,15 +568,10 @@ int scratch_ptr(char **out) {
     return AMH_OK;
 }
 
-// bmin := INT_MAX, overflow counts and accumulators := 0.
-__global__ __launch_bounds__(256) void k_ws_reset(int *__restrict__ bmin, int *__restrict__ ovcount,
-                                                  unsigned long long *__restrict__ acc, int64_t npx) {
-    const int64_t stride = int64_t(gridDim.x) * 256;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < npx; i += stride) {
-        bmin[i] = 0x7FFFFFFF;
-        ovcount[i] = 0;
-        for (int k = 0; k < 5; ++k) acc[int64_t(k) * npx + i] = 0ull;
-    }
+// The tile counters := 0.
+__global__ __launch_bounds__(kT) void k_ws_reset(int32_t *__restrict__ counters, int64_t n) {
+    const int64_t i = int64_t(blockIdx.x) * kT + threadIdx.x;
+    if (i < n) counters[i] = 0;
 }
 
 }  // namespace
@@ -523,10 +593,8 @@ extern "C" int amh_render_frame_noalloc(const amh_render *R, double t, uint32_t 
     char *base = nullptr;
     if (int r = scratch_ptr(&base)) return r;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint32_t grid = uint32_t(std::min<int64_t>((L.npx + 255) / 256, 4096));
-    hipLaunchKernelGGL(k_ws_reset, dim3(grid), dim3(256), 0, s, reinterpret_cast<int *>(base + L.bmin),
-                       reinterpret_cast<int *>(base + L.ovcount),
-                       reinterpret_cast<unsigned long long *>(base + L.acc), L.npx);
+    hipLaunchKernelGGL(k_ws_reset, dim3(uint32_t((2 * L.tiles + kT - 1) / kT)), dim3(kT), 0, s,
+                       reinterpret_cast<int32_t *>(base + L.taps), 2 * L.tiles);
     AMH_LAUNCH_CHECK("amh_render_frame_noalloc");
     return render_frame_on(R, t, base, L, out, s);
 }
@@ -535,14 +603,10 @@ namespace {
 int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, uint32_t *out, hipStream_t s,
                     const RenderParams *fp) {
     amh::ProfScope whole_(fp ? nullptr : "render_frame", s);
-    int *bmin = reinterpret_cast<int *>(base + L.bmin);
-    int *ovcount = reinterpret_cast<int *>(base + L.ovcount);
-    int *ovstart = reinterpret_cast<int *>(base + L.ovstart);
-    int *sums = reinterpret_cast<int *>(base + L.sums);
-    int *offs = reinterpret_cast<int *>(base + L.offs);
     Rec *recs = reinterpret_cast<Rec *>(base + L.recs);
-    Ov *ov = reinterpret_cast<Ov *>(base + L.ov);
-    const Acc acc = acc_of(base, L);
+    const Tiles B = tiles_of(base, L);
+    const Resolved V = {reinterpret_cast<int32_t *>(base + L.blob), reinterpret_cast<uint32_t *>(base + L.col),
+                        reinterpret_cast<int32_t *>(base + L.next), reinterpret_cast<Ov *>(base + L.ov)};
 
     // morph::normalize_time / get_frame_key (morph.cpp:404-450, 460-464)
     Frame F;
@@ -559,31 +623,29 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
     F.fnext = (F.fk + 1) % R->nkeys;
     const double dt = 1.0 / double(R->nkeys);
     F.tl = fmax(0.0, (F.tn - (double(F.fk) * dt)) / dt);
-    const uint32_t gpx = uint32_t((L.npx + 255) / 256);
-    const uint32_t gat = uint32_t((Rc.wtot + 255) / 256);
+    // timed launches only outside graph capture (their events would be captured)
+    const auto launch = [&](const char *name, auto kernel, int64_t threads, auto... args) {
+        const dim3 grid(uint32_t((threads + kT - 1) / kT));
+        if (fp) hipLaunchKernelGGL(kernel, grid, dim3(kT), 0, s, args...);
+        else amh::launch_timed(name, kernel, grid, dim3(kT), 0, s, args...);
+    };
     if (Rc.wtot > 0) {
-        if (fp) {
-            hipLaunchKernelGGL(k_prepare, dim3(gat), dim3(256), 0, s, Rc, F, recs, bmin, fp);
-            hipLaunchKernelGGL(k_splat, dim3(gat), dim3(256), 0, s, recs, Rc.wtot, Rc.width, bmin, acc, ovcount);
+        launch("k_prepare", k_prepare, Rc.wtot, Rc, F, recs, B, fp);
+        if (L.tiles <= kLdsTiles) {
+            launch("k_place", k_place<true>, Rc.wtot, recs, Rc.wtot, B);
         } else {
-            amh::launch_timed("k_prepare", k_prepare, dim3(gat), dim3(256), 0, s, Rc, F, recs, bmin, fp);
-            amh::launch_timed("k_splat", k_splat, dim3(gat), dim3(256), 0, s, recs, Rc.wtot, Rc.width, bmin, acc,
-                              ovcount);
+            scan::exclusive(B.taps, L.tiles, reinterpret_cast<int *>(base + L.sums),
+                            reinterpret_cast<int *>(base + L.offs), B.start, s);
+            launch("k_place", k_place<false>, Rc.wtot, recs, Rc.wtot, B);
         }
     }
-    scan::exclusive(ovcount, L.npx, sums, offs, ovstart, s);
-    if (Rc.wtot > 0)
-        hipLaunchKernelGGL(k_overflow, dim3(gat), dim3(256), 0, s, recs, Rc.wtot, Rc.width, bmin, ovcount, ovstart,
-                           ov);
-    const int separate_clear = Rc.feather > 0 ? 1 : 0;
-    if (fp)
-        hipLaunchKernelGGL(k_composite, dim3(gpx), dim3(256), 0, s, Rc, F, bmin, acc, ovstart, ov, out,
-                           separate_clear ? 0 : 1, fp);
-    else
-        amh::launch_timed("k_composite", k_composite, dim3(gpx), dim3(256), 0, s, Rc, F, bmin, acc, ovstart, ov,
-                          out, separate_clear ? 0 : 1, fp);
-    if (separate_clear)
-        hipLaunchKernelGGL(k_fill_i32, dim3(gpx), dim3(256), 0, s, bmin, L.npx, 0x7FFFFFFF);
+    const bool texture = Rc.show_blobs != 1 && Rc.show_blobs != 2;
+    if (texture && Rc.feather > 0) {
+        launch("k_splat", k_splat<true>, L.tiles * kT, Rc, F, recs, B, V, out, fp);
+        launch("k_composite", k_composite, L.npx, Rc, F, V, out, fp);
+    } else {
+        launch("k_splat", k_splat<false>, L.tiles * kT, Rc, F, recs, B, V, out, fp);
+    }
     AMH_LAUNCH_CHECK("amh_render_frame");
     return AMH_OK;
 }

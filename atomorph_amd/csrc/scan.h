@@ -115,6 +115,36 @@ __global__ __launch_bounds__(256) void k_blk_apply_fold(const int *__restrict__ 
     if (int(blockIdx.x) == nb - 1 && threadIdx.x == 0) out[n] = running;
 }
 
+constexpr int kBlockT = 256;
+
+// Exclusive scan of value(k) over k < n into out[0..n] (out[n] = total) by the
+// whole block of kBlockT threads in LDS: thread t takes a run of k.  value is
+// called once per k, by the thread of its run, in order.
+template <class Value>
+__device__ __forceinline__ void block_exclusive(int n, const Value &value, int *out, int *wsum) {
+    const int per = (n + kBlockT - 1) / kBlockT;
+    const int lo = min(int(threadIdx.x) * per, n), hi = min(lo + per, n);
+    int sum = 0;
+    for (int k = lo; k < hi; ++k) {
+        const int v = value(k);
+        out[k] = sum;
+        sum += v;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int off = incl - sum;
+    for (int w = 0; w < wave; ++w) off += wsum[w];
+    for (int k = lo; k < hi; ++k) out[k] += off;
+    if (threadIdx.x == kBlockT - 1) out[n] = off + sum;
+    __syncthreads();
+}
+
 }  // namespace
 
 // out[0..n] = exclusive scan of in[0..n) with out[n] = total.  Workspace:

@@ -29,29 +29,53 @@ __device__ __forceinline__ double pgrad(int hash, double x, double y) {
     const double u = h < 8 ? x : y, v = h < 4 ? y : (h == 12 || h == 14) ? x : 0.0;
     return ((h & 1) == 0 ? u : -u) + ((h & 2) == 0 ? v : -v);
 }
-__device__ double pnoise(const int *p, double x, double y) {
-    const int X = static_cast<int>(floor(x)) & 255;
-    const int Y = static_cast<int>(floor(y)) & 255;
-    x -= floor(x);
-    y -= floor(y);
-    const double u = pfade(x), v = pfade(y);
-    const int A = p[X] + Y, AA = p[A], AB = p[A + 1];
-    const int B = p[X + 1] + Y, BA = p[B], BB = p[B + 1];
-    return plerp(v, plerp(u, pgrad(p[AA], x, y), pgrad(p[BA], x - 1, y)),
-                 plerp(u, pgrad(p[AB], x, y - 1), pgrad(p[BB], x - 1, y - 1)));
+// The lag and slope noises of an atom share its coordinates, so both are
+// evaluated together from one table of packed entries: entry k holds
+// lag[k], lag[k + 1], slope[k], slope[k + 1] in its four bytes (k + 1 past
+// the end: 0, never read; the tables are permutations of bytes).  One LDS
+// read then gives both tables' neighbours at k -- 13 reads per octave instead
+// of 20 -- and the floors and fade polynomials are computed once.
+constexpr int kPerlinTab = 512;
+__device__ __forceinline__ void stage_perlin(const int32_t *lag, const int32_t *slope, uint32_t *tab, int t, int nt) {
+    for (int i = t; i < kPerlinTab; i += nt) {
+        const int j = i + 1 < kPerlinTab ? i + 1 : i;
+        tab[i] = uint32_t(lag[i] & 255) | (uint32_t(lag[j] & 255) << 8) | (uint32_t(slope[i] & 255) << 16) |
+                 (uint32_t(slope[j] & 255) << 24);
+    }
+}
+__device__ __forceinline__ void pnoise2(const uint32_t *tab, double x, double y, double &lag, double &slope) {
+    const double flx = floor(x), fly = floor(y);
+    const int X = static_cast<int>(flx) & 255;
+    const int Y = static_cast<int>(fly) & 255;
+    x -= flx;
+    y -= fly;
+    const double u = pfade(x), v = pfade(y), x1 = x - 1, y1 = y - 1;
+    const uint32_t e = tab[X];
+    const uint32_t la = tab[int(e & 255u) + Y], lb = tab[int((e >> 8) & 255u) + Y];
+    const uint32_t sa = tab[int((e >> 16) & 255u) + Y], sb = tab[int(e >> 24) + Y];
+    const int l00 = int(tab[la & 255u]), l10 = int(tab[lb & 255u]);
+    const int l01 = int(tab[(la >> 8) & 255u]), l11 = int(tab[(lb >> 8) & 255u]);
+    const int s00 = int(tab[(sa >> 16) & 255u] >> 16), s10 = int(tab[(sb >> 16) & 255u] >> 16);
+    const int s01 = int(tab[sa >> 24] >> 16), s11 = int(tab[sb >> 24] >> 16);
+    lag = plerp(v, plerp(u, pgrad(l00, x, y), pgrad(l10, x1, y)), plerp(u, pgrad(l01, x, y1), pgrad(l11, x1, y1)));
+    slope = plerp(v, plerp(u, pgrad(s00, x, y), pgrad(s10, x1, y)), plerp(u, pgrad(s01, x, y1), pgrad(s11, x1, y1)));
 }
 // Out of line (scalar arguments): inlined into a kernel, its octaves' table
 // lookups are scheduled together with the caller's values and the kernel
 // takes about forty more registers.
-__device__ __noinline__ double poctave(const int *p, double x, double y) {
-    double result = 0.0, amp = 1.0;
+__device__ __noinline__ double2 poctave2(const uint32_t *tab, double x, double y) {
+    double lag = 0.0, slope = 0.0, amp = 1.0;
+#pragma unroll 1
     for (int i = 0; i < 8; ++i) {
-        result += pnoise(p, x, y) * amp;
+        double l, s;
+        pnoise2(tab, x, y, l, s);
+        lag += l * amp;
+        slope += s * amp;
         x *= 2.0;
         y *= 2.0;
         amp *= 0.5;
     }
-    return result;
+    return double2{lag, slope};
 }
 
 // ------------------------------------------------------------- colours
@@ -79,11 +103,10 @@ __device__ uint32_t fade_mix(uint32_t c1, uint32_t c2, double lag, double slope,
 // The colour fade of get_pixels / get_background for perlin coordinates
 // (px, py) (only used for PERLIN).
 __device__ uint32_t fade_colour(uint32_t c1, uint32_t c2, double px, double py, double str, int fading,
-                                const int *lagp, const int *slopep) {
+                                const uint32_t *tab) {
     if (fading == kPerlin) {
-        const double lag = poctave(lagp, px, py) * 0.5 + 0.5;
-        const double slope = poctave(slopep, px, py) * 0.5 + 0.5;
-        return fade_mix(c1, c2, lag, slope, str, fading);
+        const double2 o = poctave2(tab, px, py);
+        return fade_mix(c1, c2, o.x * 0.5 + 0.5, o.y * 0.5 + 0.5, str, fading);
     }
     if (fading == kCosine) return fade_mix(c1, c2, 0.5, 0.5, str, fading);
     return mix(c1, c2, str);
@@ -98,8 +121,7 @@ __device__ __forceinline__ uint32_t key_px(const uint32_t *keys, int f, int W, i
 }
 
 
-__device__ uint32_t background(const amh_render &R, const Frame &F, int x, int y, const int *lagp,
-                               const int *slopep) {
+__device__ uint32_t background(const amh_render &R, const Frame &F, int x, int y, const uint32_t *tab) {
     const uint32_t c1 = key_px(R.keys_dev, F.fk, R.width, R.height, x, y);
     const uint32_t c2 = key_px(R.keys_dev, F.fnext, R.width, R.height, x, y);
     double px = 0.0, py = 0.0;
@@ -108,7 +130,7 @@ __device__ uint32_t background(const amh_render &R, const Frame &F, int x, int y
         px = ((x - R.bbox_x1) / double(bw)) * 8.0;
         py = ((y - R.bbox_y1) / double(bh)) * 8.0;
     }
-    return fade_colour(c1, c2, px, py, 1.0 - F.tl, R.fading, lagp, slopep);
+    return fade_colour(c1, c2, px, py, 1.0 - F.tl, R.fading, tab);
 }
 
 // Trajectory point of atom a at the frame's time (morph.cpp:525-531 and
@@ -183,23 +205,18 @@ __device__ inline void traj_point(const amh_render &R, const Frame &F, int64_t a
     }
 }
 
-// The PERLIN fade's lag and slope at Perlin coordinates (px, py).
-__device__ __forceinline__ double2 lag_slope_at(double px, double py, const int *lagp, const int *slopep) {
-    return double2{poctave(lagp, px, py) * 0.5 + 0.5, poctave(slopep, px, py) * 0.5 + 0.5};
-}
-
 // The PERLIN fade's lag and slope of an atom with source point p1
 // (morph.cpp:537-550): the Perlin coordinates follow p1 over the bounding
 // box.  They depend on p1, the bounding box and the two tables only, not on
 // the time.
-__device__ __forceinline__ void atom_lag_slope(const amh_render &R, uint64_t p1, const int *lagp, const int *slopep,
-                                               double &lag, double &slope) {
+__device__ __forceinline__ void atom_lag_slope(const amh_render &R, uint64_t p1, const uint32_t *tab, double &lag,
+                                               double &slope) {
     const double bw = R.bbox_x2 - R.bbox_x1 + 1.0, bh = R.bbox_y2 - R.bbox_y1 + 1.0;
     const double perx = (((int(pt_x(p1)) - R.bbox_x1) * 256 + int(pt_xf(p1))) / double(bw * 256)) * 8.0;
     const double pery = (((int(pt_y(p1)) - R.bbox_y1) * 256 + int(pt_yf(p1))) / double(bh * 256)) * 8.0;
-    const double2 v = lag_slope_at(perx, pery, lagp, slopep);
-    lag = v.x;
-    slope = v.y;
+    const double2 o = poctave2(tab, perx, pery);
+    lag = o.x * 0.5 + 0.5;
+    slope = o.y * 0.5 + 0.5;
 }
 
 // Colour of an atom at the frame's time (morph.cpp:537-550); for PERLIN
@@ -213,9 +230,9 @@ __device__ inline uint32_t atom_colour_ls(const amh_render &R, const Frame &F, u
 }
 
 __device__ inline uint32_t atom_colour(const amh_render &R, const Frame &F, uint64_t p1, uint32_t c1, uint32_t c2,
-                                       const int *lagp, const int *slopep) {
+                                       const uint32_t *tab) {
     double lag = 0.5, slope = 0.5;
-    if (R.fading == kPerlin) atom_lag_slope(R, p1, lagp, slopep, lag, slope);
+    if (R.fading == kPerlin) atom_lag_slope(R, p1, tab, lag, slope);
     return atom_colour_ls(R, F, c1, c2, lag, slope);
 }
 

@@ -162,3 +162,40 @@ def test_render_graph_replays_equal_eager_frames(golden_cfg1, variant):
     finally:
         lib.amh_render_graph_destroy(graph)
         lib.amh_stream_destroy(stream)
+
+
+@pytest.mark.parametrize("W,H,nchains,width,spread,feather", [
+    (16, 16, 3, 40, 20, 0),      # one image tile, exactly
+    (17, 33, 5, 400, 20, 0),     # ragged tiles; more atoms in a tile than its workgroup has threads
+    (65, 31, 7, 300, 12, 3),     # feather across tiles, several blobs per pixel
+    (48, 20, 40, 60, 1, 0),      # forty blobs around one pixel
+    (48, 20, 40, 60, 1, 1),
+])
+def test_render_tiles_of_overlapping_blobs(W, H, nchains, width, spread, feather):
+    """Frames of random overlapping chains, tile edges and dense tiles, are
+    within 1 LSB per channel of the oracle's (exact integer sums against its
+    FP64 sums, as in the tests above)."""
+    rng = np.random.default_rng(W * 1000 + H)
+    h = 2
+    widths = np.full(nchains, width, np.int64)
+    wtot = int(widths.sum())
+    off = np.concatenate([[0], np.cumsum(widths)[:-1]]).astype(np.int64)
+    x = np.clip(W // 2 + rng.integers(-spread, spread + 1, (wtot, h)), 0, W - 1)
+    y = np.clip(H // 2 + rng.integers(-spread, spread + 1, (wtot, h)), 0, H - 1)
+    pts = op.pack_points(x, y, rng.integers(0, 256, (wtot, h)), rng.integers(0, 256, (wtot, h)), 3).ravel()
+    keys = rng.integers(0, 256, (h, H, W, 4)).astype(np.uint8)
+    keys[..., 3] = rng.choice([0, 120, 255], (h, H, W))
+    order = np.stack([rng.permutation(nchains) for _ in range(h)]).astype(np.int32)
+    lag, slope = op.perlin_perm(3), op.perlin_perm(4)
+    vals = {"bbox": [0, 0, W - 1, H - 1], "motion": 3, "fading": 6, "show": 0, "density": 2, "feather": feather,
+            "keep_bg": 1}
+    rend = GpuRenderer(keys, pts, off, widths, order, np.zeros((h, nchains), np.uint32), vals, lag, slope)
+    cfg = op.RenderCfg(W, H, h, 0, 0, W - 1, H - 1, 3, 6, 0, 2, feather, 1, 0, 0, op.ptr(lag), op.ptr(slope))
+    want = np.zeros((H, W, 4), np.uint8)
+    for t in (0.0, 0.21, 0.5, 0.9):
+        G.log(f"render tiles {W}x{H} {nchains} chains of {width}, feather {feather}, t={t}")
+        got = rend.frame(t)
+        op.oracle().or_render_atoms(C.byref(cfg), op.ptr(keys), op.ptr(pts), op.ptr(off), op.ptr(widths), nchains,
+                                    op.ptr(order), nchains, None, t, op.ptr(want))
+        assert int(np.abs(got.astype(np.int32) - want.astype(np.int32)).max()) <= 1, t
+        assert (rend.frame(t) == got).all()
