@@ -1872,7 +1872,7 @@ __global__ __launch_bounds__(kT) void k_fluid_update(amh_render R, const FramePa
                                                     LagSlopeMemo *__restrict__ memo,
                                                     const uint64_t *__restrict__ atom_keys) {
     const Frame F = fp->F;
-    __shared__ uint32_t tab[kPerlinTab];
+    __shared__ PerlinTab tab;
     __shared__ uint64_t wsum[kT / 64];
     __shared__ int32_t choff[kChainLds];
     uint64_t tag = 0;
@@ -2026,7 +2026,7 @@ __global__ __launch_bounds__(kT) void k_fluid_compose(amh_render R, const FrameP
                                                       const uint32_t *img, const int32_t *mask) {
     const Frame F = fp->F;
     uint32_t *out = fp->out;
-    __shared__ uint32_t tab[kPerlinTab];
+    __shared__ PerlinTab tab;
     if (R.keep_background && R.fading == kPerlin)
         stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
     __syncthreads();

@@ -23,8 +23,10 @@
 // the L2: with five of them per tap into per-pixel accumulators in memory
 // (and a second, scanned list for the other blobs of a pixel) a frame took
 // 1,518 us at 2048^2 with 1.7 M atoms, 261 us at 1001 x 777 with feather 2;
-// in tiles it takes 330 and 99 us.
+// in tiles it takes 212 and 90 us (kernels at 2048^2: prepare 108, place 35,
+// splat 78 us).
 #include <mutex>
+#include <type_traits>
 
 #include "colour.h"
 #include "common.h"
@@ -61,16 +63,6 @@ struct Tiles {
     uint32_t *list;    // [<= 4 atoms] atom numbers
 };
 
-// What changes from frame to frame when frames replay from a captured
-// hipGraph: the kernels read it from device memory instead of their
-// arguments.
-struct RenderParams {
-    Frame F;
-    uint32_t *out;
-};
-
-__global__ void k_set_render_params(RenderParams *dst, RenderParams v) { *dst = v; }
-
 // The taps of `mask` (bit k: tap (k & 1, k >> 1) of the base pixel x, y) that
 // fall in tile (x / 16 + (j & 1), y / 16 + (j >> 1)).
 __device__ __forceinline__ uint32_t taps_in(uint32_t mask, uint32_t x, uint32_t y, int j) {
@@ -81,26 +73,29 @@ __device__ __forceinline__ int tile_of(uint32_t x, uint32_t y, int j, int ntx) {
     return int(y / kTile + (j >> 1)) * ntx + int(x / kTile + (j & 1));
 }
 
-// What bounds it: the PERLIN fade's 16 noise octaves per atom (FP64 and LDS
-// table reads).  The taps are counted per tile with the wave's lanes grouped
+// What bounds it: the instructions of the PERLIN fade's 16 noise octaves per
+// atom (1.7 M atoms: 246 us with one noise at a time and selects for the
+// gradients, 108 us with both together from tables).  The taps are counted per tile with the wave's lanes grouped
 // by tile first, one atomic per distinct tile: neighbouring atoms of a chain
 // fall in few tiles.
-__global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B,
-                                                const RenderParams *__restrict__ fp) {
-    if (fp) F = fp->F;
-    __shared__ uint32_t tab[kPerlinTab];
+__global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B) {
+    __shared__ PerlinTab tab;
+    const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
+    const bool in = a < R.wtot;
+    // the points first: their loads overlap the tables' and the chain search
+    const int64_t al = in ? a : 0;
+    const uint64_t p1 = R.pts_dev[int64_t(F.fk) * R.wtot + al];
+    const uint64_t p2 = R.pts_dev[int64_t(F.fnext) * R.wtot + al];
+    uint64_t tk[4] = {p1, p1, p2, p2};
+    traj_keys(R, F, al, tk);
     if (R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
     __syncthreads();
-    const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
     const int c = block_chain(R.chain_off_dev, R.nchains, a);
-    const bool in = a < R.wtot;
     uint32_t mask = 0, X = 0, Y = 0;
     if (in) {
         Rec rec = {0u, 0u, 0u, -1};
         const int W = R.width, H = R.height;
         const int b = R.rank_dev[int64_t(F.fk) * R.nchains + c];
-        const uint64_t p1 = R.pts_dev[int64_t(F.fk) * R.wtot + a];
-        const uint64_t p2 = R.pts_dev[int64_t(F.fnext) * R.wtot + a];
         const bool h1 = pt_flags(p1) & HAS_PIXEL, h2 = pt_flags(p2) & HAS_PIXEL;
         if (b >= 0 && (h1 || h2)) {
             // colours at both ends (morph.cpp:495-522); a missing end fades from /
@@ -110,7 +105,7 @@ __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__re
             if (!h2) c2 = c1 & 0x00FFFFFFu;
             else if (!h1) c1 = c2 & 0x00FFFFFFu;
             uint32_t qxf, qyf;
-            traj_point(R, F, a, p1, p2, X, Y, qxf, qyf);
+            traj_point(R, F, a, p1, p2, X, Y, qxf, qyf, tk);
             const uint32_t col = atom_colour(R, F, p1, c1, c2, tab);
             // guards and taps (morph.cpp:552-589); taps outside the image are
             // dropped (draw_atoms skips pos >= W*H)
@@ -180,11 +175,14 @@ __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int6
             todo &= ~same;
         }
     }
-    int base[4];
-    for (int j = 0; j < 4; ++j) base[j] = total[j] > 0 ? atomicAdd(&B.entries[t[j]], total[j]) : 0;
+    int base[4], first[4];
+    for (int j = 0; j < 4; ++j) {
+        base[j] = total[j] > 0 ? atomicAdd(&B.entries[t[j]], total[j]) : 0;
+        first[j] = start[max(t[j], 0)];
+    }
     for (int j = 0; j < 4; ++j) {
         const int b = __shfl(base[j], lead[j], 64);
-        if (t[j] >= 0) B.list[start[t[j]] + b + pre[j]] = uint32_t(a);
+        if (t[j] >= 0) B.list[first[j] + b + pre[j]] = uint32_t(a);
     }
 }
 
@@ -194,20 +192,24 @@ struct Px {  // one resolved (pixel, blob) colour
 };
 
 // morph.cpp:591-623 with exact integer sums: round(sum c*n / sum n), alpha
-// times min(1, count / density).
-__device__ Px resolve(uint64_t cnt, uint64_t sn, const uint64_t s[4], int density) {
-    Px q;
-    const uint64_t d2 = 2 * sn;
-    q.r = uint32_t((2 * s[0] + sn) / d2);
-    q.g = uint32_t((2 * s[1] + sn) / d2);
-    q.b = uint32_t((2 * s[2] + sn) / d2);
-    double w = density > 0 ? double(cnt) / double(density) : 0.0;
-    if (w >= 1.0) {
-        q.a = uint32_t((2 * s[3] + sn) / d2);
-    } else {
-        q.a = narrow8(round(w * (double(s[3]) / double(sn))));
+// times min(1, count / density).  The quotients are floor((2 s + sn) / (2 sn))
+// through one FP64 reciprocal: all operands are integers below 2^53, so the
+// estimate is at most one off and its remainder, exact in a fused
+// multiply-add, says which way (four 64-bit integer divisions took the splat
+// 110 registers).
+template <class T>
+__device__ __forceinline__ Px resolve(uint32_t cnt, T sn, const T s[4], int density) {
+    const double n = double(sn), d = 2.0 * n, inv = 1.0 / d;
+    uint32_t v[4];
+    for (int k = 0; k < 4; ++k) {
+        const double num = fma(2.0, double(s[k]), n);
+        const int q = int(num * inv);
+        const double rem = fma(-double(q), d, num);
+        v[k] = uint32_t(q + (rem >= d ? 1 : 0) - (rem < 0.0 ? 1 : 0));
     }
-    return q;
+    const double w = density > 0 ? double(cnt) / double(density) : 0.0;
+    if (!(w >= 1.0)) v[3] = narrow8(round(w * (double(s[3]) / n)));
+    return Px{v[0], v[1], v[2], v[3]};
 }
 
 // With feather: the resolved blobs of a pixel, in increasing blob order.  The
@@ -225,9 +227,8 @@ struct Resolved {
     Ov *ov;         // [<= 4 atoms]
 };
 
-// Does pixel q hold blob b?
-__device__ __forceinline__ bool member(const Resolved &V, int64_t q, int b) {
-    if (V.blob[q] >= b) return V.blob[q] == b;  // the pixel's smallest
+// Is blob b among the further blobs of pixel q?
+__device__ __forceinline__ bool chained(const Resolved &V, int64_t q, int b) {
     for (int i = V.next[q]; i >= 0; i = V.ov[i].next)
         if (V.ov[i].blob == b) return true;
     return false;
@@ -244,27 +245,64 @@ __device__ int feather_depth(int x, int y, int W, int H, int F, int b, const Res
     best = min(best, 65536 - x);
     best = min(best, 65536 - y);
     for (int r = 1; r < best; ++r) {
-        // pixels at L1 distance exactly r
-        for (int dx = -r; dx <= r; ++dx) {
-            const int ady = r - (dx < 0 ? -dx : dx);
-            for (int sgn = -1; sgn <= 1; sgn += 2) {
-                if (ady == 0 && sgn > 0) continue;
-                const int qx = x + dx, qy = y + sgn * ady;
-                bool in;
-                if (qx < 0 || qy < 0 || qx >= W || qy >= H) in = false;
-                else in = member(V, int64_t(qy) * W + qx, b);
-                if (!in) return r;
+        // the 4 r pixels at L1 distance r, one of each quadrant at a time, so
+        // that their first blobs are loaded together
+        for (int i = 0; i < r; ++i) {
+            const int dx[4] = {i, r - i, -i, i - r}, dy[4] = {r - i, -i, i - r, i};
+            int64_t q[4];
+            int v[4];
+            bool in = true;
+            for (int k = 0; k < 4; ++k) {
+                const int qx = x + dx[k], qy = y + dy[k];
+                const bool ok = qx >= 0 && qy >= 0 && qx < W && qy < H;
+                in = in && ok;
+                q[k] = ok ? int64_t(qy) * W + qx : 0;
+                v[k] = V.blob[q[k]];
             }
+            for (int k = 0; k < 4; ++k) in = in && (v[k] == b || (v[k] < b && chained(V, q[k], b)));
+            if (!in) return r;
         }
     }
     return best;
 }
 
-struct Fold {
+// "Over" in increasing blob order (morph.cpp:1357-1380).  Without blending
+// the first colour is only taken apart when a second follows: alone, it comes
+// back from the division by 255 and the rounding as it was.
+struct Over {
+    double r = 0, g = 0, b = 0, a = 0;
+    uint32_t one = 0;
+    int n = 0;
+    __device__ void add(uint32_t c) {
+        if (n++ == 0) {
+            one = c;
+            return;
+        }
+        if (n == 2) {
+            r = (one & 255u) / 255.0;
+            g = ((one >> 8) & 255u) / 255.0;
+            b = ((one >> 16) & 255u) / 255.0;
+            a = (one >> 24) / 255.0;
+        }
+        const double sr = (c & 255u) / 255.0, sg = ((c >> 8) & 255u) / 255.0;
+        const double sb = ((c >> 16) & 255u) / 255.0, sa = (c >> 24) / 255.0;
+        r = sa * sr + (1.0 - sa) * r;
+        g = sa * sg + (1.0 - sa) * g;
+        b = sa * sb + (1.0 - sa) * b;
+        a = a + (1.0 - a) * sa;
+    }
+    __device__ uint32_t colour() const {
+        if (n < 2) return one;
+        return rgba_pack(narrow8(round(r * 255.0)), narrow8(round(g * 255.0)), narrow8(round(b * 255.0)),
+                         narrow8(round(a * 255.0)));
+    }
+};
+
+// The same with the alpha-weighted sums that blending takes.
+struct Blend {
     double r = 0, g = 0, b = 0, a = 0, rs = 0, gs = 0, bs = 0, as = 0;
     int n = 0;
     __device__ void add(uint32_t c) {
-        // morph.cpp:1357-1380
         const double sr = (c & 255u) / 255.0, sg = ((c >> 8) & 255u) / 255.0;
         const double sb = ((c >> 16) & 255u) / 255.0, sa = (c >> 24) / 255.0;
         as += sa;
@@ -277,14 +315,14 @@ struct Fold {
             r = sa * sr + (1.0 - sa) * r;
             g = sa * sg + (1.0 - sa) * g;
             b = sa * sb + (1.0 - sa) * b;
-            a = a + (1.0 - a) * ((c >> 24) / 255.0);
+            a = a + (1.0 - a) * sa;
         }
         ++n;
     }
 };
 
 // The folded pixel over the background (morph.cpp:1381-1401, 1405-1417).
-__device__ uint32_t finish(const amh_render &R, const Fold &fold, uint32_t bg) {
+__device__ __forceinline__ uint32_t finish(const amh_render &R, const Blend &fold, uint32_t bg) {
     if (fold.n == 0) return bg;
     double r = fold.r, g = fold.g, b = fold.b, a = fold.a;
     if (R.blend_blobs) {
@@ -304,83 +342,167 @@ __device__ uint32_t finish(const amh_render &R, const Fold &fold, uint32_t bg) {
                      narrow8(round(a * 255.0)));
 }
 
-// One tile's pixels from its listed atoms.  Each pass sums, per pixel, the
-// taps of one blob (bcur) in LDS and finds the next larger blob that touches
-// the pixel (bnext) on the way; most pixels hold one or two blobs.  The first
-// atom of each thread is kept in registers for all passes (a tile lists about
-// one atom per covered pixel and density), further ones are read again.
-// kFeather: the resolved colours go to V for k_composite.  Leaves the tile's
-// counters at zero for the next frame.
-template <bool kFeather>
-__global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *__restrict__ recs, Tiles B, Resolved V,
-                                              uint32_t *__restrict__ out, const RenderParams *__restrict__ fp) {
-    if (fp) {
-        F = fp->F;
-        out = fp->out;
+// Per-pixel sums of a tile in LDS: taps, sum n and sum c * n per channel.
+// Wide: any number of taps.  Packed: a tile of at most kPackedAtoms atoms, of
+// which each gives a pixel one tap at most, so sum n < 2^24, the taps fit in
+// 8 bits and sum c * n in 32: three atomics per tap instead of five.
+constexpr int kPackedAtoms = 255;
+static_assert(255ull * 65025 * kPackedAtoms < 1ull << 32 && 65025 * kPackedAtoms < 1 << 24, "packed sums");
+
+struct PackedSums {
+    using T = uint32_t;
+    uint32_t cn[kTilePx];                         // taps << 24 | sum n
+    unsigned long long rg[kTilePx], ba[kTilePx];  // two channels each
+    __device__ __forceinline__ void clear(int p) {
+        cn[p] = 0u;
+        rg[p] = ba[p] = 0ull;
     }
-    __shared__ unsigned long long acc[5][kTilePx];  // count << 40 | sum n, then sum c * n per channel
-    __shared__ int bcur[kTilePx], bnext[kTilePx];
-    __shared__ uint32_t tab[kFeather ? 1 : kPerlinTab];
-    __shared__ int nov;
-    const int tile = int(blockIdx.x), tid = int(threadIdx.x);
-    const int x0 = (tile % B.ntx) * kTile, y0 = (tile / B.ntx) * kTile;
-    const int n = B.entries[tile], s0 = B.start[tile];
-    const uint32_t *list = B.list + s0;
-    Rec mine = {0u, 0u, 0u, 0};
-    if (tid < n) mine = recs[list[tid]];
-    if (!kFeather && R.keep_background && R.fading == kPerlin)
-        stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, tid, kT);
-    bnext[tid] = kNoBlob;
-    if (tid == 0) nov = 0;
-    __syncthreads();
-    if (tid == 0 && n > 0) {
-        B.entries[tile] = 0;
-        B.taps[tile] = 0;
+    __device__ __forceinline__ void add(int p, uint32_t n, uint32_t col) {
+        atomicAdd(&cn[p], (1u << 24) | n);
+        atomicAdd(&rg[p], (unsigned long long)(ch(col, 0) * n) | ((unsigned long long)(ch(col, 1) * n) << 32));
+        atomicAdd(&ba[p], (unsigned long long)(ch(col, 2) * n) | ((unsigned long long)(ch(col, 3) * n) << 32));
     }
-    // f(pixel of the tile, weight numerator, atom) for every tap in the tile
-    const auto taps = [&](const auto &f) {
-        for (int e = tid; e < n; e += kT) {
-            const Rec r = e == tid ? mine : recs[list[e]];
-            const uint32_t xf = r.fm & 255u, yf = (r.fm >> 8) & 255u, mask = r.fm >> 16;
-            const int lx = int(r.xy & 0xFFFFu) - x0, ly = int(r.xy >> 16) - y0;
-            for (int k = 0; k < 4; ++k) {
-                const int px = lx + (k & 1), py = ly + (k >> 1);
-                if (!((mask >> k) & 1u) || uint32_t(px) >= uint32_t(kTile) || uint32_t(py) >= uint32_t(kTile)) continue;
-                f(py * kTile + px, ((k & 1) ? xf : 255u - xf) * ((k >> 1) ? yf : 255u - yf), r);
-            }
+    __device__ __forceinline__ uint32_t get(int p, T &sn, T s[4]) const {
+        const uint32_t v = cn[p];
+        sn = v & 0xFFFFFFu;
+        s[0] = T(rg[p]);
+        s[1] = T(rg[p] >> 32);
+        s[2] = T(ba[p]);
+        s[3] = T(ba[p] >> 32);
+        return v >> 24;
+    }
+};
+struct WideSums {
+    using T = uint64_t;
+    unsigned long long cn[kTilePx], s[4][kTilePx];  // taps << 40 | sum n
+    __device__ __forceinline__ void clear(int p) {
+        cn[p] = 0ull;
+        for (int k = 0; k < 4; ++k) s[k][p] = 0ull;
+    }
+    __device__ __forceinline__ void add(int p, uint32_t n, uint32_t col) {
+        atomicAdd(&cn[p], (1ull << 40) | n);
+        for (int k = 0; k < 4; ++k) atomicAdd(&s[k][p], (unsigned long long)(ch(col, k) * n));
+    }
+    __device__ __forceinline__ uint32_t get(int p, T &sn, T v[4]) const {
+        sn = cn[p] & ((1ull << 40) - 1);
+        for (int k = 0; k < 4; ++k) v[k] = s[k][p];
+        return uint32_t(cn[p] >> 40);
+    }
+};
+
+// f(pixel of the tile at x0, y0, weight numerator, atom) for every tap in the
+// tile of its n atoms; each thread's first atom is `mine`.
+template <class F>
+__device__ __forceinline__ void for_taps(const Rec *__restrict__ recs, const uint32_t *__restrict__ list, int n,
+                                         const Rec &mine, int x0, int y0, const F &f) {
+    for (int e = threadIdx.x; e < n; e += kT) {
+        Rec r = e == int(threadIdx.x) ? mine : recs[list[e]];
+        // opaque, so that the taps' products are not kept for all passes
+        // (they took 108 registers; without them eight waves fit)
+        asm volatile("" : "+v"(r.xy), "+v"(r.fm), "+v"(r.col));
+        const uint32_t xf = r.fm & 255u, yf = (r.fm >> 8) & 255u, mask = r.fm >> 16;
+        const int lx = int(r.xy & 0xFFFFu) - x0, ly = int(r.xy >> 16) - y0;
+        for (int k = 0; k < 4; ++k) {
+            const int px = lx + (k & 1), py = ly + (k >> 1);
+            if (!((mask >> k) & 1u) || uint32_t(px) >= uint32_t(kTile) || uint32_t(py) >= uint32_t(kTile)) continue;
+            f(py * kTile + px, ((k & 1) ? xf : 255u - xf) * ((k >> 1) ? yf : 255u - yf), r);
+        }
+    }
+}
+
+// Calls emit(blob, colour) for every blob of this thread's pixel in
+// increasing blob order.  one: the blob of every atom of the tile, or -1: then
+// each pass sums, per pixel, the taps of one blob (bcur) and finds the next
+// larger one that touches the pixel (bnext) on the way.
+template <class Sums, class Emit>
+__device__ __forceinline__ void tile_blobs(Sums &acc, int *bcur, int *bnext, const Rec *__restrict__ recs,
+                                           const uint32_t *__restrict__ list, int n, const Rec &mine, int one, int x0,
+                                           int y0, int density, const Emit &emit) {
+    const int tid = threadIdx.x;
+    const auto give = [&](int b) {
+        typename Sums::T sn, s[4];
+        const uint32_t cnt = acc.get(tid, sn, s);
+        if (cnt) {
+            const Px q = resolve(cnt, sn, s, density);
+            emit(b, rgba_pack(q.r, q.g, q.b, q.a));
         }
     };
-    taps([&](int p, uint32_t, const Rec &r) { atomicMin(&bnext[p], r.blob); });
+    acc.clear(tid);
+    if (one >= 0) {
+        __syncthreads();
+        for_taps(recs, list, n, mine, x0, y0, [&](int p, uint32_t w, const Rec &r) { acc.add(p, w, r.col); });
+        __syncthreads();
+        give(one);
+        return;
+    }
+    bnext[tid] = kNoBlob;
     __syncthreads();
-    const int x = x0 + tid % kTile, y = y0 + tid / kTile;
-    const bool inside = x < R.width && y < R.height;
-    const int64_t p = int64_t(y) * R.width + x;
-    const bool texture = R.show_blobs != 1 && R.show_blobs != 2;
-    Fold fold;
-    int last = -1;  // kFeather: the pixel's last chained Ov
-    bool first = true;
+    for_taps(recs, list, n, mine, x0, y0, [&](int p, uint32_t, const Rec &r) { atomicMin(&bnext[p], r.blob); });
+    __syncthreads();
     for (;;) {
         const int b = bnext[tid];
         bcur[tid] = b;
         bnext[tid] = kNoBlob;
-        for (int k = 0; k < 5; ++k) acc[k][tid] = 0ull;
+        acc.clear(tid);
         if (!__syncthreads_or(b != kNoBlob)) break;
-        taps([&](int q, uint32_t w, const Rec &r) {
-            const int cur = bcur[q];
-            if (r.blob == cur) {
-                atomicAdd(&acc[0][q], (1ull << 40) | w);
-                for (int k = 0; k < 4; ++k) atomicAdd(&acc[1 + k][q], (unsigned long long)(ch(r.col, k) * w));
-            } else if (r.blob > cur) {
-                atomicMin(&bnext[q], r.blob);
-            }
+        for_taps(recs, list, n, mine, x0, y0, [&](int p, uint32_t w, const Rec &r) {
+            const int cur = bcur[p];
+            if (r.blob == cur) acc.add(p, w, r.col);
+            else if (r.blob > cur) atomicMin(&bnext[p], r.blob);
         });
         __syncthreads();
-        if (b != kNoBlob) {
-            const uint64_t cn = acc[0][tid];
-            const uint64_t s[4] = {acc[1][tid], acc[2][tid], acc[3][tid], acc[4][tid]};
-            const Px q = resolve(cn >> 40, cn & ((1ull << 40) - 1), s, R.density);
-            uint32_t c = rgba_pack(q.r, q.g, q.b, q.a);
-            if (kFeather) {
+        give(b);
+    }
+}
+
+// One workgroup per tile, one thread per pixel.  A tile's loads are one
+// dependent chain (counters, list, atoms), so each mode holds only the
+// registers it needs and eight workgroups fit a CU; then the LDS atomics and
+// the tap arithmetic bound it.  Hence the packed sums, and the single pass
+// over a tile whose atoms are all of one blob (most covered tiles): 109 us at
+// 2048^2 with 110 registers and five sums, 94 with 54 registers, 78 with
+// these.  Leaves the tile's counters at zero for the next frame.
+enum SplatMode {
+    kPlain,    // no background, no blending
+    kOver,     // over the background, or blending
+    kFeather,  // the resolved colours go to V for k_composite
+};
+template <SplatMode kMode>
+__global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *__restrict__ recs, Tiles B, Resolved V,
+                                              uint32_t *__restrict__ out) {
+    __shared__ union {
+        PackedSums packed;
+        WideSums wide;
+    } acc;
+    __shared__ int bcur[kTilePx], bnext[kTilePx];
+    __shared__ std::conditional_t<kMode == kOver, PerlinTab, char> tab;
+    __shared__ int nov, some;
+    const int tile = int(blockIdx.x), tid = int(threadIdx.x);
+    const int x0 = (tile % B.ntx) * kTile, y0 = (tile / B.ntx) * kTile;
+    const int x = x0 + tid % kTile, y = y0 + tid / kTile;
+    const bool inside = x < R.width && y < R.height;
+    const int64_t p = int64_t(y) * R.width + x;
+    const int n = B.entries[tile], s0 = B.start[tile];
+    std::conditional_t<kMode == kOver, Blend, Over> fold;
+    int last = -1;  // kFeather: the pixel's last chained Ov
+    bool first = true;
+    if constexpr (kMode == kOver)
+        if (R.keep_background && R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, tid, kT);
+    if (n > 0) {
+        const uint32_t *list = B.list + s0;
+        Rec mine = {0u, 0u, 0u, 0};
+        if (tid < n) mine = recs[list[tid]];
+        if (tid == 0) {
+            nov = 0;
+            some = mine.blob;
+        }
+        __syncthreads();
+        if (tid == 0) {  // every thread has read them
+            B.entries[tile] = 0;
+            B.taps[tile] = 0;
+        }
+        const auto emit = [&](int b, uint32_t c) {
+            if constexpr (kMode == kFeather) {
                 if (first) {
                     V.blob[p] = b;
                     V.col[p] = c;
@@ -393,29 +515,35 @@ __global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *
                 }
                 first = false;
             } else {
+                const bool texture = R.show_blobs != 1 && R.show_blobs != 2;
                 if (!texture && R.blob_rgba_dev) c = R.blob_rgba_dev[int64_t(F.fk) * R.nblobs + b];
                 if (c >> 24) fold.add(c);
             }
+        };
+        if (n <= kPackedAtoms) {
+            const int one = __syncthreads_or(tid < n && mine.blob != some) ? -1 : some;
+            tile_blobs(acc.packed, bcur, bnext, recs, list, n, mine, one, x0, y0, R.density, emit);
+        } else {
+            tile_blobs(acc.wide, bcur, bnext, recs, list, n, mine, -1, x0, y0, R.density, emit);
         }
+    } else if (kMode == kOver) {
+        __syncthreads();  // the noise tables
     }
     if (!inside) return;
-    if (kFeather) {
+    if constexpr (kMode == kFeather) {
         if (first) V.blob[p] = kNoBlob;
         if (last < 0) V.next[p] = -1;
-    } else {
+    } else if constexpr (kMode == kOver) {
         out[p] = finish(R, fold, R.keep_background ? background(R, F, x, y, tab) : 0u);
+    } else {
+        out[p] = fold.colour();
     }
 }
 
 // Feather and composite of the resolved blobs (texture blobs only: the other
 // modes are not feathered).
-__global__ __launch_bounds__(kT) void k_composite(amh_render R, Frame F, Resolved V, uint32_t *__restrict__ out,
-                                                  const RenderParams *__restrict__ fp) {
-    if (fp) {
-        F = fp->F;
-        out = fp->out;
-    }
-    __shared__ uint32_t tab[kPerlinTab];
+__global__ __launch_bounds__(kT) void k_composite(amh_render R, Frame F, Resolved V, uint32_t *__restrict__ out) {
+    __shared__ PerlinTab tab;
     if (R.keep_background && R.fading == kPerlin)
         stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
     __syncthreads();
@@ -423,7 +551,7 @@ __global__ __launch_bounds__(kT) void k_composite(amh_render R, Frame F, Resolve
     const int64_t p = int64_t(blockIdx.x) * kT + threadIdx.x;
     if (p >= int64_t(W) * H) return;
     const int x = int(p % W), y = int(p / W);
-    Fold fold;
+    Blend fold;
     Ov o = {V.blob[p], V.col[p], V.next[p]};
     while (o.blob != kNoBlob) {
         const int d = feather_depth(x, y, W, H, R.feather, o.blob, V);
@@ -510,10 +638,7 @@ bool render_args_ok(const amh_render *R) {
 
 // The frame itself, on a workspace laid out by `L` whose tile counters are
 // zero; leaves them at zero.
-// fp (device, may be NULL): the frame's time and output are read from it
-// (graph capture; then nothing is timed, since events would be captured).
-int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, uint32_t *out, hipStream_t s,
-                    const RenderParams *fp = nullptr);
+int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, uint32_t *out, hipStream_t s);
 
 }  // namespace
 
@@ -600,9 +725,8 @@ extern "C" int amh_render_frame_noalloc(const amh_render *R, double t, uint32_t 
 }
 
 namespace {
-int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, uint32_t *out, hipStream_t s,
-                    const RenderParams *fp) {
-    amh::ProfScope whole_(fp ? nullptr : "render_frame", s);
+int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, uint32_t *out, hipStream_t s) {
+    amh::ProfScope whole_("render_frame", s);
     Rec *recs = reinterpret_cast<Rec *>(base + L.recs);
     const Tiles B = tiles_of(base, L);
     const Resolved V = {reinterpret_cast<int32_t *>(base + L.blob), reinterpret_cast<uint32_t *>(base + L.col),
@@ -623,14 +747,11 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
     F.fnext = (F.fk + 1) % R->nkeys;
     const double dt = 1.0 / double(R->nkeys);
     F.tl = fmax(0.0, (F.tn - (double(F.fk) * dt)) / dt);
-    // timed launches only outside graph capture (their events would be captured)
     const auto launch = [&](const char *name, auto kernel, int64_t threads, auto... args) {
-        const dim3 grid(uint32_t((threads + kT - 1) / kT));
-        if (fp) hipLaunchKernelGGL(kernel, grid, dim3(kT), 0, s, args...);
-        else amh::launch_timed(name, kernel, grid, dim3(kT), 0, s, args...);
+        amh::launch_timed(name, kernel, dim3(uint32_t((threads + kT - 1) / kT)), dim3(kT), 0, s, args...);
     };
     if (Rc.wtot > 0) {
-        launch("k_prepare", k_prepare, Rc.wtot, Rc, F, recs, B, fp);
+        launch("k_prepare", k_prepare, Rc.wtot, Rc, F, recs, B);
         if (L.tiles <= kLdsTiles) {
             launch("k_place", k_place<true>, Rc.wtot, recs, Rc.wtot, B);
         } else {
@@ -641,26 +762,28 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
     }
     const bool texture = Rc.show_blobs != 1 && Rc.show_blobs != 2;
     if (texture && Rc.feather > 0) {
-        launch("k_splat", k_splat<true>, L.tiles * kT, Rc, F, recs, B, V, out, fp);
-        launch("k_composite", k_composite, L.npx, Rc, F, V, out, fp);
+        launch("k_splat", k_splat<kFeather>, L.tiles * kT, Rc, F, recs, B, V, out);
+        launch("k_composite", k_composite, L.npx, Rc, F, V, out);
+    } else if (Rc.keep_background || Rc.blend_blobs) {
+        launch("k_splat", k_splat<kOver>, L.tiles * kT, Rc, F, recs, B, V, out);
     } else {
-        launch("k_splat", k_splat<false>, L.tiles * kT, Rc, F, recs, B, V, out, fp);
+        launch("k_splat", k_splat<kPlain>, L.tiles * kT, Rc, F, recs, B, V, out);
     }
     AMH_LAUNCH_CHECK("amh_render_frame");
     return AMH_OK;
 }
 }  // namespace
 
-// --------------------------------------------------- frames from a graph
-// One frame's launches captured once and replayed for every later frame of
-// the same chains and options; only the frame's time and output, in a small
-// device block, change between replays.
+// ------------------------------------------------- frames on a kept handle
+// The render arguments and the workspace checked and kept for many frames.
+// A frame is three or four launches, which are cheaper enqueued one by one
+// than as a captured graph with a launch for the frame's time before it:
+// eight 64^2 frames took 290 us replayed and 228 us enqueued, two 2048^2
+// frames 494 and 478 us.
 struct amh_render_graph_s {
     amh_render R;
-    char *ws = nullptr;
+    char *ws;
     Layout L;
-    RenderParams *fp = nullptr;  // device
-    hipGraphExec_t exec = nullptr;
 };
 
 extern "C" int amh_render_graph_create(void **graph, const amh_render *R, void *ws, size_t ws_bytes, void *stream) {
@@ -674,32 +797,7 @@ extern "C" int amh_render_graph_create(void **graph, const amh_render *R, void *
         set_error("amh_render_graph_create: workspace %zu < %zu bytes", ws_bytes, L.total);
         return AMH_E_ARG;
     }
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    amh_render_graph_s *g = new amh_render_graph_s;
-    g->R = *R;
-    g->ws = static_cast<char *>(ws);
-    g->L = L;
-    if (int r = check_hip(hipMalloc(&g->fp, sizeof(RenderParams)), "amh_render_graph_create")) {
-        delete g;
-        return r;
-    }
-    int r = check_hip(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    if (!r) {
-        // time 0 only fixes which launches the graph holds (a frame with
-        // atoms); every replay reads its own frame from g->fp
-        const int rr = render_frame_on(&g->R, 0.0, g->ws, g->L, nullptr, s, g->fp);
-        hipGraph_t gr = nullptr;
-        const hipError_t e = hipStreamEndCapture(s, &gr);
-        r = rr ? rr : check_hip(e, "hipStreamEndCapture");
-        if (!r) r = check_hip(hipGraphInstantiate(&g->exec, gr, nullptr, nullptr, 0), "hipGraphInstantiate");
-        if (gr) (void)hipGraphDestroy(gr);
-    }
-    if (r) {
-        (void)hipFree(g->fp);
-        delete g;
-        return r;
-    }
-    *graph = g;
+    *graph = new amh_render_graph_s{*R, static_cast<char *>(ws), L};
     return AMH_OK;
 }
 
@@ -709,24 +807,13 @@ extern "C" int amh_render_graph_frame(void *graph, double t, uint32_t *out, void
         set_error("amh_render_graph_frame: invalid argument");
         return AMH_E_ARG;
     }
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    RenderParams v;
-    v.F = frame_of(t, g->R.nkeys);
-    v.out = out;
-    // a frame with nothing to draw (no atoms, or a time past the keys)
-    // launches fewer kernels than the graph holds: it runs eagerly
-    if (g->R.wtot == 0 || v.F.fk >= g->R.nkeys) return render_frame_on(&g->R, t, g->ws, g->L, out, s);
-    hipLaunchKernelGGL(k_set_render_params, dim3(1), dim3(1), 0, s, g->fp, v);
-    if (int r = check_hip(hipGetLastError(), "amh_render_graph_frame")) return r;
-    return check_hip(hipGraphLaunch(g->exec, s), "amh_render_graph_frame");
+    return render_frame_on(&g->R, t, g->ws, g->L, out, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int amh_render_graph_destroy(void *graph) {
     amh_render_graph_s *g = static_cast<amh_render_graph_s *>(graph);
     if (!g) return AMH_OK;
-    (void)hipDeviceSynchronize();  // replays may still be queued on the caller's stream
-    if (g->exec) (void)hipGraphExecDestroy(g->exec);
-    (void)hipFree(g->fp);
+    (void)hipDeviceSynchronize();  // frames may still be queued on the caller's stream
     delete g;
     return AMH_OK;
 }

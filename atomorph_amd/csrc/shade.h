@@ -24,46 +24,56 @@ struct Frame {  // per-frame scalars, computed on the host
 // the z = 1 half never contributes and is not evaluated.
 __device__ __forceinline__ double pfade(double t) { return t * t * t * (t * (t * 6 - 15) + 10); }
 __device__ __forceinline__ double plerp(double t, double a, double b) { return a + t * (b - a); }
-__device__ __forceinline__ double pgrad(int hash, double x, double y) {
-    const int h = hash & 15;
-    const double u = h < 8 ? x : y, v = h < 4 ? y : (h == 12 || h == 14) ? x : 0.0;
-    return ((h & 1) == 0 ? u : -u) + ((h & 2) == 0 ? v : -v);
-}
 // The lag and slope noises of an atom share its coordinates, so both are
-// evaluated together from one table of packed entries: entry k holds
-// lag[k], lag[k + 1], slope[k], slope[k + 1] in its four bytes (k + 1 past
-// the end: 0, never read; the tables are permutations of bytes).  One LDS
-// read then gives both tables' neighbours at k -- 13 reads per octave instead
-// of 20 -- and the floors and fade polynomials are computed once.
-constexpr int kPerlinTab = 512;
-__device__ __forceinline__ void stage_perlin(const int32_t *lag, const int32_t *slope, uint32_t *tab, int t, int nt) {
-    for (int i = t; i < kPerlinTab; i += nt) {
-        const int j = i + 1 < kPerlinTab ? i + 1 : i;
-        tab[i] = uint32_t(lag[i] & 255) | (uint32_t(lag[j] & 255) << 8) | (uint32_t(slope[i] & 255) << 16) |
-                 (uint32_t(slope[j] & 255) << 24);
+// evaluated together, from LDS tables made for it.  A gradient's dot product
+// (+-u) + (+-v) with u, v among x, y, 0 is gx x + gy y with gx, gy in
+// {-1, 0, 1}: one exact product and one fused sum, the same double (but for
+// the sign of a zero, which the octaves' sum drops).
+struct PerlinTab {
+    uint32_t next[512];           // bytes lag[k], lag[k + 1], slope[k], slope[k + 1]
+    uint2 lag_g[256], slope_g[256];  // high words of the doubles gx, gy of hash lag[k], slope[k]
+};
+// The gradient of a hash (perlin.cpp: u = h < 8 ? x : y, v = h < 4 ? y : h is
+// 12 or 14 ? x : 0, signs by bits 0 and 1).
+__device__ __forceinline__ uint2 gradient(int hash) {
+    const uint32_t one = 0x3FF00000u, h = uint32_t(hash) & 15u;
+    const uint32_t u = one | (h << 31), v = one | ((h >> 1) << 31);
+    return uint2{h < 8 ? u : (h == 12 || h == 14) ? v : 0u, h < 4 ? v : h < 8 ? 0u : u};
+}
+__device__ __forceinline__ void stage_perlin(const int32_t *lag, const int32_t *slope, PerlinTab &T, int t, int nt) {
+    for (int i = t; i < 512; i += nt) {
+        const int j = i + 1 < 512 ? i + 1 : i;  // (entry 512 is never read)
+        const int l = lag[i], s = slope[i];
+        T.next[i] = uint32_t(l & 255) | (uint32_t(lag[j] & 255) << 8) | (uint32_t(s & 255) << 16) |
+                    (uint32_t(slope[j] & 255) << 24);
+        if (i < 256) {
+            T.lag_g[i] = gradient(l);
+            T.slope_g[i] = gradient(s);
+        }
     }
 }
-__device__ __forceinline__ void pnoise2(const uint32_t *tab, double x, double y, double &lag, double &slope) {
+__device__ __forceinline__ double pgrad(uint2 g, double x, double y) {
+    return fma(__hiloint2double(int(g.x), 0), x, __hiloint2double(int(g.y), 0) * y);
+}
+__device__ __forceinline__ void pnoise2(const PerlinTab &T, double x, double y, double &lag, double &slope) {
     const double flx = floor(x), fly = floor(y);
     const int X = static_cast<int>(flx) & 255;
     const int Y = static_cast<int>(fly) & 255;
     x -= flx;
     y -= fly;
     const double u = pfade(x), v = pfade(y), x1 = x - 1, y1 = y - 1;
-    const uint32_t e = tab[X];
-    const uint32_t la = tab[int(e & 255u) + Y], lb = tab[int((e >> 8) & 255u) + Y];
-    const uint32_t sa = tab[int((e >> 16) & 255u) + Y], sb = tab[int(e >> 24) + Y];
-    const int l00 = int(tab[la & 255u]), l10 = int(tab[lb & 255u]);
-    const int l01 = int(tab[(la >> 8) & 255u]), l11 = int(tab[(lb >> 8) & 255u]);
-    const int s00 = int(tab[(sa >> 16) & 255u] >> 16), s10 = int(tab[(sb >> 16) & 255u] >> 16);
-    const int s01 = int(tab[sa >> 24] >> 16), s11 = int(tab[sb >> 24] >> 16);
-    lag = plerp(v, plerp(u, pgrad(l00, x, y), pgrad(l10, x1, y)), plerp(u, pgrad(l01, x, y1), pgrad(l11, x1, y1)));
-    slope = plerp(v, plerp(u, pgrad(s00, x, y), pgrad(s10, x1, y)), plerp(u, pgrad(s01, x, y1), pgrad(s11, x1, y1)));
+    const uint32_t e = T.next[X];
+    const uint32_t la = T.next[int(e & 255u) + Y], lb = T.next[int((e >> 8) & 255u) + Y];
+    const uint32_t sa = T.next[int((e >> 16) & 255u) + Y], sb = T.next[int(e >> 24) + Y];
+    lag = plerp(v, plerp(u, pgrad(T.lag_g[la & 255u], x, y), pgrad(T.lag_g[lb & 255u], x1, y)),
+                plerp(u, pgrad(T.lag_g[(la >> 8) & 255u], x, y1), pgrad(T.lag_g[(lb >> 8) & 255u], x1, y1)));
+    slope = plerp(v, plerp(u, pgrad(T.slope_g[(sa >> 16) & 255u], x, y), pgrad(T.slope_g[(sb >> 16) & 255u], x1, y)),
+                  plerp(u, pgrad(T.slope_g[sa >> 24], x, y1), pgrad(T.slope_g[sb >> 24], x1, y1)));
 }
 // Out of line (scalar arguments): inlined into a kernel, its octaves' table
 // lookups are scheduled together with the caller's values and the kernel
 // takes about forty more registers.
-__device__ __noinline__ double2 poctave2(const uint32_t *tab, double x, double y) {
+__device__ __noinline__ double2 poctave2(const PerlinTab &tab, double x, double y) {
     double lag = 0.0, slope = 0.0, amp = 1.0;
 #pragma unroll 1
     for (int i = 0; i < 8; ++i) {
@@ -103,7 +113,7 @@ __device__ uint32_t fade_mix(uint32_t c1, uint32_t c2, double lag, double slope,
 // The colour fade of get_pixels / get_background for perlin coordinates
 // (px, py) (only used for PERLIN).
 __device__ uint32_t fade_colour(uint32_t c1, uint32_t c2, double px, double py, double str, int fading,
-                                const uint32_t *tab) {
+                                const PerlinTab &tab) {
     if (fading == kPerlin) {
         const double2 o = poctave2(tab, px, py);
         return fade_mix(c1, c2, o.x * 0.5 + 0.5, o.y * 0.5 + 0.5, str, fading);
@@ -121,7 +131,7 @@ __device__ __forceinline__ uint32_t key_px(const uint32_t *keys, int f, int W, i
 }
 
 
-__device__ uint32_t background(const amh_render &R, const Frame &F, int x, int y, const uint32_t *tab) {
+__device__ uint32_t background(const amh_render &R, const Frame &F, int x, int y, const PerlinTab &tab) {
     const uint32_t c1 = key_px(R.keys_dev, F.fk, R.width, R.height, x, y);
     const uint32_t c2 = key_px(R.keys_dev, F.fnext, R.width, R.height, x, y);
     double px = 0.0, py = 0.0;
@@ -209,7 +219,7 @@ __device__ inline void traj_point(const amh_render &R, const Frame &F, int64_t a
 // (morph.cpp:537-550): the Perlin coordinates follow p1 over the bounding
 // box.  They depend on p1, the bounding box and the two tables only, not on
 // the time.
-__device__ __forceinline__ void atom_lag_slope(const amh_render &R, uint64_t p1, const uint32_t *tab, double &lag,
+__device__ __forceinline__ void atom_lag_slope(const amh_render &R, uint64_t p1, const PerlinTab &tab, double &lag,
                                                double &slope) {
     const double bw = R.bbox_x2 - R.bbox_x1 + 1.0, bh = R.bbox_y2 - R.bbox_y1 + 1.0;
     const double perx = (((int(pt_x(p1)) - R.bbox_x1) * 256 + int(pt_xf(p1))) / double(bw * 256)) * 8.0;
@@ -230,7 +240,7 @@ __device__ inline uint32_t atom_colour_ls(const amh_render &R, const Frame &F, u
 }
 
 __device__ inline uint32_t atom_colour(const amh_render &R, const Frame &F, uint64_t p1, uint32_t c1, uint32_t c2,
-                                       const uint32_t *tab) {
+                                       const PerlinTab &tab) {
     double lag = 0.5, slope = 0.5;
     if (R.fading == kPerlin) atom_lag_slope(R, p1, tab, lag, slope);
     return atom_colour_ls(R, F, c1, c2, lag, slope);
