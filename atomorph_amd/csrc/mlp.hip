@@ -1,16 +1,11 @@
 // The learned proposal's MLP on the CDNA4 matrix cores.
 //
 // 8 -> 128 -> 128 -> 128 -> 128 -> 2, exact GELU after each hidden layer.
-// Parameters are kept as FP32 masters (Adam state beside them) and as a
-// bfloat16 copy that the matrix products read; activations are FP32 in HBM
-// and rounded to bfloat16 when a product stages them; every product
-// accumulates in FP32 (v_mfma_f32_32x32x16_bf16).
-//
-// All products run through one tiled kernel, C = A . B with free strides on
-// both operands (so transposes cost nothing) and a fused epilogue:
-//   forward      Z_l = A_{l-1} W_l + b_l, A_l = gelu(Z_l)
-//   backward     dZ_{l-1} = (dZ_l W_l^T) * gelu'(Z_{l-1})
-//   weights      dW_l = A_{l-1}^T dZ_l (split over the batch, FP32 atomics)
+// Parameters are kept as FP32 masters (Adam state beside them) and as
+// bfloat16 images in the order the matrix operands are read; every product
+// takes bfloat16 operands and accumulates in FP32.  Inference (k_mlp_fused)
+// and the training step (k_train: forward, backward and weight gradients)
+// are one kernel each, with the activations in registers and LDS.
 // The packed parameter layout (W row-major [in][out] then b, per layer) is
 // the one the oracle and the host API use.
 #include "common.h"
@@ -29,7 +24,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kIn = 8, kH = 128, kOut = 2;
-constexpr int kDims[6] = {kIn, kH, kH, kH, kH, kOut};
+constexpr int kDims[6] = {kIn, kH, kH, kH, kH, kOut};  // (constant indices only: in a kernel others read scratch)
 constexpr int kParams = 50946;
 constexpr int kLayers = 5;
 
@@ -59,10 +54,20 @@ __device__ __forceinline__ float erf_as(float x) {
     return copysignf(y, x);
 }
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erf_as(z * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_d(float z) {
-    const float cdf = 0.5f * (1.0f + erf_as(z * 0.70710678118654752f));
-    const float pdf = __expf(-0.5f * z * z) * 0.39894228040143268f;
-    return cdf + z * pdf;
+// gelu(z) and its derivative d = cdf + z pdf; erf's exponential exp(-z^2 / 2)
+// is the density's too.
+__device__ __forceinline__ float gelu_and_d(float z, float &d) {
+    const float ax = fabsf(z * 0.70710678118654752f);
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, ax, 1.0f));
+    float poly = fmaf(t, 1.061405429f, -1.453152027f);
+    poly = fmaf(t, poly, 1.421413741f);
+    poly = fmaf(t, poly, -0.284496736f);
+    poly = fmaf(t, poly, 0.254829592f);
+    poly *= t;
+    const float e = __expf(-ax * ax);
+    const float cdf = 0.5f * (1.0f + copysignf(fmaf(-poly, e, 1.0f), z));
+    d = fmaf(z, e * 0.39894228040143268f, cdf);
+    return z * cdf;
 }
 
 template <class T> __device__ __forceinline__ uint16_t load_bf16(const T *p);
@@ -130,81 +135,72 @@ struct EpiStore {  // c[row][col] = v
     int ld;
     __device__ void operator()(int row, int col, float v) const { c[int64_t(row) * ld + col] = v; }
 };
-struct EpiAdd {  // c[row][col] += v (split-K partial sums)
-    float *c;
-    int ld;
-    __device__ void operator()(int row, int col, float v) const { atomicAdd(&c[int64_t(row) * ld + col], v); }
-};
-struct EpiBiasGelu {  // z = v + bias; act = gelu(z) when act != NULL
-    float *z, *act;
-    const float *bias;
-    int ld;
-    __device__ void operator()(int row, int col, float v) const {
-        const float zz = v + bias[col];
-        z[int64_t(row) * ld + col] = zz;
-        if (act) act[int64_t(row) * ld + col] = gelu(zz);
-    }
-};
-struct EpiGeluD {  // dz = v * gelu'(zref)
-    float *dz;
-    const float *zref;
-    int ld;
-    __device__ void operator()(int row, int col, float v) const {
-        const int64_t k = int64_t(row) * ld + col;
-        dz[k] = v * gelu_d(zref[k]);
-    }
-};
-
 template <class TB, class Epi>
 void gemm(const float *a, const TB *b, const Gemm &g, const Epi &epi, int splits, hipStream_t s) {
     dim3 grid(uint32_t((g.M + kBM - 1) / kBM), uint32_t((g.N + kBN - 1) / kBN), uint32_t(splits));
     hipLaunchKernelGGL((k_gemm<TB, Epi>), grid, dim3(256), 0, s, a, b, g, epi);
 }
 
-// --------------------------------------------------------- elementwise
-__global__ void k_to_bf16(const float *__restrict__ p, uint16_t *__restrict__ q, int n) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) q[i] = to_bf16(p[i]);
-}
+// ------------------------------------------------------- training images
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-__global__ void k_fill(float *p, int64_t n, float v) {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
-}
+// The weights as A operands of v_mfma_f32_16x16x32_bf16 (lane l: row l % 16, k =
+// 8 (l / 16) + 0..7), for products whose B operand is the accumulator of the
+// layer before: k slot j of lane group g in K step ks is feature
+// 32 ks + 16 (j / 4) + 4 g + j % 4.  The seven products of the step in their
+// order: forward Z^T = W^T A^T of layers 1 (its K padded 8 -> 128 with zeros)
+// to 4, backward dA^T = W dZ^T of layers 4 to 2; then layer 5's two products,
+// its 2 outputs padded with zeros.
+constexpr int kProducts = 7;
+struct TrainImage {
+    uint16_t w[kProducts][8][4][64][8];
+    uint16_t w5f[4][64][8];
+    uint16_t w5b[8][64][8];
+};
 
-// dout = 2 (out - t) / n; loss += sum (out - t)^2 / n
-__global__ __launch_bounds__(256) void k_mse(const float *__restrict__ out, const float *__restrict__ t, int n,
-                                            float *__restrict__ dout, float *__restrict__ loss) {
-    __shared__ float part[4];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    float l = 0.0f;
-    if (i < n * kOut) {
-        const float d = out[i] - t[i];
-        dout[i] = 2.0f * d / float(n);
-        l = d * d / float(n);
+__device__ __forceinline__ int k_step(int f) { return f / 32; }
+__device__ __forceinline__ int k_group(int f) { return f % 16 / 4; }
+__device__ __forceinline__ int k_slot(int f) { return 4 * (f % 32 / 16) + f % 4; }
+
+// Parameter i's bfloat16 value v into the images that hold it.
+template <int l>
+__device__ __forceinline__ void put_layer(TrainImage *T, int i, uint16_t v) {
+    constexpr int dout = kDims[l + 1], size = kDims[l] * dout;
+    const int k = i - int(w_off(l));
+    if (k < 0 || k >= size) return;
+    const int in = k / dout, out = k % dout;
+    if constexpr (l == 0) {  // (the inputs are not an accumulator: feature k in slot k of group 0)
+        T->w[0][out / 16][0][out % 16][in] = v;
+    } else if constexpr (l < kLayers - 1) {
+        T->w[l][out / 16][k_step(in)][16 * k_group(in) + out % 16][k_slot(in)] = v;
+        T->w[7 - l][in / 16][k_step(out)][16 * k_group(out) + in % 16][k_slot(out)] = v;
+    } else {
+        T->w5f[k_step(in)][16 * k_group(in) + out][k_slot(in)] = v;
+        T->w5b[in / 16][in % 16][out] = v;
     }
-    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = l;
-    __syncthreads();
-    if (threadIdx.x == 0 && loss) atomicAdd(loss, part[0] + part[1] + part[2] + part[3]);
+}
+__device__ __forceinline__ void put_image(TrainImage *T, int i, uint16_t v) {
+    put_layer<0>(T, i, v);
+    put_layer<1>(T, i, v);
+    put_layer<2>(T, i, v);
+    put_layer<3>(T, i, v);
+    put_layer<4>(T, i, v);
 }
 
-// db[c] += column sums of dz[n][ld] over a chunk of rows; grid (chunks, cols)
-__global__ __launch_bounds__(256) void k_colsum(const float *__restrict__ dz, int n, int ld, float *__restrict__ db) {
-    __shared__ float part[4];
-    const int c = blockIdx.y;
-    float s = 0.0f;
-    for (int r = blockIdx.x * 256 + threadIdx.x; r < n; r += gridDim.x * 256) s += dz[int64_t(r) * ld + c];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&db[c], part[0] + part[1] + part[2] + part[3]);
+// New parameters: the bfloat16 copies, and no Adam state.
+__global__ void k_set_params(const float *__restrict__ p, uint16_t *__restrict__ pb, TrainImage *__restrict__ T,
+                             float *__restrict__ m, float *__restrict__ v, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    pb[i] = to_bf16(p[i]);
+    put_image(T, i, pb[i]);
+    m[i] = v[i] = 0.0f;
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 masters; refreshes the bfloat16 copy.
-__global__ void k_adam(float *__restrict__ p, uint16_t *__restrict__ pb, const float *__restrict__ g,
-                       float *__restrict__ m, float *__restrict__ v, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
+// Adam (Kingma & Ba 2015) on the FP32 masters; refreshes the bfloat16 copies.
+__global__ void k_adam(float *__restrict__ p, uint16_t *__restrict__ pb, TrainImage *__restrict__ T,
+                       const float *__restrict__ g, float *__restrict__ m, float *__restrict__ v, int n, float lr,
+                       float b1, float b2, float eps, float c1, float c2) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const float gi = g[i];
@@ -215,6 +211,7 @@ __global__ void k_adam(float *__restrict__ p, uint16_t *__restrict__ pb, const f
     const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     p[i] = pi;
     pb[i] = to_bf16(pi);
+    put_image(T, i, pb[i]);
 }
 
 // ------------------------------------------------------- fused forward
@@ -354,6 +351,317 @@ __global__ __launch_bounds__(kFusedThreads) void k_mlp_fused(const float *__rest
     }
 }
 
+// --------------------------------------------------------- training step
+// Forward, backward and weight gradients of kTrainRows rows per workgroup and
+// turn, 16 per wave: Z^T = W^T A^T, so a layer's accumulator (lane = row,
+// registers = features) is the next product's B operand, forward and
+// backward, and never leaves the registers.  GELU' of the four hidden layers
+// waits there too, in FP32, from the forward pass for the backward.  The
+// weight gradients dW = A^T dZ contract over the rows: each layer's A and dZ
+// are put into LDS as bfloat16 (what the product rounds them to) with the
+// rows of a feature consecutive, and each wave computes 32 columns of dW.
+// Bias gradients are FP32 sums of the unrounded dZ.  Each workgroup leaves
+// its partial gradient (stored in its first turn, added to in later ones) and
+// loss for k_train_reduce.
+//
+// One wave per SIMD (512 registers).  The layers are loops, not unrolled: at
+// the trainer's 16,384 rows each CU has one turn of one workgroup, which
+// would wait for 68 KB of straight-line code (78 us; as loops 69, and 43 with
+// the weights' registers named, see below).  GELU' moves through the four
+// register arrays by copies.  What is left is about a third of it VALU work,
+// the rest the layers' dependent chain and the 52 MB of partials.  The step
+// with k_train_reduce (12 us, at the memory's rate) takes 55 us; with one
+// tiled product per layer and direction, atomics for the split weight
+// gradients and the activations in memory it took 708.
+constexpr int kTrainRows = 64, kTrainThreads = 256;
+constexpr int kRowPad = kTrainRows + 8;  // 144 bytes per feature: 16 lanes' 16-byte reads hit distinct banks
+constexpr int kPart = kParams + 1;       // partial gradient, then the loss
+
+struct TrainLds {
+    bf16x8 w[8][4][64];          // the current product's weights
+    uint16_t a[4][kH][kRowPad];  // A1..A4
+    uint16_t dz[kH][kRowPad];    // the current layer's dZ
+    uint16_t x[16][kRowPad];     // the inputs (rows 8..15 zero)
+    uint16_t d5[16][kRowPad];    // dZ5 (rows 2..15 zero)
+    float b[4][kH];
+    float db[4][4][kH];          // per wave: bias gradients of the hidden layers
+    float db5[4][kOut];
+    float loss[4];
+};
+static_assert(sizeof(TrainLds) <= 160 * 1024, "one workgroup per CU");
+
+__device__ __forceinline__ floatx4 mfma16(const bf16x8 &a, const bf16x8 &b, const floatx4 &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Sum over each row of 16 lanes, in its last lane.
+template <int CTRL>
+__device__ __forceinline__ float row_shr(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float row_sum(float v) {
+    v += row_shr<0x111>(v);
+    v += row_shr<0x112>(v);
+    v += row_shr<0x114>(v);
+    v += row_shr<0x118>(v);
+    return v;
+}
+
+// A layer's 32 values of this lane (its row, features 16 mb + 4 g + r) ->
+// B operands, and into LDS with the rows of a feature consecutive.
+__device__ __forceinline__ void to_operands(const float (&v)[32], bf16x8 (&B)[4], uint16_t (*lds)[kRowPad], int g,
+                                            int row) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        uint16_t q[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            q[j] = to_bf16(v[8 * s + j]);
+            lds[32 * s + 16 * (j / 4) + 4 * g + j % 4][row] = q[j];
+        }
+        B[s] = pack8(q);
+    }
+}
+
+__global__ __launch_bounds__(kTrainThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_train(
+    const float *__restrict__ x, const float *__restrict__ t, int n, const TrainImage *__restrict__ T,
+    const float *__restrict__ p, float *__restrict__ part) {
+    extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+    TrainLds &S = *reinterpret_cast<TrainLds *>(lds_raw);
+    const int tid = threadIdx.x, wave = tid >> 6;
+    for (int e = tid; e < 16 * kRowPad; e += kTrainThreads) (&S.x[0][0])[e] = (&S.d5[0][0])[e] = 0;
+    constexpr int kStride = kH * kH + kH;  // from one hidden layer's biases to the next's
+    for (int e = tid; e < 4 * kH; e += kTrainThreads) S.b[e / kH][e % kH] = p[b_off(0) + e / kH * kStride + e % kH];
+    for (int e = tid; e < 16 * kH; e += kTrainThreads) (&S.db[0][0][0])[e] = 0.0f;
+    const float b50 = p[b_off(4)], b51 = p[b_off(4) + 1];
+    const bf16x8 *w5f = reinterpret_cast<const bf16x8 *>(T->w5f), *w5b = reinterpret_cast<const bf16x8 *>(T->w5b);
+    // the products' weights pass through S.w; each is loaded into registers
+    // during the product before
+    // (eight named registers: an array here went to scratch memory, whose
+    // stores waited for the loads)
+    static_assert(sizeof(S.w) == 8 * 16 * kTrainThreads, "eight 16-byte loads per thread");
+    uint4 pre0, pre1, pre2, pre3, pre4, pre5, pre6, pre7;
+    const auto prefetch = [&](int k) {
+        const uint4 *src = reinterpret_cast<const uint4 *>(T->w[k]) + tid;
+        pre0 = src[0], pre1 = src[kTrainThreads], pre2 = src[2 * kTrainThreads], pre3 = src[3 * kTrainThreads];
+        src += 4 * kTrainThreads;
+        pre4 = src[0], pre5 = src[kTrainThreads], pre6 = src[2 * kTrainThreads], pre7 = src[3 * kTrainThreads];
+    };
+    const auto stage = [&] {
+        uint4 *dst = reinterpret_cast<uint4 *>(S.w) + tid;
+        dst[0] = pre0, dst[kTrainThreads] = pre1, dst[2 * kTrainThreads] = pre2, dst[3 * kTrainThreads] = pre3;
+        dst += 4 * kTrainThreads;
+        dst[0] = pre4, dst[kTrainThreads] = pre5, dst[2 * kTrainThreads] = pre6, dst[3 * kTrainThreads] = pre7;
+    };
+
+    const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    float *out = part + size_t(blockIdx.x) * kPart;
+    float loss = 0.0f, db50 = 0.0f, db51 = 0.0f;
+    const float inv_n = 1.0f / float(n);
+    prefetch(0);
+    __syncthreads();
+
+    const int tiles = (n + kTrainRows - 1) / kTrainRows;
+#pragma unroll 1
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+        const int lr = 16 * wave + c;  // this lane's row of the workgroup's rows
+        const int64_t row = int64_t(tile) * kTrainRows + lr;
+        const bool valid = row < n, again = tile != int(blockIdx.x);
+        // a weight gradient of this turn into the workgroup's partial
+        const auto put = [&](uint32_t at, float v) { out[at] = again ? out[at] + v : v; };
+        bf16x8 B[4];
+        {
+            uint16_t q[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) q[j] = (g == 0 && valid) ? to_bf16(x[row * kIn + j]) : uint16_t(0);
+            if (g == 0)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) S.x[j][lr] = q[j];
+            B[0] = pack8(q);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) q[j] = 0;
+            B[1] = B[2] = B[3] = pack8(q);
+        }
+        float gd[4][32];  // gelu' of hidden layers 1..4 (the newest in gd[3])
+#pragma unroll
+        for (int k = 0; k < 32; ++k) gd[1][k] = gd[2][k] = gd[3][k] = 0.0f;
+#pragma unroll 1
+        for (int l = 0; l < 4; ++l) {
+            stage();
+            prefetch(l + 1);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 32; ++k) {
+                gd[0][k] = gd[1][k];
+                gd[1][k] = gd[2][k];
+                gd[2][k] = gd[3][k];
+            }
+            float a[32];
+#pragma unroll
+            for (int mb = 0; mb < 8; mb += 4) {
+                floatx4 z[4] = {zero, zero, zero, zero};
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) z[q] = mfma16(S.w[mb + q][ks][lane], B[ks], z[q]);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int k = 4 * (mb + q) + r;
+                        a[k] = gelu_and_d(z[q][r] + S.b[l][16 * (mb + q) + 4 * g + r], gd[3][k]);
+                    }
+            }
+            to_operands(a, B, S.a[l], g, lr);
+            __syncthreads();  // S.w is free
+        }
+        // output, loss, dZ5 (lanes of group 0 hold their row's two values)
+        floatx4 o = zero;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) o = mfma16(w5f[ks * 64 + lane], B[ks], o);
+        float d0 = 0.0f, d1 = 0.0f;
+        if (g == 0 && valid) {
+            d0 = o[0] + b50 - t[row * kOut];
+            d1 = o[1] + b51 - t[row * kOut + 1];
+        }
+        loss += (d0 * d0 + d1 * d1) * inv_n;
+        d0 *= 2.0f * inv_n;
+        d1 *= 2.0f * inv_n;
+        db50 += d0;
+        db51 += d1;
+        uint16_t q5[8] = {to_bf16(d0), to_bf16(d1), 0, 0, 0, 0, 0, 0};
+        if (g == 0) {
+            S.d5[0][lr] = q5[0];
+            S.d5[1][lr] = q5[1];
+        }
+        const bf16x8 b5 = pack8(q5);  // (zero outside group 0)
+        float dz[32];
+#pragma unroll
+        for (int mb = 0; mb < 8; ++mb) {
+            const floatx4 da = mfma16(w5b[mb * 64 + lane], b5, zero);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dz[4 * mb + r] = da[r] * gd[3][4 * mb + r];
+        }
+        __syncthreads();  // S.a and S.d5 are complete
+        // dW5 = A4^T dZ5, this wave's 32 rows
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            floatx4 v = zero;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+                v = mfma16(*reinterpret_cast<const bf16x8 *>(&S.a[3][32 * wave + 16 * k + c][32 * ks + 8 * g]),
+                           *reinterpret_cast<const bf16x8 *>(&S.d5[c][32 * ks + 8 * g]), v);
+            if (c < kOut)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) put(uint32_t(w_off(4)) + (32 * wave + 16 * k + 4 * g + r) * kOut + c, v[r]);
+        }
+        // dZ of hidden layer l + 1: the gradients of its weights (input: A of
+        // layer l, or x) and biases, then the dZ below
+#pragma unroll 1
+        for (int l = 3; l >= 0; --l) {
+            to_operands(dz, B, S.dz, g, lr);
+#pragma unroll
+            for (int k = 0; k < 32; ++k) {
+                const float s = row_sum(dz[k]);
+                if (c == 15) atomicAdd(&S.db[wave][l][16 * (k / 4) + 4 * g + k % 4], s);  // (no other adds here)
+            }
+            if (l > 0) {
+                stage();
+                prefetch(l > 1 ? 8 - l : 0);  // products 4, 5, 6 are staged at l = 3, 2, 1
+            }
+            __syncthreads();
+            if (l > 0) {
+#pragma unroll
+                for (int mb = 0; mb < 8; mb += 4) {
+                    floatx4 z[4] = {zero, zero, zero, zero};
+#pragma unroll
+                    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) z[q] = mfma16(S.w[mb + q][ks][lane], B[ks], z[q]);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) dz[4 * (mb + q) + r] = z[q][r] * gd[2][4 * (mb + q) + r];
+                }
+#pragma unroll
+                for (int k = 0; k < 32; ++k) {
+                    gd[2][k] = gd[1][k];
+                    gd[1][k] = gd[0][k];
+                }
+            }
+            // dW = A^T dZ over the workgroup's rows, this wave's 32 columns
+            bf16x8 bz[2][2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb)
+                    bz[ks][nb] = *reinterpret_cast<const bf16x8 *>(&S.dz[32 * wave + 16 * nb + c][32 * ks + 8 * g]);
+            const uint16_t(*a)[kRowPad] = l > 0 ? S.a[l - 1] : S.x;
+            uint32_t at = (l == 0 ? uint32_t(w_off(0)) : uint32_t(w_off(1)) + uint32_t(l - 1) * kStride) +
+                          uint32_t(4 * g * kH + 32 * wave + c);
+            const bool rows = l > 0 || g < 2;
+#pragma unroll 2
+            for (int mb = 0; mb < (l > 0 ? 8 : 1); ++mb, at += 16 * kH) {
+                const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(&a[16 * mb + c][8 * g]);
+                const bf16x8 a1 = *reinterpret_cast<const bf16x8 *>(&a[16 * mb + c][32 + 8 * g]);
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    const floatx4 v = mfma16(a1, bz[1][nb], mfma16(a0, bz[0][nb], zero));
+                    if (rows)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) put(at + uint32_t(r * kH + 16 * nb), v[r]);
+                }
+            }
+            __syncthreads();  // S.dz and S.w are free
+        }
+    }
+
+    loss = row_sum(loss);
+    db50 = row_sum(db50);
+    db51 = row_sum(db51);
+    if ((tid & 63) == 15) {
+        S.loss[wave] = loss;
+        S.db5[wave][0] = db50;
+        S.db5[wave][1] = db51;
+    }
+    __syncthreads();
+    for (int e = tid; e < 4 * kH; e += kTrainThreads) {
+        const int l = e / kH, f = e % kH;
+        out[b_off(0) + l * kStride + f] = (S.db[0][l][f] + S.db[1][l][f]) + (S.db[2][l][f] + S.db[3][l][f]);
+    }
+    if (tid < kOut) out[b_off(4) + tid] = (S.db5[0][tid] + S.db5[1][tid]) + (S.db5[2][tid] + S.db5[3][tid]);
+    if (tid == 0) out[kParams] = (S.loss[0] + S.loss[1]) + (S.loss[2] + S.loss[3]);
+}
+
+// The workgroups' partial gradients summed in FP32, in a fixed order: 64
+// parameters per block, a quarter of the partials per wave.
+__global__ __launch_bounds__(256) void k_train_reduce(const float *__restrict__ part, int parts,
+                                                     float *__restrict__ g, float *__restrict__ grad,
+                                                     float *__restrict__ loss) {
+    __shared__ float sum[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    float s[8] = {};
+    if (i < kPart) {
+        int k = wave;
+        for (; k + 28 < parts; k += 32)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s[j] += part[size_t(k + 4 * j) * kPart + i];
+        for (; k < parts; k += 4) s[0] += part[size_t(k) * kPart + i];
+    }
+    sum[wave][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    __syncthreads();
+    if (wave != 0 || i >= kPart) return;
+    const float v = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
+    if (i < kParams) {
+        g[i] = v;
+        if (grad) grad[i] = v;
+    } else if (loss) {
+        *loss += v;
+    }
+}
+
 }  // namespace
 
 // ------------------------------------------------------------- handle
@@ -364,49 +672,38 @@ struct amh_mlp_s {
     uint16_t *pb = nullptr;                                         // bfloat16 copy
     FusedLds *image = nullptr;  // weights in the fused forward's LDS order
     bool image_stale = true;
-    float *z[kLayers] = {};    // [batch][dims[l+1]] pre-activations
-    float *act[kLayers] = {};  // [batch][dims[l]] inputs of layer l (act[0] unused: the caller's x)
-    float *dz[2] = {};         // [batch][128] ping-pong gradients
-    float *loss = nullptr;     // [1]
+    TrainImage *train = nullptr;  // weights in the training step's operand order
+    float *part = nullptr;        // [workgroups][kPart] partial gradients
     int64_t step = 0;
 };
 
 namespace {
 int g_cus = 0;
 int g_fused = -1;  // -1 unknown, 0 no, 1 yes
-// The fused forward needs kFusedLds bytes of LDS in one workgroup.
+// The fused kernels' LDS (110 KB and 137 KB in one workgroup).
 bool fused_ok() {
     if (g_fused >= 0) return g_fused == 1;
-    int dev = 0, lds = 0, cus = 0;
+    int dev = 0, cus = 0;
     g_fused = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return false;
-    if (size_t(lds) < kFusedLds) return false;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mlp_fused), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            int(kFusedLds)) != hipSuccess)
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mlp_fused), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            int(kFusedLds)) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void *>(&k_train), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            int(sizeof(TrainLds))) != hipSuccess)
         return false;
     g_cus = cus;
     g_fused = 1;
     return true;
 }
 
-size_t mlp_bytes(int32_t batch) {
-    const size_t B = size_t(batch);
-    return 4 * kParams * 4 + kParams * 2 + kFusedLds + B * kH * 4 * (kLayers + kLayers + 2) + 64 * 256;
-}
+// Workgroups of the training step on n rows: one per CU at most.
+int train_groups(int n) { return std::min(g_cus, (n + kTrainRows - 1) / kTrainRows); }
 
-// forward of rows [0, n) of x (n <= batch) into M->z[4] (n x 2)
-void forward_batch(amh_mlp_s *M, const float *x, int n, hipStream_t s) {
-    const float *in = x;
-    for (int l = 0; l < kLayers; ++l) {
-        const int din = kDims[l], dout = kDims[l + 1];
-        Gemm g{n, dout, din, din, 1, dout, 1, din};
-        EpiBiasGelu e{M->z[l], l < kLayers - 1 ? M->act[l + 1] : nullptr, M->p + b_off(l), dout};
-        gemm(in, M->pb + w_off(l), g, e, 1, s);
-        if (l < kLayers - 1) in = M->act[l + 1];
-    }
+int stage_image(amh_mlp_s *M, hipStream_t s) {
+    hipLaunchKernelGGL(k_fused_stage, dim3(64), dim3(256), 0, s, M->pb, M->p, M->image);
+    M->image_stale = false;
+    return AMH_OK;
 }
 }  // namespace
 
@@ -415,28 +712,27 @@ extern "C" int amh_mlp_create(void **mlp, int32_t batch_max, void *stream) {
         set_error("amh_mlp_create: invalid argument");
         return AMH_E_ARG;
     }
+    if (!fused_ok()) return check_hip(hipErrorInvalidDevice, "amh_mlp_create: the kernels' LDS");
     amh_mlp_s *M = new amh_mlp_s;
     M->batch = batch_max;
-    const size_t bytes = mlp_bytes(batch_max);
-    if (int r = check_hip(hipMalloc(&M->buf, bytes), "amh_mlp_create")) {
+    const auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const size_t vec = al(kParams * 4), half = al(kParams * 2), train = al(sizeof(TrainImage));
+    const size_t held = 4 * vec + half + al(kFusedLds) + train;
+    if (int r = check_hip(hipMalloc(&M->buf, held + size_t(train_groups(batch_max)) * kPart * 4), "amh_mlp_create")) {
         delete M;
         return r;
     }
     char *q = static_cast<char *>(M->buf);
-    auto take = [&](size_t b) { char *r = q; q += (b + 255) & ~size_t(255); return r; };
-    M->p = reinterpret_cast<float *>(take(kParams * 4));
-    M->g = reinterpret_cast<float *>(take(kParams * 4));
-    M->m = reinterpret_cast<float *>(take(kParams * 4));
-    M->v = reinterpret_cast<float *>(take(kParams * 4));
-    M->pb = reinterpret_cast<uint16_t *>(take(kParams * 2));
-    M->image = reinterpret_cast<FusedLds *>(take(kFusedLds));
-    const size_t B = size_t(batch_max);
-    for (int l = 0; l < kLayers; ++l) M->z[l] = reinterpret_cast<float *>(take(B * kH * 4));
-    for (int l = 0; l < kLayers; ++l) M->act[l] = reinterpret_cast<float *>(take(B * kH * 4));
-    M->dz[0] = reinterpret_cast<float *>(take(B * kH * 4));
-    M->dz[1] = reinterpret_cast<float *>(take(B * kH * 4));
-    M->loss = reinterpret_cast<float *>(take(256));
-    if (int r = check_hip(hipMemsetAsync(M->buf, 0, bytes, static_cast<hipStream_t>(stream)), "amh_mlp_create")) {
+    const auto take = [&](size_t b) { char *r = q; q += b; return r; };
+    M->p = reinterpret_cast<float *>(take(vec));
+    M->g = reinterpret_cast<float *>(take(vec));
+    M->m = reinterpret_cast<float *>(take(vec));
+    M->v = reinterpret_cast<float *>(take(vec));
+    M->pb = reinterpret_cast<uint16_t *>(take(half));
+    M->image = reinterpret_cast<FusedLds *>(take(al(kFusedLds)));
+    M->train = reinterpret_cast<TrainImage *>(take(train));
+    M->part = reinterpret_cast<float *>(q);
+    if (int r = check_hip(hipMemsetAsync(M->buf, 0, held, static_cast<hipStream_t>(stream)), "amh_mlp_create")) {
         (void)hipFree(M->buf);
         delete M;
         return r;
@@ -458,15 +754,10 @@ extern "C" int amh_mlp_set_params(void *mlp, const float *host, void *stream) {
     if (!M || !host) { set_error("amh_mlp_set_params: NULL"); return AMH_E_ARG; }
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (int r = check_hip(hipMemcpyAsync(M->p, host, kParams * 4, hipMemcpyHostToDevice, s), "set_params")) return r;
-    hipLaunchKernelGGL(k_to_bf16, dim3((kParams + 255) / 256), dim3(256), 0, s, M->p, M->pb, kParams);
-    hipLaunchKernelGGL(k_fill, dim3((kParams + 255) / 256), dim3(256), 0, s, M->m, int64_t(kParams), 0.0f);
-    hipLaunchKernelGGL(k_fill, dim3((kParams + 255) / 256), dim3(256), 0, s, M->v, int64_t(kParams), 0.0f);
+    hipLaunchKernelGGL(k_set_params, dim3((kParams + 255) / 256), dim3(256), 0, s, M->p, M->pb, M->train, M->m, M->v,
+                       kParams);
     M->step = 0;
-    M->image_stale = true;
-    if (fused_ok()) {  // the fused forward's weight image, now rather than at the first forward
-        hipLaunchKernelGGL(k_fused_stage, dim3(64), dim3(256), 0, s, M->pb, M->p, M->image);
-        M->image_stale = false;
-    }
+    stage_image(M, s);  // the forward's weight image, now rather than at the first forward
     AMH_LAUNCH_CHECK("amh_mlp_set_params");
     return check_hip(hipStreamSynchronize(s), "set_params");
 }
@@ -479,32 +770,17 @@ extern "C" int amh_mlp_get_params(void *mlp, float *host, void *stream) {
     return check_hip(hipStreamSynchronize(s), "get_params");
 }
 
-// Inference: out[n][2] for x[n][8], in batches of the handle's size.
+// Inference: out[n][2] for x[n][8].
 extern "C" int amh_mlp_forward(void *mlp, const float *x, int64_t n, float *out, void *stream) {
     amh_mlp_s *M = static_cast<amh_mlp_s *>(mlp);
     if (!M || (n > 0 && (!x || !out)) || n < 0) { set_error("amh_mlp_forward: invalid argument"); return AMH_E_ARG; }
     hipStream_t s = static_cast<hipStream_t>(stream);
     amh::ProfScope ps_("mlp_forward", s);
     if (n == 0) return AMH_OK;
-    if (fused_ok()) {
-        const int64_t tiles = (n + 31) / 32;
-        const uint32_t grid = uint32_t(std::min<int64_t>(g_cus, (tiles + kFusedThreads / 64 - 1) / (kFusedThreads / 64)));
-        if (M->image_stale) {
-            hipLaunchKernelGGL(k_fused_stage, dim3(64), dim3(256), 0, s, M->pb, M->p, M->image);
-            M->image_stale = false;
-        }
-        hipLaunchKernelGGL(k_mlp_fused, dim3(grid), dim3(kFusedThreads), kFusedLds, s, x, n, M->image, out);
-        AMH_LAUNCH_CHECK("amh_mlp_forward");
-        return AMH_OK;
-    }
-    for (int64_t i = 0; i < n; i += M->batch) {
-        const int c = int(std::min<int64_t>(M->batch, n - i));
-        forward_batch(M, x + i * kIn, c, s);
-        if (int r = check_hip(hipMemcpyAsync(out + i * kOut, M->z[kLayers - 1], size_t(c) * kOut * 4,
-                                             hipMemcpyDeviceToDevice, s),
-                              "amh_mlp_forward"))
-            return r;
-    }
+    const int64_t tiles = (n + 31) / 32;
+    const uint32_t grid = uint32_t(std::min<int64_t>(g_cus, (tiles + kFusedThreads / 64 - 1) / (kFusedThreads / 64)));
+    if (M->image_stale) stage_image(M, s);
+    hipLaunchKernelGGL(k_mlp_fused, dim3(grid), dim3(kFusedThreads), kFusedLds, s, x, n, M->image, out);
     AMH_LAUNCH_CHECK("amh_mlp_forward");
     return AMH_OK;
 }
@@ -518,32 +794,10 @@ extern "C" int amh_mlp_gradients(void *mlp, const float *x, const float *t, int3
     if (!M || !x || !t || n <= 0 || n > M->batch) { set_error("amh_mlp_gradients: invalid argument"); return AMH_E_ARG; }
     hipStream_t s = static_cast<hipStream_t>(stream);
     amh::ProfScope ps_("mlp_gradients", s);
-    forward_batch(M, x, n, s);
-    hipLaunchKernelGGL(k_fill, dim3((kParams + 255) / 256), dim3(256), 0, s, M->g, int64_t(kParams), 0.0f);
-    float *dcur = M->dz[0], *dnext = M->dz[1];
-    hipLaunchKernelGGL(k_mse, dim3((n * kOut + 255) / 256), dim3(256), 0, s, M->z[kLayers - 1], t, n, dcur, loss_dev);
-    // the weight gradients sum over the batch: split it over blocks (~512
-    // rows each) that add their partial products
-    const int splits = std::max(1, std::min(64, n / 512));
-    const int klen = ((n + splits - 1) / splits + kBK - 1) / kBK * kBK;
-    for (int l = kLayers - 1; l >= 0; --l) {
-        const int din = kDims[l], dout = kDims[l + 1];
-        const float *ain = l == 0 ? x : M->act[l];
-        // dW_l = A_{l-1}^T dz_l: M = din, N = dout, K = n
-        Gemm gw{din, dout, n, 1, din, dout, 1, klen};
-        gemm(ain, static_cast<const float *>(dcur), gw, EpiAdd{M->g + w_off(l), dout}, (n + klen - 1) / klen, s);
-        hipLaunchKernelGGL(k_colsum, dim3(uint32_t(std::min(64, (n + 255) / 256)), uint32_t(dout)), dim3(256), 0, s,
-                           dcur, n, dout, M->g + b_off(l));
-        if (l == 0) break;
-        // dz_{l-1} = (dz_l W_l^T) * gelu'(z_{l-1}): M = n, N = din, K = dout
-        Gemm gd{n, din, dout, dout, 1, 1, dout, dout};
-        gemm(dcur, M->pb + w_off(l), gd, EpiGeluD{dnext, M->z[l - 1], din}, 1, s);
-        std::swap(dcur, dnext);
-    }
-    if (grad && grad != M->g) {
-        if (int r = check_hip(hipMemcpyAsync(grad, M->g, kParams * 4, hipMemcpyDeviceToDevice, s), "gradients"))
-            return r;
-    }
+    const int groups = train_groups(n);
+    hipLaunchKernelGGL(k_train, dim3(uint32_t(groups)), dim3(kTrainThreads), sizeof(TrainLds), s, x, t, int(n),
+                       M->train, M->p, M->part);
+    hipLaunchKernelGGL(k_train_reduce, dim3((kPart + 63) / 64), dim3(256), 0, s, M->part, groups, M->g, grad, loss_dev);
     AMH_LAUNCH_CHECK("amh_mlp_gradients");
     return AMH_OK;
 }
@@ -557,8 +811,8 @@ extern "C" int amh_mlp_adam_step(void *mlp, float lr, void *stream) {
     M->image_stale = true;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - std::pow(b1, float(M->step)), c2 = 1.0f - std::pow(b2, float(M->step));
-    hipLaunchKernelGGL(k_adam, dim3((kParams + 255) / 256), dim3(256), 0, s, M->p, M->pb, M->g, M->m, M->v, kParams,
-                       lr, b1, b2, 1e-8f, c1, c2);
+    hipLaunchKernelGGL(k_adam, dim3((kParams + 255) / 256), dim3(256), 0, s, M->p, M->pb, M->train, M->g, M->m, M->v,
+                       kParams, lr, b1, b2, 1e-8f, c1, c2);
     AMH_LAUNCH_CHECK("amh_mlp_adam_step");
     return AMH_OK;
 }

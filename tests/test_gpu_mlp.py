@@ -99,6 +99,59 @@ def test_gradients_match_oracle():
             o_ += size
 
 
+def _gradients(h, x, t):
+    T = G.torch()
+    dx, dt = G.to_dev(x), G.to_dev(t)
+    dg, dl = G.zeros(op.MLP_PARAMS, T.float32), G.zeros(1, T.float32)
+    G.check(G.lib().amh_mlp_gradients(h, G.dptr(dx), G.dptr(dt), len(x), G.dptr(dg), G.dptr(dl), G.stream()), "grad")
+    return G.to_host(dg, np.float32).astype(np.float64), float(G.to_host(dl, np.float32)[0])
+
+
+@pytest.mark.parametrize("n", [1, 15, 64, 65])
+def test_gradients_of_few_rows_match_oracle(n):
+    """Row counts around a wave's 16 and a workgroup's 64; tolerances as in
+    the test above, for the whole gradient."""
+    rng = np.random.default_rng(100 + n)
+    p = _mlp_params(rng)
+    x, t = rng.normal(0, 1, (n, 8)).astype(np.float32), rng.normal(0, 1, (n, 2)).astype(np.float32)
+    want = np.zeros(op.MLP_PARAMS)
+    loss_want = op.oracle().or_mlp_grad(op.ptr(p), op.ptr(x), op.ptr(t), n, 1, op.ptr(want))
+    h = _mlp(n, p)
+    try:
+        G.log(f"mlp gradients {n} rows")
+        got, loss = _gradients(h, x, t)
+    finally:
+        G.lib().amh_mlp_destroy(h)
+    assert abs(loss - loss_want) <= 1e-3 * loss_want
+    assert np.linalg.norm(got - want) < 1e-2 * np.linalg.norm(want)
+
+
+def test_gradients_over_several_turns_add_up():
+    """More rows than one turn of every workgroup takes: the gradient is the
+    weighted mean of its parts' (which one turn each computes), to FP32
+    rounding of sums over the rows (relative error at most about sqrt(n) 2^-24
+    = 1e-5; 1e-4 asserted)."""
+    rng = np.random.default_rng(7)
+    p = _mlp_params(rng)
+    parts = [16000, 9000, 777]
+    n = sum(parts)
+    x, t = rng.normal(0, 1, (n, 8)).astype(np.float32), rng.normal(0, 1, (n, 2)).astype(np.float32)
+    h = _mlp(n, p)
+    try:
+        G.log(f"mlp gradients {n} rows")
+        got, loss = _gradients(h, x, t)
+        want, loss_want, at = np.zeros(op.MLP_PARAMS), 0.0, 0
+        for k in parts:
+            g, l_ = _gradients(h, x[at:at + k], t[at:at + k])
+            want += g * (k / n)
+            loss_want += l_ * (k / n)
+            at += k
+    finally:
+        G.lib().amh_mlp_destroy(h)
+    assert abs(loss - loss_want) <= 1e-4 * loss_want
+    assert np.linalg.norm(got - want) <= 1e-4 * np.linalg.norm(want)
+
+
 def test_adam_training_reduces_loss():
     """A few hundred Adam steps on a smooth target (the identity on two
     inputs plus a bend) cut the loss by well over an order of magnitude."""
