@@ -143,6 +143,43 @@ def test_blob_stats_and_grouping(which, golden_cfg1):
         assert (bop[lab < 0] == -1).all()
 
 
+@pytest.mark.parametrize("w,h,cover", [(64, 64, 0.5), (64, 65, 0.6), (65, 31, 0.6), (129, 33, 0.3), (200, 161, 0.62),
+                                       (1, 1, 1.0), (300, 7, 0.45)])
+def test_dithered_frames_around_tile_edges(w, h, cover):
+    """Random dithers (hundreds of blobs in a tile, blobs across tile edges)
+    at one tile, one pixel more, and ragged sizes: labels, statistics and
+    grouping are exactly those of the oracle's labels."""
+    rng = np.random.default_rng(w * 1000 + h)
+    fr = rng.integers(0, 256, (h, w, 4)).astype(np.uint8)
+    fr[..., 3] = np.where(rng.uniform(size=(h, w)) < cover, rng.integers(1, 256, (h, w)), 0)
+    G.log(f"dither {w}x{h} {cover}")
+    _, lab_d = _segment(fr)
+    lab, n = op.segment(fr)
+    assert (G.to_host(lab_d, np.int32) == lab).all()
+    nb, bop, stats, first, plist, _ = _stats_and_groups(fr)
+    roots = np.unique(lab[lab >= 0])
+    assert nb == n == roots.size
+    want = np.where(lab >= 0, np.searchsorted(roots, lab), -1)
+    assert (bop == want).all()
+    idx = np.flatnonzero(want >= 0)
+    order = idx[np.argsort(want[idx], kind="stable")]
+    assert (plist[:idx.size] == order).all()
+    counts = np.bincount(want[idx], minlength=nb)
+    assert (first == np.concatenate([[0], np.cumsum(counts)])).all()
+    stored, _ = op.ingest(synth.to_words(fr), 1)
+    x, y = idx % w, idx // w
+    s = stats[:nb]
+    assert [v.count for v in s] == counts.tolist() and [v.first for v in s] == roots.tolist()
+    for got, value in (("sum_x", x), ("sum_y", y)):
+        assert [getattr(v, got) for v in s] == [int(q) for q in np.bincount(want[idx], value, minlength=nb)]
+    for k in range(4):
+        sums = np.bincount(want[idx], (stored[idx] >> (8 * k)) & 255, minlength=nb)
+        assert [v.sum_c[k] for v in s] == [int(q) for q in sums]
+    for b in range(0, nb, max(1, nb // 50)):
+        m = want[idx] == b
+        assert (s[b].x1, s[b].y1, s[b].x2, s[b].y2) == (x[m].min(), y[m].min(), x[m].max(), y[m].max())
+
+
 def _group(bop_host, nb):
     T = G.torch()
     lib = G.lib()
@@ -190,6 +227,24 @@ def test_group_pixels_any_blob_count(case):
     want = idx[np.argsort(bop[idx], kind="stable")]
     assert np.array_equal(plist[:idx.size], want)
     assert ws <= 24 * bop.size + 16 * nb + (1 << 20)
+
+
+@pytest.mark.parametrize("n,nb,kind", [(4096, 1024, "any"), (4096, 1025, "any"), (4097, 1024, "any"),  # one workgroup
+                                       (2048 * 31 + 5, 2048, "band"), (100_003, 3000, "few")])
+def test_group_pixels_at_path_edges(n, nb, kind):
+    """The one-workgroup grouping's limits and just beyond them; a band of
+    pixels of as many blobs as it has pixels; few of many blobs present."""
+    rng = np.random.default_rng(n + nb)
+    bop = rng.integers(-1, nb, n).astype(np.int32)
+    if kind == "band":
+        bop[:2048] = rng.permutation(nb)
+    elif kind == "few":
+        bop = rng.choice([-1, 0, 1, 2, 1500, 2999], n).astype(np.int32)
+    G.log(f"group pixels {n}, {nb} blobs, {kind}")
+    first, plist, _ = _group(bop, nb)
+    idx = np.flatnonzero(bop >= 0)
+    assert np.array_equal(first, np.concatenate([[0], np.cumsum(np.bincount(bop[idx], minlength=nb))]))
+    assert np.array_equal(plist[:idx.size], idx[np.argsort(bop[idx], kind="stable")])
 
 
 def test_engine_detects_checkerboard_alpha():
