@@ -50,17 +50,20 @@ __host__ __device__ __forceinline__ uint32_t ceil_log2(uint32_t n) {
 
 // Balanced 4-round Feistel permutation of [0, 2^k) (k even), cycle-walked
 // onto [0, n).
+__host__ __device__ __forceinline__ uint32_t feistel_half(uint32_t n) {
+    return (ceil_log2(n < 2 ? 2 : n) + 1) / 2;
+}
+__host__ __device__ __forceinline__ uint32_t feistel_round(uint64_t key, uint32_t R, uint32_t r, uint32_t mask) {
+    return uint32_t(mix64(key ^ (uint64_t(R) << 8) ^ r)) & mask;
+}
 __host__ __device__ inline uint32_t feistel_perm(uint32_t i, uint32_t n, uint64_t key) {
-    uint32_t k = ceil_log2(n < 2 ? 2 : n);
-    if (k & 1) ++k;
-    const uint32_t half = k / 2, mask = (1u << half) - 1u;
+    const uint32_t half = feistel_half(n), mask = (1u << half) - 1u;
     uint32_t v = i;
     do {
         uint32_t L = v >> half, R = v & mask;
         for (uint32_t r = 0; r < 4; ++r) {
-            uint32_t f = uint32_t(mix64(key ^ (uint64_t(R) << 8) ^ r)) & mask;
-            uint32_t nl = R;
-            R = L ^ f;
+            const uint32_t nl = R;
+            R = L ^ feistel_round(key, R, r, mask);
             L = nl;
         }
         v = (L << half) | R;

@@ -137,55 +137,158 @@ __global__ __launch_bounds__(kRoundThreads) void k_refine_round(uint64_t *__rest
     flush_stats<kRoundThreads>(st, att, acc, gain);
 }
 
+// --------------------------------------------------- rounds in LDS
+// The slots as the rounds hold them: P[i], a point unpacked to its two
+// coordinates (24 bits, the word's other two bytes on top), and S[i], the sums
+// of its two neighbours.  A swap exchanges points.
+__device__ __forceinline__ uint2 slot_point(uint64_t w) {
+    const uint32_t lo = uint32_t(w), hi = uint32_t(w >> 32);
+    return uint2{((lo & 0xFFFFu) << 8) | (hi & 0xFFu) | (hi >> 16 << 24),
+                 (lo >> 16 << 8) | ((hi >> 8) & 0xFFu) | (hi & 0xFF000000u)};
+}
+__device__ __forceinline__ uint64_t slot_word(const uint2 &p) {
+    const uint32_t lo = ((p.x >> 8) & 0xFFFFu) | ((p.y >> 8) << 16);
+    const uint32_t hi = (p.x & 0xFFu) | ((p.y & 0xFFu) << 8) | ((p.x >> 24) << 16) | (p.y & 0xFF000000u);
+    return uint64_t(lo) | (uint64_t(hi) << 32);
+}
+__device__ __forceinline__ int2 slot_sums(uint64_t prev, uint64_t next) {
+    return int2{pt_fx(prev) + pt_fx(next), pt_fy(prev) + pt_fy(next)};
+}
+
+template <class T>
+__device__ __forceinline__ T &at_byte(T *base, uint32_t byte) {
+    return *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte);
+}
+
+// `rounds` rounds over the n slots in P, S (n >= 2, in LDS, visible to every
+// thread on entry and exit).  att and acc, uniform in a wave, count the wave's
+// pairs and swaps; gain is this thread's.
+//
+// What bounds it: for a few slots the latency of a round (read, test, write,
+// barrier), for thousands LDS and instructions, about equally.  So the
+// workgroup is as wide as its pairs need and one wave goes without barriers;
+// the rounds' random c come from LDS, hashed side by side ahead of them
+// (hashing c in each round was a chain of 64-bit products before every
+// round's first read); points and sums are two arrays of 8 bytes, which
+// consecutive slots read and write without bank conflicts; and slots are
+// byte offsets that wrap by one unsigned min.  A thread's pairs of a round
+// are disjoint, so all their reads are issued before any swap.
+//
+// Measured on one MI355X, before with c hashed in each round, points unpacked
+// for each test and a group's slots found by hashing, twice: 16 passes of 32 rounds over a 1024x1024 frame's
+// chains in groups of up to 8192 slots 717 -> 567 us (44.8 -> 35.3 us a
+// pass); visits of 2^16 attempts at chains of 100 to 8000 slots 113 -> 24 to
+// 131 us, 8 to 19 of them 4,035 -> 2,068 us.
+template <int CAP, int NT>
+__device__ __forceinline__ void run_rounds(uint2 *P, int2 *S, uint32_t *cs, int n, uint64_t rounds, uint64_t seed,
+                                           uint64_t sid, uint64_t &att, uint64_t &acc, int64_t &gain) {
+    constexpr int kPer = (CAP / 2 + NT - 1) / NT;
+    constexpr uint32_t kCoord = 0xFFFFFFu;
+    const uint32_t tid = threadIdx.x, un = uint32_t(n), n8 = 8 * un;
+    int64_t down = 0;
+    for (uint64_t r0 = 0; r0 < rounds; r0 += NT) {
+        const uint32_t batch = uint32_t(rounds - r0 < NT ? rounds - r0 : NT);
+        if (tid < batch) {
+            const RoundPar rp = round_params(seed, sid, r0 + tid, un);
+            cs[tid] = 2 * rp.base + rp.odd;
+        }
+        __syncthreads();
+        uint32_t c = __builtin_amdgcn_readfirstlane(cs[0]), pairs = 0, swaps = 0;
+        for (uint32_t r = 0; r < batch; ++r) {
+            const uint32_t next = cs[r + 1 < batch ? r + 1 : r];
+            const uint32_t base = c >> 1, odd = c & 1u, npairs = odd ? un / 2 : (un - 1) / 2;
+            // pair t of the round is round_pair's, in bytes
+            const uint32_t i0 = 8 * (base + 1 + tid), j0 = 8 * (base + odd - 1 - tid);
+            uint32_t i[kPer], j[kPer];
+            uint2 pi[kPer], pj[kPer];
+            int2 si[kPer], sj[kPer];
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) {
+                if (tid + k * NT < npairs) {
+                    i[k] = min(i0 + 8 * k * NT, i0 + (8 * k * NT - n8));
+                    j[k] = min(j0 - 8 * k * NT, j0 + (n8 - 8 * k * NT));
+                    pi[k] = at_byte(P, i[k]);
+                    si[k] = at_byte(S, i[k]);
+                    pj[k] = at_byte(P, j[k]);
+                    sj[k] = at_byte(S, j[k]);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) {
+                bool swap = false;
+                if (tid + k * NT < npairs) {
+                    const int64_t d =
+                        int64_t(int32_t(pi[k].x & kCoord) - int32_t(pj[k].x & kCoord)) * int64_t(si[k].x - sj[k].x) +
+                        int64_t(int32_t(pi[k].y & kCoord) - int32_t(pj[k].y & kCoord)) * int64_t(si[k].y - sj[k].y);
+                    swap = d <= 0;
+                    if (swap) {
+                        at_byte(P, i[k]) = pj[k];
+                        at_byte(P, j[k]) = pi[k];
+                        down += d;
+                    }
+                }
+                swaps += uint32_t(__popcll(__ballot(swap)));
+            }
+            pairs += npairs;
+            c = __builtin_amdgcn_readfirstlane(next);
+            // (one wave: its LDS accesses are in order anyway)
+            if (NT > 64) __syncthreads();
+            else __builtin_amdgcn_wave_barrier();
+        }
+        att += pairs;
+        acc += swaps;
+        __syncthreads();
+    }
+    gain -= 2 * down;
+}
+
 // ---------------------------- plain: a whole visit of one chain, one launch
 // All `rounds` rounds of one visit in one workgroup, for chains of up to
 // kVisitCap slots: row y and the slots' neighbour sums are staged in LDS,
 // the rounds run there (they are sequential: each reads the swaps of the
-// one before, hence a barrier between rounds), and the row is written back
-// once.  The same pairs in the same order as one k_refine_round launch per
-// round.
-constexpr int kVisitThreads = 1024;
+// one before), and the row is written back once.  The same pairs in the same
+// order as one k_refine_round launch per round.
 constexpr int kVisitCap = 8192;
 
-__global__ __launch_bounds__(kVisitThreads) void k_refine_visit(uint64_t *__restrict__ pts, int h, int64_t wtot,
-                                                                int64_t off, int32_t w, int32_t y, uint64_t seed,
-                                                                uint64_t stream_id, uint64_t rounds,
-                                                                amh_refine_stats *st) {
-    __shared__ uint64_t C[kVisitCap];
-    __shared__ int2 S[kVisitCap];  // neighbour sums (x, y) of each slot
+template <int CAP, int NT>
+__global__ __launch_bounds__(NT) void k_refine_visit(uint64_t *__restrict__ pts, int h, int64_t wtot, int64_t off,
+                                                     int32_t w, int32_t y, uint64_t seed, uint64_t stream_id,
+                                                     uint64_t rounds, amh_refine_stats *st) {
+    __shared__ uint2 P[CAP];
+    __shared__ int2 S[CAP];
+    __shared__ uint32_t cs[NT];
     const int yp = y > 0 ? y - 1 : h - 1, yn = (y + 1) % h;
     uint64_t *row = pts + int64_t(y) * wtot + off;
     const uint64_t *rprev = pts + int64_t(yp) * wtot + off;
     const uint64_t *rnext = pts + int64_t(yn) * wtot + off;
-    for (int l = threadIdx.x; l < w; l += kVisitThreads) {
-        const uint64_t p = rprev[l], q = rnext[l];
-        C[l] = row[l];
-        S[l] = make_int2(pt_fx(p) + pt_fx(q), pt_fy(p) + pt_fy(q));
+    for (int l = threadIdx.x; l < w; l += NT) {
+        P[l] = slot_point(row[l]);
+        S[l] = slot_sums(rprev[l], rnext[l]);
     }
     __syncthreads();
     uint64_t att = 0, acc = 0;
     int64_t gain = 0;
-    for (uint64_t r = 0; r < rounds; ++r) {
-        const RoundPar rp = round_params(seed, stream_id, r, uint32_t(w));
-        for (uint32_t t = threadIdx.x; t < rp.npairs; t += kVisitThreads) {
-            uint32_t i, j;
-            round_pair(rp, uint32_t(w), t, i, j);
-            const uint64_t ci = C[i], cj = C[j];
-            const int2 si = S[i], sj = S[j];
-            const int64_t d = swap_test(ci, cj, si.x, si.y, sj.x, sj.y);
-            ++att;
-            if (d <= 0) {
-                C[i] = cj;
-                C[j] = ci;
-                ++acc;
-                gain += -2 * d;
-            }
-        }
-        __syncthreads();
-    }
-    for (int l = threadIdx.x; l < w; l += kVisitThreads) row[l] = C[l];
-    flush_stats<kVisitThreads>(st, att, acc, gain);
+    run_rounds<CAP, NT>(P, S, cs, w, rounds, seed, stream_id, att, acc, gain);
+    for (int l = threadIdx.x; l < w; l += NT) row[l] = slot_word(P[l]);
+    flush_stats<NT>(st, threadIdx.x == 0 ? att : 0, threadIdx.x % 64 == 0 ? acc : 0, gain);
 }
+
+// One pair per thread while the workgroup has room, so a round is as short
+// as it can be (a visit of 2^16 attempts at 100 slots has 1,311 rounds): two
+// pairs per thread in half the threads took 194 us instead of 131 up to 256
+// slots, 108 instead of 75 up to 512 and 40 instead of 31 up to 2048.
+using VisitFn = void (*)(uint64_t *, int, int64_t, int64_t, int32_t, int32_t, uint64_t, uint64_t, uint64_t,
+                         amh_refine_stats *);
+struct VisitVariant {
+    int cap, threads;
+    VisitFn fn;
+};
+const VisitVariant kVisits[] = {
+    {128, 64, k_refine_visit<128, 64>},       {256, 128, k_refine_visit<256, 128>},
+    {512, 256, k_refine_visit<512, 256>},     {1024, 512, k_refine_visit<1024, 512>},
+    {2048, 1024, k_refine_visit<2048, 1024>}, {4096, 1024, k_refine_visit<4096, 1024>},
+    {kVisitCap, 1024, k_refine_visit<kVisitCap, 1024>},
+};
 
 // ------------------------------------- batched: persistent, LDS resident
 // queue[0] = next item, queue[1] = workgroups finished, queue[2] = pass
@@ -194,14 +297,52 @@ __global__ __launch_bounds__(kVisitThreads) void k_refine_visit(uint64_t *__rest
 // node; with pass == kPassFromQueue every replay runs the next pass.
 constexpr uint64_t kPassFromQueue = ~0ull;
 
+// The row's slots of one group, at[k] that of local slot tid + k * NT < n: the
+// pass's Feistel permutation at g0, g0 + 1, ...  Its round functions take half
+// the bits of a slot number, so their four tables are laid out in `tab` first:
+// a wave's walk onto [0, w) is as long as its longest lane's, about a dozen
+// tries of four 64-bit mixes where w is little over a power of four.  They
+// must fit there (group_tables), in 2 * CAP words, which also keeps them less
+// work than the group's own CAP slots.
+template <int CAP>
+__device__ __forceinline__ bool group_tables(uint32_t w) {
+    return (4u << feistel_half(w)) <= 2u * CAP;
+}
+template <int CAP, int NT>
+__device__ __forceinline__ void group_slots(uint32_t *tab, int g0, int n, uint32_t w, uint64_t key,
+                                            uint32_t (&at)[CAP / NT]) {
+    const int tid = threadIdx.x;
+    const uint32_t half = feistel_half(w), mask = (1u << half) - 1u;
+    for (uint32_t e = tid; e < 4u << half; e += NT) tab[e] = feistel_round(key, e & mask, e >> half, mask);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < CAP / NT; ++k) {
+        const int l = tid + k * NT;
+        uint32_t v = uint32_t(g0 + l);
+        if (l < n) {
+            do {
+                uint32_t x = v >> half, y = v & mask;
+                x ^= tab[y];
+                y ^= tab[(1u << half) + x];
+                x ^= tab[(2u << half) + y];
+                y ^= tab[(3u << half) + x];
+                v = (x << half) | y;
+            } while (v >= w);
+        }
+        at[k] = v;
+    }
+    __syncthreads();
+}
+
 template <int CAP, int NT>
 __global__ __launch_bounds__(NT) void k_refine_pass(uint64_t *__restrict__ pts, int h, int64_t wtot,
                                                     const int64_t *__restrict__ off, const int32_t *__restrict__ cw,
                                                     const int32_t *__restrict__ items, int nitems, uint64_t pass,
                                                     int rounds, uint64_t seed, uint32_t *queue,
                                                     amh_refine_stats *st) {
-    __shared__ uint64_t C[CAP];
-    __shared__ int2 S[CAP];  // neighbour sums (x, y), one 8-byte LDS load per slot
+    __shared__ uint2 P[CAP];
+    __shared__ int2 S[CAP];
+    __shared__ uint32_t cs[NT];
     __shared__ int item_s;
     __shared__ uint32_t pass_s;
     const int tid = threadIdx.x;
@@ -233,61 +374,46 @@ __global__ __launch_bounds__(NT) void k_refine_pass(uint64_t *__restrict__ pts, 
         const int gs = (w + ng - 1) / ng;
         const int g0 = g * gs;
         const int n = min(gs, w - g0);
-        const bool permuted = ng > 1;
-        const uint64_t pkey = pass_stream(uint64_t(c), pass, 0xFFFFFFFFull);
         const uint64_t *rprev = pts + int64_t(yp) * wtot + o;
         const uint64_t *rnext = pts + int64_t(yn) * wtot + o;
         uint64_t *row = pts + int64_t(y) * wtot + o;
-        for (int l = tid; l < n; l += NT) {
-            const uint32_t s = permuted ? feistel_perm(uint32_t(g0 + l), uint32_t(w), pkey) : uint32_t(l);
-            const uint64_t p = rprev[s], q = rnext[s];
-            C[l] = row[s];
-            S[l] = make_int2(pt_fx(p) + pt_fx(q), pt_fy(p) + pt_fy(q));
+        const uint64_t pkey = pass_stream(uint64_t(c), pass, 0xFFFFFFFFull);
+        auto load = [&](int l, uint32_t s) {
+            P[l] = slot_point(row[s]);
+            S[l] = slot_sums(rprev[s], rnext[s]);
+        };
+        const bool walk = ng > 1 && !group_tables<CAP>(uint32_t(w));
+        uint32_t at[CAP / NT];  // this thread's slots in the row, unless it walks
+        if (walk) {
+#pragma unroll 1
+            for (int l = tid; l < n; l += NT) load(l, feistel_perm(uint32_t(g0 + l), uint32_t(w), pkey));
+        } else {
+            if (ng > 1) {
+                group_slots<CAP, NT>(reinterpret_cast<uint32_t *>(S), g0, n, uint32_t(w), pkey, at);
+            } else {
+#pragma unroll
+                for (int k = 0; k < CAP / NT; ++k) at[k] = uint32_t(tid + k * NT);
+            }
+#pragma unroll
+            for (int k = 0; k < CAP / NT; ++k)
+                if (tid + k * NT < n) load(tid + k * NT, at[k]);
         }
         __syncthreads();
-        if (n >= 2) {
-            const uint64_t sid = pass_stream(uint64_t(c), pass, uint64_t(g));
-            for (int r = 0; r < rounds; ++r) {
-                const RoundPar rp = round_params(seed, sid, uint64_t(r), uint32_t(n));
-                // A thread's pairs of the round (at most kPer): the pairs are
-                // disjoint, so all their loads are issued before any swap.
-                constexpr int kPer = (CAP / 2 + NT - 1) / NT;
-                uint32_t pi[kPer], pj[kPer];
-                uint64_t ci[kPer], cj[kPer];
-                int2 si[kPer], sj[kPer];
+        if (n >= 2)
+            run_rounds<CAP, NT>(P, S, cs, n, uint64_t(rounds), seed, pass_stream(uint64_t(c), pass, uint64_t(g)), att,
+                                acc, gain);
+        if (walk) {
+#pragma unroll 1
+            for (int l = tid; l < n; l += NT)
+                row[feistel_perm(uint32_t(g0 + l), uint32_t(w), pkey)] = slot_word(P[l]);
+        } else {
 #pragma unroll
-                for (int k = 0; k < kPer; ++k) {
-                    const uint32_t t = uint32_t(tid + k * NT);
-                    if (t < rp.npairs) {
-                        round_pair(rp, uint32_t(n), t, pi[k], pj[k]);
-                        ci[k] = C[pi[k]];
-                        cj[k] = C[pj[k]];
-                        si[k] = S[pi[k]];
-                        sj[k] = S[pj[k]];
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < kPer; ++k) {
-                    if (uint32_t(tid + k * NT) >= rp.npairs) continue;
-                    const int64_t d = swap_test(ci[k], cj[k], si[k].x, si[k].y, sj[k].x, sj[k].y);
-                    ++att;
-                    if (d <= 0) {
-                        C[pi[k]] = cj[k];
-                        C[pj[k]] = ci[k];
-                        ++acc;
-                        gain += -2 * d;
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        for (int l = tid; l < n; l += NT) {
-            const uint32_t s = permuted ? feistel_perm(uint32_t(g0 + l), uint32_t(w), pkey) : uint32_t(l);
-            row[s] = C[l];
+            for (int k = 0; k < CAP / NT; ++k)
+                if (tid + k * NT < n) row[at[k]] = slot_word(P[tid + k * NT]);
         }
         __syncthreads();
     }
-    flush_stats<NT>(st, att, acc, gain);
+    flush_stats<NT>(st, tid == 0 ? att : 0, tid % 64 == 0 ? acc : 0, gain);
     if (tid == 0) {
         __threadfence();
         const uint32_t done = atomicAdd(&queue[1], 1u);
@@ -574,9 +700,11 @@ extern "C" int amh_refine_chain(uint64_t *pts_dev, int32_t nkeys, int64_t wtot, 
     if (nkeys < 2 || chain_w < 2) return AMH_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (rounds > 1 && chain_w <= kVisitCap) {
-        // the whole visit in one launch
-        amh::launch_timed("k_refine_visit", k_refine_visit, dim3(1), dim3(kVisitThreads), 0, s, pts_dev, int(nkeys),
-                          wtot, chain_off, chain_w, y, seed, stream_id, rounds, stats_dev);
+        // the whole visit in one launch, of the narrowest variant that holds it
+        const VisitVariant *v = kVisits;
+        while (v->cap < chain_w) ++v;
+        amh::launch_timed("k_refine_visit", v->fn, dim3(1), dim3(v->threads), 0, s, pts_dev, int(nkeys), wtot, chain_off,
+                          chain_w, y, seed, stream_id, rounds, stats_dev);
         AMH_LAUNCH_CHECK("amh_refine_chain");
         return AMH_OK;
     }

@@ -128,6 +128,48 @@ def test_refine_batched_bitexact_all_tiles():
             assert G.to_host(queue, np.int32).tolist() == [0, 0, 3, 0]
 
 
+@pytest.mark.parametrize("rounds", [1, 130, 1027])
+def test_refine_visit_bitexact_at_width_edges(rounds):
+    """Whole visits at the widths where the workgroup's size changes, with
+    rounds over several of its batches."""
+    T = G.torch()
+    lib = G.lib()
+    rng = np.random.default_rng(rounds)
+    for w in (2, 3, 127, 128, 129, 256, 257, 511, 513, 1024, 1025, 2048, 2049, 4095, 4097, 8192, 8193):
+        pts, off, wid = _chains(rng, [w], 3, lim=65000)
+        dev = G.to_dev(G.key_major(pts, 3))
+        stats = G.zeros(4, T.int64)
+        G.log(f"refine_chain w={w} rounds={rounds}")
+        G.check(lib.amh_refine_chain(G.dptr(dev), 3, w, 0, w, 2, rounds, 99, w, G.dptr(stats), G.stream()),
+                "amh_refine_chain")
+        want, acc, gain, att = op.refine_rounds(pts, 3, 2, rounds, 99, w)
+        assert (G.atom_major(G.to_host(dev, np.uint64), 3) == want).all(), w
+        st = G.to_host(stats, np.int64)
+        assert (st[0], st[1], st[2]) == (att, acc, gain), w
+
+
+@pytest.mark.parametrize("width", [1025, 4097, 262144, 262145])
+def test_refine_groups_of_wide_rows_bitexact(width):
+    """Rows split over groups by the pass's permutation, at widths just past a
+    power of four and on both sides of the smallest tile's table limit."""
+    T = G.torch()
+    lib = G.lib()
+    rng = np.random.default_rng(width)
+    tile, cap, thr = _tiles()[0]
+    pts, off, wid = _chains(rng, [width], 2, lim=4000)
+    items, nitems = _items(wid, tile)
+    dev = G.to_dev(G.key_major(pts, 2))
+    off_d, w_d, it_d = G.to_dev(off), G.to_dev(wid.astype(np.int32)), G.to_dev(items)
+    queue, stats = G.zeros(4, T.int32), G.zeros(4, T.int64)
+    want = pts
+    for p in range(2):
+        G.log(f"refine_batched w={width} cap={cap} threads={thr} pass={p} items={nitems}")
+        G.check(lib.amh_refine_batched(G.dptr(dev), 2, width, G.dptr(off_d), G.dptr(w_d), G.dptr(it_d), nitems, tile,
+                                       p, 3, 31, G.dptr(queue), G.dptr(stats), G.stream()), "amh_refine_batched")
+        want, acc, gain, att = op.refine_pass(want, off, wid, 2, cap, p, 3, 31)
+    assert (G.atom_major(G.to_host(dev, np.uint64), 2) == want).all()
+
+
 def test_refine_knn_bitexact():
     """kNN-guided passes, every variant: the same points, counters and queue
     state as the oracle's replay, chains split over groups included."""
