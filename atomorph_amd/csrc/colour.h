@@ -90,4 +90,65 @@ __host__ __device__ inline uint32_t hsp_to_rgb(uint32_t c) {
                      narrow8(fmin(round(b * 255.0), 255.0)), c >> 24);
 }
 
+// The same two in float, for a colour whose channels all land further than
+// kClear from where the 8-bit rounding turns; false where one does not (about
+// 1 colour in 30, mostly exact ties), and the double-precision form above decides.  Float is off
+// by at most half of kClear: whole numbers up to 255 in, no differences of
+// rounded terms, and at most ten roundings of 2^-24 of values up to 255.  The
+// colours are few enough that all of them are compared.
+//
+// Measured on one MI355X, 2048x2048 pixels, 36% opaque, both ways: 52 -> 26 us.
+// In double precision the dozen divisions and two roots of a pixel bound it.
+constexpr float kClear = 1.f / 4096;
+__device__ __forceinline__ bool round_clear(float v, uint32_t *out) {
+    const float r = rintf(v);
+    *out = uint32_t(r);
+    return fabsf(v - r) < 0.5f - kClear;
+}
+__device__ __forceinline__ bool rgb_to_hsp_clear(uint32_t c, uint32_t *hsp) {
+    const float R = float(c & 255u), G = float((c >> 8) & 255u), B = float((c >> 16) & 255u);
+    uint32_t h = 0, s = 0, p = 0;
+    bool clear = round_clear(__builtin_amdgcn_sqrtf(R * R * 0.299f + G * G * 0.587f + B * B * 0.114f), &p);
+    if (R != G || R != B) {
+        const bool r = R >= G && R >= B, g = G >= R && G >= B;
+        const float top = r ? R : g ? G : B, after = r ? G : g ? B : R, before = r ? B : g ? R : G;
+        const bool down = before >= after;
+        const float origin = r ? (down ? 255.f : 0.f) : g ? 85.f : 170.f;
+        const float low = down ? after : before, part = 42.5f * (after - before);
+        clear &= round_clear(origin + part * __builtin_amdgcn_rcpf(top - low), &h);
+        clear &= round_clear(255.f * (top - low) * __builtin_amdgcn_rcpf(top), &s);
+    }
+    *hsp = rgba_pack(h, s, p, c >> 24);
+    return clear;
+}
+__device__ __forceinline__ bool hsp_to_rgb_clear(uint32_t c, uint32_t *rgb) {
+    const uint32_t h6 = 6 * (c & 255u), sext = min(h6 / 255u, 5u);
+    const float f = float((sext & 1) ? 255 * (sext + 1) - h6 : h6 - 255 * sext) * (1.f / 255);
+    const float S = float((c >> 8) & 255u), P = float((c >> 16) & 255u);
+    const float wbig = (sext == 0 || sext == 5) ? 0.299f : sext < 3 ? 0.587f : 0.114f;
+    const float wmid = (sext == 0 || sext == 3) ? 0.587f : (sext == 1 || sext == 4) ? 0.299f : 0.114f;
+    const float wlow = 1.f - wbig - wmid;  // (exact to a rounding)
+    float lo = 0.f, mid, hi;
+    if (S < 255.f) {
+        const float grow = 255.f * __builtin_amdgcn_rcpf(255.f - S);  // largest / smallest
+        const float part = 1.f + f * S * __builtin_amdgcn_rcpf(255.f - S);
+        lo = P * __builtin_amdgcn_rsqf(wbig * grow * grow + wmid * part * part + wlow);
+        hi = lo * grow;
+        mid = lo * part;
+    } else {
+        hi = P * __builtin_amdgcn_rsqf(wbig + wmid * f * f);
+        mid = hi * f;
+    }
+    uint32_t a, b, d;
+    bool clear = round_clear(fminf(hi, 255.f), &a);
+    clear &= round_clear(fminf(mid, 255.f), &b);
+    clear &= round_clear(fminf(lo, 255.f), &d);
+    const bool r_big = sext == 0 || sext == 5, r_mid = sext == 1 || sext == 4;
+    const bool g_big = sext == 1 || sext == 2, g_mid = sext == 0 || sext == 3;
+    const bool b_big = sext == 3 || sext == 4;
+    *rgb = rgba_pack(r_big ? a : r_mid ? b : d, g_big ? a : g_mid ? b : d, b_big ? a : (sext == 2 || sext == 5) ? b : d,
+                     c >> 24);
+    return clear;
+}
+
 }  // namespace amh
