@@ -128,81 +128,90 @@ __device__ Box block_box(bool valid, int cx, int cy, int *red) {
 }
 
 // Runs of consecutive lanes whose particles share a stencil origin form
-// segments (the cell order makes such runs common).  seg_sum leaves each
-// segment's total in its last lane, so one lane per segment scatters.
+// segments (the cell order makes such runs common), cut at the rows of 16
+// lanes that DPP shifts within.  seg_sums leaves each segment's totals in its
+// last lane, so one lane per segment scatters.
 struct Seg {
-    int lane, start;  // start: first lane of this lane's segment
-    bool tail;        // last lane of its segment
+    int run;    // lanes of this lane's segment before it (0..15)
+    bool tail;  // last lane of its segment
+    bool more;  // the segment may continue one in the lanes before its row
 };
 
-// The neighbours' origins come by DPP wave shifts and the segment starts
+// The neighbours' origins come by DPP row shifts and the segment starts
 // from a ballot of the heads, so no LDS round trip is on this path.
 __device__ __forceinline__ Seg segments(bool valid, int cx, int cy) {
     Seg s;
-    s.lane = threadIdx.x & 63;
-    // origin key; an invalid lane matches no origin (nodes are < 65535)
+    const int lane = threadIdx.x & 63;
+    // origin key; an invalid lane matches no origin (nodes are < 65535), nor
+    // does a row's end
     const int key = valid ? int((uint32_t(cx) << 16) | (uint32_t(cy) & 0xFFFFu)) : -1;
-    const int prev = __builtin_amdgcn_update_dpp(-1, key, 0x138, 0xF, 0xF, false);  // wave_shr:1, lane - 1
-    const int next = __builtin_amdgcn_update_dpp(-1, key, 0x130, 0xF, 0xF, false);  // wave_shl:1, lane + 1
-    const bool head = !valid || s.lane == 0 || prev != key;
-    s.tail = !valid || s.lane == 63 || next != key;
-    const uint64_t heads = __ballot(head) & ((2ull << s.lane) - 1ull);  // heads at or below this lane
-    s.start = 63 - __clzll(static_cast<long long>(heads));               // lane 0 is always a head
+    const int prev = __builtin_amdgcn_update_dpp(-1, key, 0x111, 0xF, 0xF, false);  // row_shr:1, lane - 1
+    const int next = __builtin_amdgcn_update_dpp(-1, key, 0x101, 0xF, 0xF, false);  // row_shl:1, lane + 1
+    const bool head = !valid || prev != key;
+    s.tail = !valid || next != key;
+    const uint64_t heads = __ballot(head) & ((2ull << lane) - 1ull);     // heads at or below this lane
+    s.run = lane - (63 - __clzll(static_cast<long long>(heads)));         // lane 0 is always a head
+    // (wave_shr:1; what lies before the wave is not known here)
+    const int before = __builtin_amdgcn_update_dpp(key, key, 0x138, 0xF, 0xF, false);
+    const uint64_t cut = __ballot(valid && (lane & 15) == 0 && before == key);
+    s.more = valid && s.run == (lane & 15) && ((cut >> (lane & 48)) & 1u);
     return s;
 }
 
-// DPP move of v: row_shr:k (0x110 + k), row_bcast:15 (0x142) or
-// row_bcast:31 (0x143); lanes without a source (or outside row_mask) get 0.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false));
+// DPP row_shr:K of v; lanes without a source get 0.
+template <int K>
+__device__ __forceinline__ float row_shr(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x110 + K, 0xF, 0xF, false));
+}
+template <int K, int N>
+__device__ __forceinline__ void seg_step(float (&c)[N], const Seg &s) {
+    const bool in = s.run >= K;
+    if (__ballot(in) == 0) return;
+    for (int k = 0; k < N; ++k) {
+        const float t = c[k] + row_shr<K>(c[k]);
+        c[k] = in ? t : c[k];
+    }
 }
 
-// Inclusive segmented sum over lanes [start, lane]; every lane of the wave
-// must take part.
-__device__ __forceinline__ float seg_sum(float v, const Seg &s) {
-    float t;
-    t = dpp<0x111, 0xF>(v);
-    if (s.lane - 1 >= s.start) v += t;
-    t = dpp<0x112, 0xF>(v);
-    if (s.lane - 2 >= s.start) v += t;
-    t = dpp<0x114, 0xF>(v);
-    if (s.lane - 4 >= s.start) v += t;
-    t = dpp<0x118, 0xF>(v);
-    if (s.lane - 8 >= s.start) v += t;
-    t = dpp<0x142, 0xA>(v);  // lane 15 -> row 1, lane 47 -> row 3
-    if ((s.lane & 16) && s.start <= (s.lane & ~15) - 1) v += t;
-    t = dpp<0x143, 0xC>(v);  // lane 31 -> rows 2 and 3
-    if (s.lane >= 32 && s.start <= 31) v += t;
-    return v;
+// Inclusive segmented sums of N values; every lane of the wave must take part
+// (zeros from lanes that do not contribute).  A step is two instructions per
+// value and is taken only when the wave has a segment that long; crossing
+// the rows would take two more steps of five.
+template <int N>
+__device__ __forceinline__ void seg_sums(float (&c)[N], const Seg &s) {
+    seg_step<1>(c, s);
+    seg_step<2>(c, s);
+    seg_step<4>(c, s);
+    seg_step<8>(c, s);
 }
 
 // ------------------------------------------------------------ P2G
 // Mass (= density), density gradient and strength-weighted colour
-// (fluidmodel.cpp:191-249).  With e = x - cx - 1 in [-0.5, 0.5) the
-// quadratic B-spline weights and their gradients are polynomials in e:
-//   px[a] = sum_p kW[a][p] e^p,   gx[a] = sum_p kD[a][p] e^p,
-// so the node sums of px[a] py[b], gx[a] py[b] and px[a] gy[b] over the
-// particles of one cell follow from the cell's nine moments
-// M[p][q] = sum e^p h^q (h likewise in y).  A particle therefore adds 9
-// moments and 5 colour sums to its one cell instead of 8 values to each of 9
-// nodes; the nodes are assembled from the 3x3 cells around them.
-__constant__ float kW[3][3] = {{0.125f, -0.5f, 0.5f}, {0.75f, 0.0f, -1.0f}, {0.125f, 0.5f, 0.5f}};
-__constant__ float kD[3][3] = {{0.5f, -1.0f, 0.0f}, {0.0f, 2.0f, 0.0f}, {-0.5f, -1.0f, 0.0f}};
-constexpr int kCellSums = 14;  // 9 moments (p-major), then s*r, s*g, s*b, s*a, s
+// (fluidmodel.cpp:191-249).  A particle at e = x - cx - 1 in [-0.5, 0.5) of
+// its cell has the quadratic B-spline weights
+//   w[0] = (0.5 - e)^2 / 2,  w[1] = 0.75 - e^2,  w[2] = (0.5 + e)^2 / 2
+// (h likewise in y), whose gradients are combinations of them: with
+// 1 = w[0] + w[1] + w[2] and e = w[2] - w[0], gx[a] = sum_p kG[a][p] w[p].  So
+// the node sums of px[a] py[b], gx[a] py[b] and px[a] gy[b] over the
+// particles of one cell follow from the cell's nine sums of w[p](e) w[q](h).
+// A particle therefore adds 9 products and 5 colour sums to its one cell
+// instead of 8 values to each of 9 nodes; the nodes are assembled from the
+// 3x3 cells around them.  The products, and so the masses that the later
+// phases divide by, keep their precision however small they are (sums of the
+// powers of e and h lose it where a weight nearly vanishes).
+constexpr int kCellSums = 14;  // 9 products (p-major), then s*r, s*g, s*b, s*a, s
 
-// The 8 node values (m, gx, gy, r, g, b, a, w) that the sums c[] of cell
-// (node - (a, b)) contribute to the node.
-__device__ __forceinline__ void cell_to_node(const float *c, int a, int b, float *v) {
-    float xw[3], xd[3];  // sum_p kW[a][p] M[p][q], sum_p kD[a][p] M[p][q]
-    for (int q = 0; q < 3; ++q) {
-        xw[q] = kW[a][0] * c[q] + kW[a][1] * c[3 + q] + kW[a][2] * c[6 + q];
-        xd[q] = kD[a][0] * c[q] + kD[a][1] * c[3 + q] + kD[a][2] * c[6 + q];
-    }
-    v[0] = kW[b][0] * xw[0] + kW[b][1] * xw[1] + kW[b][2] * xw[2];
-    v[1] = kW[b][0] * xd[0] + kW[b][1] * xd[1] + kW[b][2] * xd[2];
-    v[2] = kD[b][0] * xw[0] + kD[b][1] * xw[1] + kD[b][2] * xw[2];
-    for (int k = 0; k < 5; ++k) v[3 + k] = c[9 + k];
+__device__ __forceinline__ void basis(double e, double (&w)[3]) {
+    w[0] = 0.5 * (0.5 - e) * (0.5 - e);
+    w[1] = 0.75 - e * e;
+    w[2] = 0.5 * (0.5 + e) * (0.5 + e);
+}
+// The gradient of weight a from the sums w[] of the three weights.
+__device__ __forceinline__ float basis_gradient(int a, float w0, float w1, float w2) {
+    const float k0 = a == 0 ? 1.5f : a == 1 ? -2.0f : 0.5f;
+    const float k1 = a == 0 ? 0.5f : a == 1 ? 0.0f : -0.5f;
+    const float k2 = a == 0 ? -0.5f : a == 1 ? 2.0f : -1.5f;
+    return k0 * w0 + k1 * w1 + k2 * w2;
 }
 
 __device__ __forceinline__ float nd(const float *f, int i, int j, int gsx, int gsy) {
@@ -610,7 +619,7 @@ __device__ __forceinline__ void run_item(int slot, bool home, const Fetch &fetch
                                          const Prologue &prologue) {
     const auto item = fetch(slot);
     prologue();
-    body(slot, home, item);
+    if (__ballot(slot >= 0)) body(slot, home, item);  // a sparse tile leaves whole waves empty
 }
 
 __device__ __forceinline__ void put_node(float *f, int64_t k, float v, bool single) {
@@ -659,34 +668,79 @@ struct Halo {
     }
 };
 
+// Sums of N values per cell in reach of a tile, over an item whose entries
+// are in cell order.  Each cell is one run of entries, so a segment's totals
+// are stored, not added, unless its run was cut at a row's start: those
+// totals are kept aside and added once the stores are done.  (LDS float
+// atomics take about one cycle per lane and bound these kernels when each
+// segment added its totals.)
+constexpr int kRows = kT / 16;  // rows of lanes
+
+template <int N>
+struct CellSums {
+    float v[N][kReach * kReach];
+    float cut[N][kRows];
+    int cell[kRows];  // the cell of a row's cut run, -1 none
+
+    __device__ __forceinline__ void clear() {
+        for (int k = threadIdx.x; k < N * kReach * kReach; k += kT) (&v[0][0])[k] = 0.0f;
+        if (threadIdx.x < kRows) cell[threadIdx.x] = -1;
+    }
+    // Every lane of the wave calls it (c: zeros unless valid, destroyed);
+    // origin (cx, cy) in reach of the tile at (x0, y0) where valid.
+    __device__ __forceinline__ void put(float (&c)[N], bool valid, int cx, int cy, int x0, int y0) {
+        const Seg S = segments(valid, cx, cy);
+        seg_sums(c, S);
+        if (!valid || !S.tail) return;
+        const int idx = (cx - x0 + 2) * kReach + (cy - y0 + 2), row = threadIdx.x / 16;
+        if (S.more) {
+            cell[row] = idx;
+            for (int k = 0; k < N; ++k) cut[k][row] = c[k];
+        } else {
+            for (int k = 0; k < N; ++k) v[k][idx] = c[k];
+        }
+    }
+    // After a barrier; the sums are whole after another.
+    __device__ __forceinline__ void join() {
+        const int row = threadIdx.x % kRows, at = cell[row];
+        if (at < 0) return;
+        for (int k = threadIdx.x / kRows; k < N; k += kT / kRows) atomicAdd(&v[k][at], cut[k][row]);
+    }
+};
+
 struct P2gItem {
     double x, y, s, r, g, b, a;
     int mature;
 };
 
 // Mass (= density), density gradient and strength-weighted colour of the
-// tile's nodes from the moments of the cells that reach them.
+// tile's nodes from the sums of the cells that reach them.
 //
 // The block first counting-sorts its chunk by cell (the kReach x
 // kReach cells in reach, then the entries out of reach) through LDS, sums
-// the moments in that order, and leaves the chunk of the bin list in that
-// order for k_forces and k_g2p.  Particles move about two cells per step,
-// so the frame's cell order is gone after one step; without the sort, runs
-// of lanes on one cell (summed with DPP before one LDS atomic per run)
-// shrink to about one lane and every lane pays its own atomics.
+// the cells in that order, and leaves the chunk of the bin list in that
+// order for k_forces and k_g2p, whose sums rest on it too.  Particles move
+// about two cells per step, so the frame's cell order is gone after one
+// step; without the sort a cell would be many runs.
 //
-// Six waves per SIMD (79 VGPRs): the LDS (18 KB) allows eight blocks per
-// CU; seven waves spill 12 bytes per lane, which measured slower, and
-// without a bound the node assembly's scheduling takes 95 VGPRs (five).
+// Instructions and LDS bound this kernel, k_forces and k_g2p.  One MI355X,
+// 229k particles on 276^2 nodes (1044^2), us: here 18.2 -> 13.6 (37 -> 22),
+// k_forces 12.5 -> 10.1 (26 -> 20), k_g2p 14.7 -> 11.2 (34 -> 21), before with
+// LDS atomics per run and node and sums carried across the lanes' rows.
+//
+// Six waves per SIMD (72 VGPRs): the LDS (19 KB) allows eight blocks per
+// CU; seven waves spilled when there were more registers, which measured
+// slower.
 __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_p2g(Particles P, Grid Gd, int gsx,
                                                                                    int gsy, Bins B) {
-    __shared__ float cs[kCellSums][kReach * kReach];
+    __shared__ CellSums<kCellSums> sums;
+    const auto &cs = sums.v;
     constexpr int kCells = kReach * kReach;  // local cells; bucket kCells: out of reach
     __shared__ int cellpos[kCells + 2];  // per bucket: count, then first place
     __shared__ int2 mine[kT];            // per thread: its list entry, (bucket << 8) | rank (-1: no entry)
     __shared__ int perm[kT];             // sorted place -> thread
     // The chunk's items (position and colour terms), one array per field so
-    // that consecutive lanes write consecutive words; dead once the moments
+    // that consecutive lanes write consecutive words; dead once the cells
     // are summed, so they share their space with the node assembly's partials.
     union Stage {
         struct {
@@ -697,6 +751,7 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     };
     __shared__ Stage stage;
     static_assert(kCells + 2 <= 2 * 64, "one wave scans the buckets, two per lane");
+    static_assert(kTile * kTile == 64, "one wave per column of cells in the node assembly");
     const int nchunks = *B.nchunks;
     // the step before's counts, read by every placing block, are cleared
     // here for the next step's counting
@@ -716,7 +771,7 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             return P2gItem{P.x[q], P.y[q], P.strength[q], P.r[q], P.g[q], P.b[q], P.a[q], P.mature[q]};
         };
         const auto clear = [&] {
-            for (int k = threadIdx.x; k < kCellSums * kReach * kReach; k += kT) (&cs[0][0])[k] = 0.0f;
+            sums.clear();
             if (threadIdx.x < kCells + 2) cellpos[threadIdx.x] = 0;
             // an empty item (a tile that has just emptied) never runs the body
             mine[threadIdx.x] = make_int2(0, -1);
@@ -732,25 +787,20 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             t[3] = tint ? float(it.s * it.a) : 0.0f;
             t[4] = tint ? float(it.s) : 0.0f;
         };
-        // The moments of one particle at (x, y) with colour terms t (valid:
-        // in reach of the tile) added to its cell's LDS sums; every lane of
-        // the block calls it.  Branch-free: selects instead of conditional
+        // The products of one particle at (x, y) and its colour terms t (valid:
+        // in reach of the tile) into its cell's LDS sums; every lane of
+        // the wave calls it.  Branch-free: selects instead of conditional
         // blocks, so no load is deferred into a branch.
-        const auto moments = [&](bool valid, double x, double y, const float (&t)[5]) {
+        const auto sum_cells = [&](bool valid, double x, double y, const float (&t)[5]) {
             const int cx = static_cast<int>(x - 0.5), cy = static_cast<int>(y - 0.5);
             float c[kCellSums];
-            const double e = x - cx - 1.0, h = y - cy - 1.0;
-            const double ep[3] = {1.0, e, e * e}, hp[3] = {1.0, h, h * h};
+            double ex[3], hy[3];
+            basis(x - cx - 1.0, ex);
+            basis(y - cy - 1.0, hy);
             for (int p = 0; p < 3; ++p)
-                for (int q = 0; q < 3; ++q) c[p * 3 + q] = valid ? float(ep[p] * hp[q]) : 0.0f;
+                for (int q = 0; q < 3; ++q) c[p * 3 + q] = valid ? float(ex[p] * hy[q]) : 0.0f;
             for (int k = 0; k < 5; ++k) c[9 + k] = valid ? t[k] : 0.0f;
-            const Seg S = segments(valid, cx, cy);
-            for (int k = 0; k < kCellSums; ++k) c[k] = seg_sum(c[k], S);
-            if (valid && S.tail) {
-                const int idx = (cx - x0 + 2) * kReach + (cy - y0 + 2);
-                for (int k = 0; k < kCellSums; ++k)
-                    if (c[k] != 0.0f) atomicAdd(&cs[k][idx], c[k]);
-            }
+            sums.put(c, valid, cx, cy, x0, y0);
         };
         {
             // at most kT entries: one pass, ranks fit in 8 bits
@@ -798,27 +848,31 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             const double x = in ? stage.item.x[src] : 0.0, y = in ? stage.item.y[src] : 0.0;
             float t[5];
             for (int k = 0; k < 5; ++k) t[k] = stage.item.t[k][src];
-            moments(in, x, y, t);
+            if (__ballot(in)) sum_cells(in, x, y, t);
         }
+        __syncthreads();
+        sums.join();
         __syncthreads();
         // Nodes from the cells: thread (a, node) sums the three cells
         // (node - (a, b)), then one thread per node adds the three partials.
         auto &part = stage.part;
         static_assert(3 * kTile * kTile <= kT, "one thread per (a, node)");
         {
-            const int t = threadIdx.x, node = t % (kTile * kTile), a = t / (kTile * kTile);
+            const int node = threadIdx.x % (kTile * kTile);
+            // (the same in all of a wave)
+            const int a = __builtin_amdgcn_readfirstlane(threadIdx.x / (kTile * kTile));
             if (a < 3) {
-                const int ni = x0 + node / kTile, nj = y0 + node % kTile;
+                const int ni = node / kTile, nj = node % kTile;
                 float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
                 for (int b = 0; b < 3; ++b) {
                     // an empty cell's sums are zero and add nothing; no branch on
                     // it, so the three cells' LDS loads are in flight together
-                    const int cell = (ni - a - x0 + 2) * kReach + (nj - b - y0 + 2);
-                    float m[kCellSums];
-                    for (int k = 0; k < kCellSums; ++k) m[k] = cs[k][cell];
-                    float v[8];
-                    cell_to_node(m, a, b, v);
-                    for (int f = 0; f < 8; ++f) acc[f] += v[f];
+                    const int cell = (ni - a + 2) * kReach + (nj - b + 2);
+                    const float r0 = cs[a * 3][cell], r1 = cs[a * 3 + 1][cell], r2 = cs[a * 3 + 2][cell];
+                    acc[0] += b == 0 ? r0 : b == 1 ? r1 : r2;
+                    acc[1] += basis_gradient(a, cs[b][cell], cs[3 + b][cell], cs[6 + b][cell]);
+                    acc[2] += basis_gradient(b, r0, r1, r2);
+                    for (int k = 0; k < 5; ++k) acc[3 + k] += cs[9 + k][cell];
                 }
                 for (int f = 0; f < 8; ++f) part[a][f][node] = acc[f];
             }
@@ -839,36 +893,30 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     }
 }
 
-// Sums v (zeros for lanes that do not contribute) over runs of lanes with
-// the same stencil origin and adds the run totals to node (cx + a, cy + b)
-// of the tile's LDS sums when that node belongs to the tile.
-__device__ __forceinline__ void tile_add2(float (&acc)[2][kTile * kTile], const Seg &S, bool valid, int cx, int cy,
-                                          int x0, int y0, int a, int b, float v0, float v1) {
-    v0 = seg_sum(v0, S);
-    v1 = seg_sum(v1, S);
-    const int li = cx + a - x0, lj = cy + b - y0;
-    if (valid && S.tail && li >= 0 && li < kTile && lj >= 0 && lj < kTile) {
-        if (v0 != 0.0f) atomicAdd(&acc[0][li * kTile + lj], v0);
-        if (v1 != 0.0f) atomicAdd(&acc[1][li * kTile + lj], v1);
-    }
-}
+// Per cell what its particles add to the two sums of node (cell + (a, b)):
+// [3 a + b] and [9 + 3 a + b].
+using StencilSums = CellSums<18>;
 
-// Stores (or adds) the tile's two LDS sums into fields f0, f1: node k's
-// values at f0[stride*k], f1[stride*k].
-__device__ __forceinline__ void store_tile2(const float (&acc)[2][kTile * kTile], float *f0, float *f1, int stride,
-                                            int x0, int y0, int gsx, int gsy, bool single) {
-    for (int t = threadIdx.x; t < kTile * kTile; t += kT) {
-        const int ni = x0 + t / kTile, nj = y0 + t % kTile;
-        if (ni >= gsx || nj >= gsy) continue;
-        const int64_t k = int64_t(ni) * gsy + nj;
-        put_node(f0, stride * k, acc[0][t], single);
-        put_node(f1, stride * k, acc[1][t], single);
-    }
+// Stores (or adds) the tile's node sums into fields f0, f1, each node's from
+// the cells that reach it: node k's values at f0[stride*k], f1[stride*k].
+__device__ __forceinline__ void store_tile2(StencilSums &sums, float *f0, float *f1, int stride, int x0, int y0,
+                                            int gsx, int gsy, bool single) {
+    sums.join();
+    __syncthreads();
+    const int t = threadIdx.x % (kTile * kTile), f = threadIdx.x / (kTile * kTile);
+    if (f >= 2) return;
+    const int ni = x0 + t / kTile, nj = y0 + t % kTile;
+    if (ni >= gsx || nj >= gsy) return;
+    float s = 0.0f;
+    for (int k = 0; k < 9; ++k)
+        s += sums.v[9 * f + k][(t / kTile + 2 - k / 3) * kReach + (t % kTile + 2 - k % 3)];
+    const int64_t k = int64_t(ni) * gsy + nj;
+    put_node(f == 0 ? f0 : f1, stride * k, s, single);
 }
 
 // Node accelerations: pressure and wall forces (fluidmodel.cpp:251-357).
 __global__ __launch_bounds__(kT) void k_forces(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
-    __shared__ float acc[2][kTile * kTile];
+    __shared__ StencilSums acc;
     __shared__ float nodes[3][kHalo * kHalo];  // m, gx, gy
     const int nchunks = *B.nchunks;
     for (int item = int(blockIdx.x);; item += int(gridDim.x)) {
@@ -877,7 +925,7 @@ __global__ __launch_bounds__(kT) void k_forces(Particles P, Grid Gd, int gsx, in
         if (!tile_item(B, nchunks, item, tile, single, slot0, home0)) break;
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
-        for (int k = threadIdx.x; k < 2 * kTile * kTile; k += kT) (&acc[0][0])[k] = 0.0f;
+        acc.clear();
         // the halo's loads are issued beside the particles', which are
         // unconditional (slot -1 reads particle 0)
         Halo<3> halo;
@@ -900,14 +948,22 @@ __global__ __launch_bounds__(kT) void k_forces(Particles P, Grid Gd, int gsx, in
             weights(x, y, cx, cy, px, py, gx, gy);
             const bool valid = slot >= 0 && in_reach(cx, cy, x0, y0);
             if (valid) particle_forces(x, y, node, gsx, gsy, pressure, fx, fy);  // LDS reads only
-            const Seg S = segments(valid, cx, cy);
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) {
+            float v[18];
+            if (__ballot(fx != 0.0 || fy != 0.0)) {  // near a wall
+                for (int k = 0; k < 9; ++k) {
+                    const int a = k / 3, b = k % 3;
                     const double phi = px[a] * py[b];
-                    const float v0 = valid ? float(-((gx[a] * py[b]) * pressure) + fx * phi) : 0.0f;
-                    const float v1 = valid ? float(-((px[a] * gy[b]) * pressure) + fy * phi) : 0.0f;
-                    tile_add2(acc, S, valid, cx, cy, x0, y0, a, b, v0, v1);
+                    v[k] = valid ? float(-((gx[a] * py[b]) * pressure) + fx * phi) : 0.0f;
+                    v[9 + k] = valid ? float(-((px[a] * gy[b]) * pressure) + fy * phi) : 0.0f;
                 }
+            } else {
+                for (int k = 0; k < 9; ++k) {
+                    const int a = k / 3, b = k % 3;
+                    v[k] = valid ? float(-((gx[a] * py[b]) * pressure)) : 0.0f;
+                    v[9 + k] = valid ? float(-((px[a] * gy[b]) * pressure)) : 0.0f;
+                }
+            }
+            acc.put(v, valid, cx, cy, x0, y0);
         }, stage);
         __syncthreads();
         store_tile2(acc, Gd.ax, Gd.ay, 1, x0, y0, gsx, gsy, single);
@@ -924,7 +980,7 @@ struct G2pItem {
 // the particle's home tile), then the momentum of the tile's nodes
 // (fluidmodel.cpp:359-437).
 __global__ __launch_bounds__(kT) void k_g2p(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
-    __shared__ float acc[2][kTile * kTile];
+    __shared__ StencilSums acc;
     __shared__ float accel[2][kHalo * kHalo];  // node accelerations per mass
     const int nchunks = *B.nchunks;
     for (int item = int(blockIdx.x);; item += int(gridDim.x)) {
@@ -933,7 +989,7 @@ __global__ __launch_bounds__(kT) void k_g2p(Particles P, Grid Gd, int gsx, int g
         if (!tile_item(B, nchunks, item, tile, single, slot0, home0)) break;
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
-        for (int k = threadIdx.x; k < 2 * kTile * kTile; k += kT) (&acc[0][0])[k] = 0.0f;
+        acc.clear();
         // as in k_forces: halo loads beside the unconditional particle loads
         Halo<3> halo;
         halo.load(x0, y0, gsx, gsy,
@@ -955,21 +1011,28 @@ __global__ __launch_bounds__(kT) void k_g2p(Particles P, Grid Gd, int gsx, int g
             double cax, cay;  // attractor, 0.03 per step (fluidmodel.cpp:383-410)
             toward(x, y, it.gx, it.gy, 0.03, cax, cay);
             double u = it.u, v = it.v;
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) {
-                    const double phi = px[a] * py[b];
-                    double ax = 0.0, ay = 0.0;
-                    if (valid) {  // in reach: the node is staged
-                        const int e = halo_index(cx + a, cy + b, x0, y0);
-                        ax = accel[0][e];
-                        ay = accel[1][e];
-                    } else if (home) {
-                        ax = nd_m(Gd.ax, Gd.muvw, cx + a, cy + b, gsx, gsy);
-                        ay = nd_m(Gd.ay, Gd.muvw, cx + a, cy + b, gsx, gsy);
+            float nax[9], nay[9];
+            const int e = valid ? halo_index(cx, cy, x0, y0) : 0;
+            for (int k = 0; k < 9; ++k) {
+                nax[k] = accel[0][e + k / 3 * kHalo + k % 3];
+                nay[k] = accel[1][e + k / 3 * kHalo + k % 3];
+            }
+            if (home && !valid) {  // a stencil that leaves the grid
+#pragma unroll 1
+                for (int k = 0; k < 9; ++k) {
+                    const float ax = nd_m(Gd.ax, Gd.muvw, cx + k / 3, cy + k % 3, gsx, gsy);
+                    const float ay = nd_m(Gd.ay, Gd.muvw, cx + k / 3, cy + k % 3, gsx, gsy);
+                    for (int q = 0; q < 9; ++q) {  // (no indexed registers)
+                        nax[q] = q == k ? ax : nax[q];
+                        nay[q] = q == k ? ay : nay[q];
                     }
-                    u += phi * (ax + cax);
-                    v += phi * (ay + cay);
                 }
+            }
+            for (int k = 0; k < 9; ++k) {
+                const double phi = px[k / 3] * py[k % 3];
+                u += phi * (nax[k] + cax);
+                v += phi * (nay[k] + cay);
+            }
             if (home) {  // other tiles still read the old velocity
                 P.u2[slot] = u;
                 P.v2[slot] = v;
@@ -977,14 +1040,13 @@ __global__ __launch_bounds__(kT) void k_g2p(Particles P, Grid Gd, int gsx, int g
             const bool act = valid || home;
             const double mu = act ? (it.mature ? u : u * 0.0) : 0.0;
             const double mv = act ? (it.mature ? v : v * 0.0) : 0.0;
-            const Seg S = segments(valid, cx, cy);
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) {
-                    const double phi = px[a] * py[b];
-                    const float v0 = valid ? float(phi * mu) : 0.0f;
-                    const float v1 = valid ? float(phi * mv) : 0.0f;
-                    tile_add2(acc, S, valid, cx, cy, x0, y0, a, b, v0, v1);
-                }
+            float p[18];
+            for (int k = 0; k < 9; ++k) {
+                const double phi = px[k / 3] * py[k % 3];
+                p[k] = valid ? float(phi * mu) : 0.0f;
+                p[9 + k] = valid ? float(phi * mv) : 0.0f;
+            }
+            acc.put(p, valid, cx, cy, x0, y0);
         }, stage);
         __syncthreads();
         store_tile2(acc, Gd.muvw + 1, Gd.muvw + 2, 4, x0, y0, gsx, gsy, single);

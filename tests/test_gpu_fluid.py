@@ -96,6 +96,35 @@ def test_fluid_step_matches_oracle_many_particles(layout):
         assert (outs[k][:, 16] == Q[:, 16]).all()
 
 
+@pytest.mark.parametrize("crowd", [1, 15, 16, 17, 63, 64, 65, 256, 257, 600])
+def test_fluid_step_of_crowded_cells_matches_oracle(crowd):
+    """Cells of `crowd` particles among thinly filled ones: runs of entries
+    that end at, before and after the cuts of the lanes' rows, of a wave and of
+    a work item, by a wall and away from it, in tiles that share nodes."""
+    rng = np.random.default_rng(crowd)
+    gsx, gsy = 64, 40
+    xy = [np.array([c]) + rng.uniform(0, 1, (crowd, 2)) for c in ((30.5, 20.5), (31.5, 20.5), (2.5, 3.5), (39.5, 23.5))]
+    xy.append(rng.uniform((2, 2), (gsx - 3, gsy - 3), (150, 2)))
+    xy = np.concatenate(xy)[rng.permutation(4 * crowd + 150)]
+    n = len(xy)
+    P = np.zeros((n, 20))
+    P[:, 0:2] = xy
+    P[:, 2:4] = rng.normal(0, 0.2, (n, 2))
+    P[:, 4:6] = xy + rng.normal(0, 3, (n, 2))
+    P[:, 6] = 1.0
+    P[:, 7:15] = rng.uniform(0, 1, (n, 8))
+    P[:, 15] = 1.0
+    P[:, 16] = 1.0
+    P[:, 17] = rng.integers(0, 2, n)
+    G.log(f"fluid step, {crowd} particles in a cell")
+    got = _step_gpu(P, gsx, gsy, 1, 20.0)[0]
+    want = P.copy()
+    op.oracle().or_fluid_step(op.ptr(want), n, gsx, gsy, 0, 20.0, 0)
+    for col, tol in TOL.items():
+        d = np.abs(got[:, col] - want[:, col]).max()
+        assert d <= tol, (col, d)
+
+
 def _clustered(rng, n, lo, hi, shift=0.0):
     """Particles in runs of 256 around random centres in [lo, hi)^2 (moved by
     shift cells), with velocities, attractors and colours."""
