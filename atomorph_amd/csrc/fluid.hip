@@ -80,53 +80,6 @@ __device__ __forceinline__ void weights(double x, double y, int &cx, int &cy, do
 __device__ __forceinline__ bool node_ok(int i, int j, int gsx, int gsy) { return i >= 0 && j >= 0 && i < gsx && j < gsy; }
 
 // ---------------------------------------------------- stencil scatter
-// Particles scatter into the 3x3 nodes around them.  Neighbouring atoms of a
-// chain stay close together, so the nodes one block's particles touch form a
-// small box: the block sums its contributions into an LDS copy of that box
-// (LDS atomics) and then adds each touched node to the grid once per field.
-// That turns ~9 contended global atomics per particle and field into one per
-// node.  A block whose box exceeds the tile scatters straight to the grid.
-struct Box {
-    int x0, y0, w, h;
-    bool fits;
-};
-
-// Bounding box of the E x E stencils at (cx, cy) of the block's valid
-// particles; fits when it has at most NODES entries.
-template <int NODES, int E = 3>
-__device__ Box block_box(bool valid, int cx, int cy, int *red) {
-    int mnx = valid ? cx : 0x7FFFFFFF, mny = valid ? cy : 0x7FFFFFFF;
-    int mxx = valid ? cx : -0x7FFFFFFF, mxy = valid ? cy : -0x7FFFFFFF;
-    for (int off = 32; off > 0; off >>= 1) {
-        mnx = min(mnx, __shfl_xor(mnx, off, 64));
-        mny = min(mny, __shfl_xor(mny, off, 64));
-        mxx = max(mxx, __shfl_xor(mxx, off, 64));
-        mxy = max(mxy, __shfl_xor(mxy, off, 64));
-    }
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        red[wave * 4 + 0] = mnx;
-        red[wave * 4 + 1] = mny;
-        red[wave * 4 + 2] = mxx;
-        red[wave * 4 + 3] = mxy;
-    }
-    __syncthreads();
-    for (int w = 0; w < kT / 64; ++w) {
-        mnx = min(mnx, red[w * 4 + 0]);
-        mny = min(mny, red[w * 4 + 1]);
-        mxx = max(mxx, red[w * 4 + 2]);
-        mxy = max(mxy, red[w * 4 + 3]);
-    }
-    Box b;
-    b.x0 = mnx;
-    b.y0 = mny;
-    const int64_t w = int64_t(mxx) - mnx + E, h = int64_t(mxy) - mny + E;
-    b.fits = mnx <= mxx && w * h <= NODES;
-    b.w = b.fits ? int(w) : 0;
-    b.h = b.fits ? int(h) : 0;
-    return b;
-}
-
 // Runs of consecutive lanes whose particles share a stencil origin form
 // segments (the cell order makes such runs common), cut at the rows of 16
 // lanes that DPP shifts within.  seg_sums leaves each segment's totals in its
@@ -308,7 +261,8 @@ struct Bins {
     int32_t *start;     // [tiles + 1]
     int32_t *rank;      // [4][n]: place of particle i's j-th entry in its bin
     int32_t *list;      // [<= 4n] slot | kHome, grouped by bin
-    // Work items of kT entries at most, each one workgroup (chunk NULL:
+    int32_t item;         // entries of a work item at most, one per thread
+    // Work items of `item` entries at most, each one workgroup (chunk NULL:
     // whole bins, one workgroup per tile, from start[]).  A dense bin is
     // split over several items, which add their node sums with atomics to
     // nodes cleared when the bins were placed; a tile with one item stores
@@ -316,12 +270,11 @@ struct Bins {
     // for each tile that had entries in the step before and has none now,
     // which stores zeros: a tile empty in both steps keeps the zeros stored
     // then.  chunk[b] = (tile, entries, only item of its tile, 0), b <
-    // *nchunks, in tile order; item b's entries are list[kT * b ...], so a
+    // nchunks[par], tiles in groups; item b's entries are list[item * b ...], so a
     // tile kernel loads its entry together with the descriptor.
     int4 *chunk;
-    int32_t *nchunks;     // this step's item count
-    int32_t max_chunks;   // capacity of chunk (an upper bound of *nchunks)
-    int32_t *items;       // [tiles] items per tile (scratch of grids beyond kLdsTiles)
+    int32_t *nchunks;     // [2] item count per step parity; the other parity is zero
+    int32_t max_chunks;   // capacity of chunk (an upper bound of the item count)
     int32_t par;          // this step's count parity (the other is cleared by k_p2g)
 };
 constexpr int kLdsTiles = 4096;  // up to this many tiles the placing blocks scan the counts in LDS
@@ -357,21 +310,16 @@ struct StencilTiles {  // the step: tiles holding the 3x3 stencil nodes
         stencil_tiles(P.x[i], P.y[i], gsx, gsy, tx0, tx1, ty0, ty1);
         return act != 0;
     }
-    // Zeroes every field of tile t's nodes (the workgroup together).
+    // Zeroes every field of tile t's nodes (a wave, one node per lane).
     __device__ __forceinline__ void clear_tile(int t, int nty) const {
-        const int x0 = (t / nty) * kTile, y0 = (t % nty) * kTile;
-        for (int e = threadIdx.x; e < kTile * kTile * kGridFields; e += kT) {
-            const int node = e % (kTile * kTile), field = e / (kTile * kTile);
-            const int ni = x0 + node / kTile, nj = y0 + node % kTile;
-            if (ni >= gsx || nj >= gsy) continue;
-            const int64_t k = int64_t(ni) * gsy + nj;
-            if (field < 4) G.muvw[4 * k + field] = 0.0f;
-            else if (field < 8) G.col[4 * k + field - 4] = 0.0f;
-            else {
-                float *f[4] = {G.gx, G.gy, G.ax, G.ay};
-                f[field - 8][k] = 0.0f;
-            }
-        }
+        static_assert(kTile * kTile == 64, "one node per lane");
+        const int lane = threadIdx.x & 63;
+        const int ni = (t / nty) * kTile + lane / kTile, nj = (t % nty) * kTile + lane % kTile;
+        if (ni >= gsx || nj >= gsy) return;
+        const int64_t k = int64_t(ni) * gsy + nj;
+        reinterpret_cast<float4 *>(G.muvw)[k] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+        reinterpret_cast<float4 *>(G.col)[k] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+        G.gx[k] = G.gy[k] = G.ax[k] = G.ay[k] = 0.0f;
     }
 };
 
@@ -446,15 +394,15 @@ __global__ __launch_bounds__(kT) void k_bin_count(Tiles tiles_of, int n, Bins B,
 }
 
 // Work items of a tile with c entries that had `before` entries in the step
-// before: ceil(c / kT) chunks, or one empty item (which zeroes the tile's
+// before: ceil(c / item) chunks, or one empty item (which zeroes the tile's
 // nodes) when the tile has just emptied, or none.
-__device__ __forceinline__ int work_items(int c, int before) {
-    return c > 0 ? (c + kT - 1) / kT : (before > 0 ? 1 : 0);
+__device__ __forceinline__ int work_items(const Bins &B, int c, int before) {
+    return c > 0 ? (c + B.item - 1) / B.item : (before > 0 ? 1 : 0);
 }
 
 // The nc work items of tile t (c entries) at B.chunk[c0 ...].
 __device__ __forceinline__ void put_items(const Bins &B, int c0, int nc, int t, int c) {
-    for (int j = 0; j < nc; ++j) B.chunk[c0 + j] = make_int4(t, max(0, min(kT, c - j * kT)), nc == 1, 0);
+    for (int j = 0; j < nc; ++j) B.chunk[c0 + j] = make_int4(t, max(0, min(B.item, c - j * B.item)), nc == 1, 0);
 }
 
 // Nothing more for particle i (k_bin_place's default tail).
@@ -496,19 +444,44 @@ __global__ __launch_bounds__(kT) void k_bin_place(Tiles tiles_of, int n, Bins B,
     if (i < n) tail(i);
 }
 
-// Work items per tile from its count and the step before's (grids beyond
-// kLdsTiles tiles, before the device scan of B.items into B.start).
-__global__ __launch_bounds__(kT) void k_tile_items(Bins B, int tiles, int par) {
-    const int k = blockIdx.x * kT + threadIdx.x;
-    if (k < tiles) B.items[k] = work_items(B.count[par][k], B.count[par ^ 1][k]);
+// The work items of kItemTiles tiles per workgroup (grids beyond kLdsTiles
+// tiles): their places are a scan within the group from a base taken off the
+// step's item count, so groups lie in any order, and B.start[t] is the first
+// of tile t.  Nodes of tiles split over several items start from zero.
+// (One launch of 5 us where items per tile, their device scan and the
+// descriptors took three of 14 us together, at 17,161 tiles.)
+constexpr int kItemTiles = 128;
+
+__global__ __launch_bounds__(kT) void k_tile_items(StencilTiles tiles_of, Bins B, int tiles, int par) {
+    __shared__ int sfirst[kItemTiles + 1], scount[kItemTiles];
+    __shared__ int wsum[kT / 64];
+    __shared__ int sbase;
+    const int t0 = blockIdx.x * kItemTiles, m = min(kItemTiles, tiles - t0);
+    scan::block_exclusive(m, [&](int k) {
+        const int c = B.count[par][t0 + k], before = B.count[par ^ 1][t0 + k];
+        scount[k] = c;
+        return work_items(B, c, before);
+    }, sfirst, wsum);
+    if (threadIdx.x == 0) sbase = sfirst[m] > 0 ? atomicAdd(&B.nchunks[par], sfirst[m]) : 0;
+    __syncthreads();
+    for (int k = threadIdx.x; k < m; k += kT) {
+        const int first = sbase + sfirst[k];
+        B.start[t0 + k] = first;
+        put_items(B, first, sfirst[k + 1] - sfirst[k], t0 + k, scount[k]);
+    }
+    // each wave its quarter of the group
+    const int lane = threadIdx.x & 63, k0 = int(threadIdx.x >> 6) * (kItemTiles / (kT / 64));
+    const bool split = lane < kItemTiles / (kT / 64) && k0 + lane < m && scount[k0 + lane] > B.item;
+    for (uint64_t todo = __ballot(split); todo; todo &= todo - 1)
+        tiles_of.clear_tile(t0 + k0 + __ffsll((unsigned long long)todo) - 1, B.nty);
 }
 
-// The fluid steps' bins: tile t's entries are laid out from list[kT *
-// first[t]], kT per work item (the last item of a tile partly filled), so
-// that item b's entries sit at list[kT * b ...].  first[] is the scan of
+// The fluid steps' bins: tile t's entries are laid out from list[item *
+// first[t]], `item` per work item (the last item of a tile partly filled), so
+// that item b's entries sit at list[item * b ...].  first[] is the scan of
 // the tiles' item counts: with kLds every block scans them in LDS (block 0
-// also writes the item descriptors and their number); otherwise B.start
-// holds it already (k_tile_items and the device scan).  The step before's
+// also writes the item descriptors and their number); otherwise k_tile_items
+// has placed the items.  The step before's
 // counts, which every placing block reads here, are cleared by k_p2g.  The
 // grid covers max(n, tiles) threads.
 template <bool kLds>
@@ -528,27 +501,21 @@ __global__ __launch_bounds__(kT) void k_item_place(StencilTiles tiles_of, int n,
         scan::block_exclusive(tiles, [&](int k) {
             const int c = B.count[par][k], before = B.count[par ^ 1][k];
             scount[k] = c;
-            return work_items(c, before);
+            return work_items(B, c, before);
         }, sfirst, wsum);
         first = sfirst;
         if (blockIdx.x == 0) {
             for (int k = threadIdx.x; k < tiles; k += kT) put_items(B, sfirst[k], sfirst[k + 1] - sfirst[k], k, scount[k]);
-            if (threadIdx.x == 0) *B.nchunks = sfirst[tiles];
+            if (threadIdx.x == 0) B.nchunks[par] = sfirst[tiles];
         }
         // nodes of tiles split over several items start from zero
-        for (int t = blockIdx.x; t < tiles; t += gridDim.x)
-            if (scount[t] > kT) tiles_of.clear_tile(t, B.nty);
-    } else {
-        for (int k = blockIdx.x * kT + threadIdx.x; k < tiles; k += gridDim.x * kT)
-            put_items(B, first[k], first[k + 1] - first[k], k, B.count[par][k]);
-        if (blockIdx.x == 0 && threadIdx.x == 0) *B.nchunks = first[tiles];
-        for (int t = blockIdx.x; t < tiles; t += gridDim.x)
-            if (B.count[par][t] > kT) tiles_of.clear_tile(t, B.nty);
+        for (int t = blockIdx.x * (kT / 64) + int(threadIdx.x >> 6); t < tiles; t += gridDim.x * (kT / 64))
+            if (scount[t] > B.item) tiles_of.clear_tile(t, B.nty);
     }
     if (!binned) return;
     for (int j = 0; j < 4; ++j) {
         const int t = entry_tile(j, tx0, tx1, ty0, ty1, B.nty);
-        if (t >= 0) B.list[int64_t(first[t]) * kT + rank[j]] = i | (j == 0 ? kHome : 0);
+        if (t >= 0) B.list[int64_t(first[t]) * B.item + rank[j]] = i | (j == 0 ? kHome : 0);
     }
 }
 
@@ -587,27 +554,31 @@ __device__ __forceinline__ void for_bin(const Bins &B, int s0, int s1, const Fet
     }
 }
 
-// Work item b of a tile kernel: tile t, whether it is the tile's only item
-// (then it stores its nodes; otherwise it adds them atomically), and this
-// thread's entry of it (slot -1 past the item's entries, home: the
-// particle's home tile).  The item's entries are list[kT * b ...], so the
-// entry is loaded together with the descriptor, not after it (both reads
-// are in bounds for every b: b is clamped to the descriptors' capacity and
-// the list holds kT entries per descriptor).  false: past the last item.
-// Workgroups take items b = blockIdx.x, blockIdx.x + gridDim.x, ...;
-// nchunks = *B.nchunks.
-__device__ __forceinline__ bool tile_item(const Bins &B, int nchunks, int b, int &t, bool &single, int &slot,
-                                          bool &home) {
+// Work item b of a tile kernel as its workgroup reads it: the descriptor and
+// this thread's entry.  The item's entries are list[NT * b ...], so the
+// entry is loaded together with the descriptor, not after it; k_p2g loads
+// both for its next item while it works on one (the reads are in bounds
+// for every b: b is clamped to the descriptors' capacity and the list holds
+// NT entries per descriptor).  Workgroups take items b = blockIdx.x,
+// blockIdx.x + gridDim.x, ... below B.nchunks[B.par].
+struct ItemWords {
+    int4 c;
+    int e;
+};
+template <int NT>
+__device__ __forceinline__ ItemWords load_item(const Bins &B, int b) {
     const int bc = min(b, B.max_chunks - 1);
-    const int4 c = B.chunk[bc];
-    const int e = B.list[int64_t(bc) * kT + threadIdx.x];
-    if (b >= nchunks) return false;
-    t = c.x;
-    single = c.z != 0;
-    const bool has = int(threadIdx.x) < c.y;
-    slot = has ? (e & 0x7FFFFFFF) : -1;
-    home = has && e < 0;
-    return true;
+    return {B.chunk[bc], B.list[int64_t(bc) * NT + threadIdx.x]};
+}
+// Its tile, whether it is the tile's only item (then it stores its nodes;
+// otherwise it adds them atomically), and this thread's entry (slot -1
+// past the item's entries, home: the particle's home tile).
+__device__ __forceinline__ void tile_item(const ItemWords &w, int &t, bool &single, int &slot, bool &home) {
+    t = w.c.x;
+    single = w.c.z != 0;
+    const bool has = int(threadIdx.x) < w.c.y;
+    slot = has ? (w.e & 0x7FFFFFFF) : -1;
+    home = has && w.e < 0;
 }
 
 // body(slot, home, item) on this thread's entry, item = fetch(slot) holding
@@ -643,28 +614,30 @@ __device__ __forceinline__ int halo_index(int i, int j, int x0, int y0) {
 }
 
 // A node halo staged in LDS in two parts: load() issues this thread's loads
-// of R raw fields (thread e < kHalo^2 takes halo entry e, the others repeat
-// the last entry, so no load or LDS write sits in a branch and the loads
+// of R raw fields (thread e takes halo entries e, e + NT, the last ones past
+// the end, so no load or LDS write sits in a branch and the loads
 // overlap the bin list's), store() writes F fields computed from them once
 // they arrive.  raw(f, k) = raw field f at grid index k; value(f, r) = staged
 // field f from the raw values r.  Nodes outside the grid stage 0.
-static_assert(kHalo * kHalo <= kT, "one halo entry per thread");
-template <int R>
+template <int R, int NT>
 struct Halo {
-    float r[R];
-    int e;
-    bool ok;
+    static constexpr int kPer = (kHalo * kHalo + NT - 1) / NT;
+    float r[kPer][R];
+    bool ok[kPer];
+    __device__ __forceinline__ static int entry(int q) { return min(int(threadIdx.x) + q * NT, kHalo * kHalo - 1); }
     template <class Raw>
     __device__ __forceinline__ void load(int x0, int y0, int gsx, int gsy, const Raw &raw) {
-        e = min(int(threadIdx.x), kHalo * kHalo - 1);
-        const int i = x0 - 2 + e / kHalo, j = y0 - 2 + e % kHalo;
-        ok = node_ok(i, j, gsx, gsy);
-        const int64_t k = ok ? int64_t(i) * gsy + j : 0;
-        for (int f = 0; f < R; ++f) r[f] = raw(f, k);
+        for (int q = 0; q < kPer; ++q) {
+            const int e = entry(q), i = x0 - 2 + e / kHalo, j = y0 - 2 + e % kHalo;
+            ok[q] = node_ok(i, j, gsx, gsy);
+            const int64_t k = ok[q] ? int64_t(i) * gsy + j : 0;
+            for (int f = 0; f < R; ++f) r[q][f] = raw(f, k);
+        }
     }
     template <int F, class Value>
     __device__ __forceinline__ void store(float (&sm)[F][kHalo * kHalo], const Value &value) const {
-        for (int f = 0; f < F; ++f) sm[f][e] = ok ? value(f, r) : 0.0f;
+        for (int q = 0; q < kPer; ++q)
+            for (int f = 0; f < F; ++f) sm[f][entry(q)] = ok[q] ? value(f, r[q]) : 0.0f;
     }
 };
 
@@ -674,16 +647,15 @@ struct Halo {
 // totals are kept aside and added once the stores are done.  (LDS float
 // atomics take about one cycle per lane and bound these kernels when each
 // segment added its totals.)
-constexpr int kRows = kT / 16;  // rows of lanes
-
-template <int N>
+template <int N, int NT>
 struct CellSums {
+    static constexpr int kRows = NT / 16;  // rows of lanes
     float v[N][kReach * kReach];
     float cut[N][kRows];
     int cell[kRows];  // the cell of a row's cut run, -1 none
 
     __device__ __forceinline__ void clear() {
-        for (int k = threadIdx.x; k < N * kReach * kReach; k += kT) (&v[0][0])[k] = 0.0f;
+        for (int k = threadIdx.x; k < N * kReach * kReach; k += NT) (&v[0][0])[k] = 0.0f;
         if (threadIdx.x < kRows) cell[threadIdx.x] = -1;
     }
     // Every lane of the wave calls it (c: zeros unless valid, destroyed);
@@ -704,7 +676,7 @@ struct CellSums {
     __device__ __forceinline__ void join() {
         const int row = threadIdx.x % kRows, at = cell[row];
         if (at < 0) return;
-        for (int k = threadIdx.x / kRows; k < N; k += kT / kRows) atomicAdd(&v[k][at], cut[k][row]);
+        for (int k = threadIdx.x / kRows; k < N; k += NT / kRows) atomicAdd(&v[k][at], cut[k][row]);
     }
 };
 
@@ -724,43 +696,48 @@ struct P2gItem {
 // step; without the sort a cell would be many runs.
 //
 // Instructions and LDS bound this kernel, k_forces and k_g2p.  One MI355X,
-// 229k particles on 276^2 nodes (1044^2), us: here 18.2 -> 13.6 (37 -> 22),
-// k_forces 12.5 -> 10.1 (26 -> 20), k_g2p 14.7 -> 11.2 (34 -> 21), before with
-// LDS atomics per run and node and sums carried across the lanes' rows.
+// 229k particles on 276^2 nodes (1044^2), us: here 18.2 -> 12.4 (37 -> 18.5),
+// k_forces 12.5 -> 10.1 (26 -> 17), k_g2p 14.7 -> 11.5 (34 -> 20), before with
+// LDS atomics per run and node, sums carried across the lanes' rows and kT
+// threads on either grid.
 //
 // Six waves per SIMD (72 VGPRs): the LDS (19 KB) allows eight blocks per
 // CU; seven waves spilled when there were more registers, which measured
 // slower.
-__global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_p2g(Particles P, Grid Gd, int gsx,
+template <int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_p2g(Particles P, Grid Gd, int gsx,
                                                                                    int gsy, Bins B) {
-    __shared__ CellSums<kCellSums> sums;
+    __shared__ CellSums<kCellSums, NT> sums;
     const auto &cs = sums.v;
     constexpr int kCells = kReach * kReach;  // local cells; bucket kCells: out of reach
     __shared__ int cellpos[kCells + 2];  // per bucket: count, then first place
-    __shared__ int2 mine[kT];            // per thread: its list entry, (bucket << 8) | rank (-1: no entry)
-    __shared__ int perm[kT];             // sorted place -> thread
+    __shared__ int2 mine[NT];            // per thread: its list entry, (bucket << 8) | rank (-1: no entry)
+    __shared__ int perm[NT];             // sorted place -> thread
     // The chunk's items (position and colour terms), one array per field so
     // that consecutive lanes write consecutive words; dead once the cells
     // are summed, so they share their space with the node assembly's partials.
     union Stage {
         struct {
-            double x[kT], y[kT];
-            float t[5][kT];
+            double x[NT], y[NT];
+            float t[5][NT];
         } item;
         float part[3][8][kTile * kTile];
     };
     __shared__ Stage stage;
     static_assert(kCells + 2 <= 2 * 64, "one wave scans the buckets, two per lane");
     static_assert(kTile * kTile == 64, "one wave per column of cells in the node assembly");
-    const int nchunks = *B.nchunks;
+    const int nchunks = B.nchunks[B.par];
+    ItemWords next = load_item<NT>(B, int(blockIdx.x));
     // the step before's counts, read by every placing block, are cleared
     // here for the next step's counting
-    for (int k = blockIdx.x * kT + threadIdx.x; k < B.ntx * B.nty; k += gridDim.x * kT) B.count[B.par ^ 1][k] = 0;
-    for (int item = int(blockIdx.x);; item += int(gridDim.x)) {
+    for (int k = blockIdx.x * NT + threadIdx.x; k < B.ntx * B.nty; k += gridDim.x * NT) B.count[B.par ^ 1][k] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) B.nchunks[B.par ^ 1] = 0;
+    for (int item = int(blockIdx.x); item < nchunks; item += int(gridDim.x)) {
         int tile, slot0;
         bool single, home0;
-        if (!tile_item(B, nchunks, item, tile, single, slot0, home0)) break;
-        const int64_t s0 = int64_t(item) * kT;  // the item's entries in the list
+        tile_item(next, tile, single, slot0, home0);
+        next = load_item<NT>(B, item + int(gridDim.x));
+        const int64_t s0 = int64_t(item) * NT;  // the item's entries in the list
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
         // every field load is unconditional (slot -1, past the end of the
@@ -772,7 +749,7 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
         };
         const auto clear = [&] {
             sums.clear();
-            if (threadIdx.x < kCells + 2) cellpos[threadIdx.x] = 0;
+            for (int k = threadIdx.x; k < kCells + 2; k += NT) cellpos[k] = 0;
             // an empty item (a tile that has just emptied) never runs the body
             mine[threadIdx.x] = make_int2(0, -1);
             __syncthreads();
@@ -803,7 +780,7 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             sums.put(c, valid, cx, cy, x0, y0);
         };
         {
-            // at most kT entries: one pass, ranks fit in 8 bits
+            // at most NT entries: one pass, ranks fit in 8 bits
             run_item(slot0, home0, fetch, [&](int slot, bool home, const P2gItem &it) {
                 const int cx = static_cast<int>(it.x - 0.5), cy = static_cast<int>(it.y - 0.5);
                 const int bucket = in_reach(cx, cy, x0, y0) ? (cx - x0 + 2) * kReach + (cy - y0 + 2) : kCells;
@@ -853,15 +830,13 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
         __syncthreads();
         sums.join();
         __syncthreads();
-        // Nodes from the cells: thread (a, node) sums the three cells
+        // Nodes from the cells: one wave per a, thread (a, node) sums the three cells
         // (node - (a, b)), then one thread per node adds the three partials.
         auto &part = stage.part;
-        static_assert(3 * kTile * kTile <= kT, "one thread per (a, node)");
         {
             const int node = threadIdx.x % (kTile * kTile);
             // (the same in all of a wave)
-            const int a = __builtin_amdgcn_readfirstlane(threadIdx.x / (kTile * kTile));
-            if (a < 3) {
+            for (int a = __builtin_amdgcn_readfirstlane(threadIdx.x / 64); a < 3; a += NT / 64) {
                 const int ni = node / kTile, nj = node % kTile;
                 float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
                 for (int b = 0; b < 3; ++b) {
@@ -895,14 +870,17 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(6))) void k_
 
 // Per cell what its particles add to the two sums of node (cell + (a, b)):
 // [3 a + b] and [9 + 3 a + b].
-using StencilSums = CellSums<18>;
+template <int NT>
+using StencilSums = CellSums<18, NT>;
 
 // Stores (or adds) the tile's node sums into fields f0, f1, each node's from
 // the cells that reach it: node k's values at f0[stride*k], f1[stride*k].
-__device__ __forceinline__ void store_tile2(StencilSums &sums, float *f0, float *f1, int stride, int x0, int y0,
+template <int NT>
+__device__ __forceinline__ void store_tile2(StencilSums<NT> &sums, float *f0, float *f1, int stride, int x0, int y0,
                                             int gsx, int gsy, bool single) {
     sums.join();
     __syncthreads();
+    static_assert(2 * kTile * kTile <= NT, "one thread per node and field");
     const int t = threadIdx.x % (kTile * kTile), f = threadIdx.x / (kTile * kTile);
     if (f >= 2) return;
     const int ni = x0 + t / kTile, nj = y0 + t % kTile;
@@ -915,20 +893,21 @@ __device__ __forceinline__ void store_tile2(StencilSums &sums, float *f0, float 
 }
 
 // Node accelerations: pressure and wall forces (fluidmodel.cpp:251-357).
-__global__ __launch_bounds__(kT) void k_forces(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
-    __shared__ StencilSums acc;
+template <int NT>
+__global__ __launch_bounds__(NT) void k_forces(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
+    __shared__ StencilSums<NT> acc;
     __shared__ float nodes[3][kHalo * kHalo];  // m, gx, gy
-    const int nchunks = *B.nchunks;
-    for (int item = int(blockIdx.x);; item += int(gridDim.x)) {
+    const int nchunks = B.nchunks[B.par];
+    for (int item = int(blockIdx.x); item < nchunks; item += int(gridDim.x)) {
         int tile, slot0;
         bool single, home0;
-        if (!tile_item(B, nchunks, item, tile, single, slot0, home0)) break;
+        tile_item(load_item<NT>(B, item), tile, single, slot0, home0);
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
         acc.clear();
         // the halo's loads are issued beside the particles', which are
         // unconditional (slot -1 reads particle 0)
-        Halo<3> halo;
+        Halo<3, NT> halo;
         halo.load(x0, y0, gsx, gsy,
                   [&](int f, int64_t k) { return f == 0 ? Gd.muvw[4 * k] : f == 1 ? Gd.gx[k] : Gd.gy[k]; });
         const auto stage = [&] {
@@ -966,7 +945,7 @@ __global__ __launch_bounds__(kT) void k_forces(Particles P, Grid Gd, int gsx, in
             acc.put(v, valid, cx, cy, x0, y0);
         }, stage);
         __syncthreads();
-        store_tile2(acc, Gd.ax, Gd.ay, 1, x0, y0, gsx, gsy, single);
+        store_tile2<NT>(acc, Gd.ax, Gd.ay, 1, x0, y0, gsx, gsy, single);
         __syncthreads();  // the LDS sums are reused by the next item
     }
 }
@@ -979,19 +958,20 @@ struct G2pItem {
 // Particle velocity from node accelerations plus the attractor (written by
 // the particle's home tile), then the momentum of the tile's nodes
 // (fluidmodel.cpp:359-437).
-__global__ __launch_bounds__(kT) void k_g2p(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
-    __shared__ StencilSums acc;
+template <int NT>
+__global__ __launch_bounds__(NT) void k_g2p(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
+    __shared__ StencilSums<NT> acc;
     __shared__ float accel[2][kHalo * kHalo];  // node accelerations per mass
-    const int nchunks = *B.nchunks;
-    for (int item = int(blockIdx.x);; item += int(gridDim.x)) {
+    const int nchunks = B.nchunks[B.par];
+    for (int item = int(blockIdx.x); item < nchunks; item += int(gridDim.x)) {
         int tile, slot0;
         bool single, home0;
-        if (!tile_item(B, nchunks, item, tile, single, slot0, home0)) break;
+        tile_item(load_item<NT>(B, item), tile, single, slot0, home0);
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
         acc.clear();
         // as in k_forces: halo loads beside the unconditional particle loads
-        Halo<3> halo;
+        Halo<3, NT> halo;
         halo.load(x0, y0, gsx, gsy,
                   [&](int f, int64_t k) { return f == 0 ? Gd.ax[k] : f == 1 ? Gd.ay[k] : Gd.muvw[4 * k]; });
         const auto stage = [&] {
@@ -1049,7 +1029,7 @@ __global__ __launch_bounds__(kT) void k_g2p(Particles P, Grid Gd, int gsx, int g
             acc.put(p, valid, cx, cy, x0, y0);
         }, stage);
         __syncthreads();
-        store_tile2(acc, Gd.muvw + 1, Gd.muvw + 2, 4, x0, y0, gsx, gsy, single);
+        store_tile2<NT>(acc, Gd.muvw + 1, Gd.muvw + 2, 4, x0, y0, gsx, gsy, single);
         __syncthreads();  // the LDS sums are reused by the next item
     }
 }
@@ -1466,12 +1446,22 @@ struct amh_fluid_s {
 };
 
 namespace {
+// Entries of a work item at most, and threads of its workgroup.  A grid of one
+// particle per node has about 100 entries in a filled tile, and half the
+// workgroup idles at kT (229k particles on 1044^2 nodes, 13 per tile: four
+// frames 3.9 ms at kT, 3.7 at kT / 2); the denser grids fill kT and would be
+// split, and added with atomics, twice as often (276^2 nodes, 187 per tile).
+size_t item_size(size_t tiles, size_t n) { return n > 64 * tiles ? kT : kT / 2; }
+
 // Upper bound of the chunks: every tile has at least one, and a particle
 // has at most 4 entries.
-size_t max_chunks(size_t tiles, size_t n) { return tiles + (4 * n + kT - 1) / kT + 1; }
-// Entries of the list: kT per work item (the steps' items start on kT
-// boundaries), at least the 4n of whole bins (the splat shares the list).
-size_t list_entries(size_t tiles, size_t n) { return std::max(4 * n, size_t(kT) * max_chunks(tiles, n)); }
+size_t max_chunks(size_t tiles, size_t n) {
+    const size_t item = item_size(tiles, n);
+    return tiles + (4 * n + item - 1) / item + 1;
+}
+// Entries of the list: item_size per work item, at least the 4n of whole bins
+// (the splat shares the list).
+size_t list_entries(size_t tiles, size_t n) { return std::max(4 * n, item_size(tiles, n) * max_chunks(tiles, n)); }
 
 size_t fluid_bytes(int gsx, int gsy, int count, int W, int H, int nkeys) {
     const size_t n = size_t(count), nn = size_t(gsx) * gsy, npx = size_t(W) * H;
@@ -1481,8 +1471,8 @@ size_t fluid_bytes(int gsx, int gsy, int count, int W, int H, int nkeys) {
     (void)nkeys;
     // every carved array is rounded up to 256 bytes: the last term covers that
     return 2 * (n * 8 * kParticleDoubles + n * 4 * kParticleInts) + n * 4 * 3 + (nn + kIdleBuckets + 1) * 4 * 2 +
-           (2 * nb + 1) * 4 + nn * 4 + (3 * tiles + 1) * 4 + n * 4 * 4 + list_entries(tiles, n) * 4 + tiles * 4 +
-           (3 * ptiles + 1) * 4 + n * (4 + 32 + 4) + max_chunks(tiles, n) * 16 + 4 + nn * 4 * kGridFields +
+           (2 * nb + 1) * 4 + nn * 4 + (3 * tiles + 1) * 4 + n * 4 * 4 + list_entries(tiles, n) * 4 +
+           (3 * ptiles + 1) * 4 + n * (4 + 32 + 4) + max_chunks(tiles, n) * 16 + 8 + nn * 4 * kGridFields +
            npx * 4 * 2 + 256 + n * sizeof(LagSlopeMemo) + 128 * 256;
 }
 
@@ -1536,11 +1526,11 @@ extern "C" int amh_fluid_create(void **fluid, int32_t gsx, int32_t gsy, int32_t 
     f->bins.count[1] = reinterpret_cast<int32_t *>(take(tiles * 4));
     f->bins.start = reinterpret_cast<int32_t *>(take((tiles + 1) * 4));
     f->bins.rank = reinterpret_cast<int32_t *>(take(n * 4 * 4));
+    f->bins.item = int32_t(item_size(tiles, n));
     f->bins.max_chunks = int32_t(max_chunks(tiles, n));
     f->bins.list = reinterpret_cast<int32_t *>(take(list_entries(tiles, n) * 4));
     f->bins.chunk = reinterpret_cast<int4 *>(take(size_t(f->bins.max_chunks) * 16));
-    f->bins.nchunks = reinterpret_cast<int32_t *>(take(4));
-    f->bins.items = reinterpret_cast<int32_t *>(take(tiles * 4));
+    f->bins.nchunks = reinterpret_cast<int32_t *>(take(8));
     f->pbins.ntx = (width + kPxTile - 1) / kPxTile;
     f->pbins.nty = (height + kPxTile - 1) / kPxTile;
     const size_t ptiles = size_t(f->pbins.ntx) * size_t(f->pbins.nty);
@@ -1551,8 +1541,8 @@ extern "C" int amh_fluid_create(void **fluid, int32_t gsx, int32_t gsy, int32_t 
     f->pbins.list = f->bins.list;
     f->pbins.chunk = nullptr;  // one workgroup per pixel tile
     f->pbins.nchunks = nullptr;
-    f->pbins.items = nullptr;
     f->pbins.max_chunks = 0;
+    f->pbins.item = 0;
     f->sxy = reinterpret_cast<uint32_t *>(take(n * 4));
     f->staps = reinterpret_cast<double *>(take(n * 32));
     f->scol = reinterpret_cast<uint32_t *>(take(n * 4));
@@ -1703,19 +1693,17 @@ void bin_particles(const Tiles &tiles_of, int n, const Bins &B, int tiles, int p
 }
 
 // The fluid steps' bins and work items (counted: the counts and ranks are in
-// place already).  Beyond kLdsTiles tiles the tiles' item counts are
-// scanned first, by the device scan (scan::exclusive) on the workspace
-// sums, offs (scan::blocks(tiles) and one more).
+// place already).
 void place_items(const StencilTiles &tiles_of, int n, const Bins &B, int tiles, int par, hipStream_t s,
-                 bool counted, int *sums, int *offs) {
+                 bool counted) {
     const uint32_t gp = uint32_t((n + kT - 1) / kT);
     if (!counted) hipLaunchKernelGGL(k_bin_count<StencilTiles>, dim3(gp), dim3(kT), 0, s, tiles_of, n, B, par);
     const uint32_t gb = uint32_t((std::max(n, tiles) + kT - 1) / kT);
     if (tiles <= kLdsTiles) {
         hipLaunchKernelGGL(k_item_place<true>, dim3(gb), dim3(kT), 0, s, tiles_of, n, B, tiles, par);
     } else {
-        hipLaunchKernelGGL(k_tile_items, dim3(uint32_t((tiles + kT - 1) / kT)), dim3(kT), 0, s, B, tiles, par);
-        scan::exclusive(B.items, tiles, sums, offs, B.start, s);
+        hipLaunchKernelGGL(k_tile_items, dim3(uint32_t((tiles + kItemTiles - 1) / kItemTiles)), dim3(kT), 0, s,
+                           tiles_of, B, tiles, par);
         hipLaunchKernelGGL(k_item_place<false>, dim3(gb), dim3(kT), 0, s, tiles_of, n, B, tiles, par);
     }
 }
@@ -1743,12 +1731,14 @@ int fluid_step_on(amh_fluid_s *f, const Particles &Q, const int32_t *atom, int32
     const uint32_t grid = uint32_t(std::min(B.max_chunks, 2 * std::min(tiles, kLdsTiles)));
     {
         amh::ProfScope ps_("fluid_bins", s);
-        place_items(StencilTiles{Q, f->gsx, f->gsy, f->G}, f->count, B, tiles, par, s, counted, f->scan_sums,
-                    f->scan_offs);
+        place_items(StencilTiles{Q, f->gsx, f->gsy, f->G}, f->count, B, tiles, par, s, counted);
     }
-    amh::launch_timed("k_p2g", k_p2g, dim3(grid), dim3(kT), 0, s, Q, f->G, f->gsx, f->gsy, B);
-    amh::launch_timed("k_forces", k_forces, dim3(grid), dim3(kT), 0, s, Q, f->G, f->gsx, f->gsy, B);
-    amh::launch_timed("k_g2p", k_g2p, dim3(grid), dim3(kT), 0, s, Q, f->G, f->gsx, f->gsy, B);
+    const bool whole = B.item == kT;
+    const dim3 items(uint32_t(B.item));
+    amh::launch_timed("k_p2g", whole ? k_p2g<kT> : k_p2g<kT / 2>, dim3(grid), items, 0, s, Q, f->G, f->gsx, f->gsy, B);
+    amh::launch_timed("k_forces", whole ? k_forces<kT> : k_forces<kT / 2>, dim3(grid), items, 0, s, Q, f->G, f->gsx,
+                      f->gsy, B);
+    amh::launch_timed("k_g2p", whole ? k_g2p<kT> : k_g2p<kT / 2>, dim3(grid), items, 0, s, Q, f->G, f->gsx, f->gsy, B);
     const uint32_t gp = uint32_t((f->count + kT - 1) / kT);
     if (splat)  // the frame's last step: the splat's per-particle half too
         amh::launch_timed("k_advect", k_advect<true>, dim3(gp), dim3(kT), 0, s, Q, f->count, f->G, f->gsx, f->gsy,

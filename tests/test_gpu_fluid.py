@@ -97,15 +97,16 @@ def test_fluid_step_matches_oracle_many_particles(layout):
 
 
 @pytest.mark.parametrize("crowd", [1, 15, 16, 17, 63, 64, 65, 256, 257, 600])
-def test_fluid_step_of_crowded_cells_matches_oracle(crowd):
+@pytest.mark.parametrize("fill", [150, 6000])  # both sizes of work items
+def test_fluid_step_of_crowded_cells_matches_oracle(crowd, fill):
     """Cells of `crowd` particles among thinly filled ones: runs of entries
     that end at, before and after the cuts of the lanes' rows, of a wave and of
     a work item, by a wall and away from it, in tiles that share nodes."""
     rng = np.random.default_rng(crowd)
     gsx, gsy = 64, 40
     xy = [np.array([c]) + rng.uniform(0, 1, (crowd, 2)) for c in ((30.5, 20.5), (31.5, 20.5), (2.5, 3.5), (39.5, 23.5))]
-    xy.append(rng.uniform((2, 2), (gsx - 3, gsy - 3), (150, 2)))
-    xy = np.concatenate(xy)[rng.permutation(4 * crowd + 150)]
+    xy.append(rng.uniform((2, 2), (gsx - 3, gsy - 3), (fill, 2)))
+    xy = np.concatenate(xy)[rng.permutation(4 * crowd + fill)]
     n = len(xy)
     P = np.zeros((n, 20))
     P[:, 0:2] = xy
