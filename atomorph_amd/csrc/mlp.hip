@@ -53,7 +53,7 @@ __device__ __forceinline__ float erf_as(float x) {
     const float y = fmaf(-poly, __expf(-ax * ax), 1.0f);
     return copysignf(y, x);
 }
-__device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erf_as(z * 0.70710678118654752f)); }
+__device__ __forceinline__ float gelu(float z) { return z * fmaf(0.5f, erf_as(z * 0.70710678118654752f), 0.5f); }
 // gelu(z) and its derivative d = cdf + z pdf; erf's exponential exp(-z^2 / 2)
 // is the density's too.
 __device__ __forceinline__ float gelu_and_d(float z, float &d) {
@@ -297,7 +297,10 @@ __global__ __launch_bounds__(kFusedThreads) void k_mlp_fused(const float *__rest
 
     const int64_t tiles = (n + 31) / 32;
     constexpr int kWaves = kFusedThreads / 64;
-    for (int64_t tile = int64_t(blockIdx.x) * kWaves + wave; tile < tiles; tile += int64_t(gridDim.x) * kWaves) {
+    // (a last turn that is not full leaves every workgroup some waves, not
+    // some workgroups none: 229k rows, 1.75 turns, 87 -> 73 us.  GELU, 94 of
+    // a SIMD's cycles for 64 values, bounds the rest.)
+    for (int64_t tile = int64_t(wave) * gridDim.x + blockIdx.x; tile < tiles; tile += int64_t(gridDim.x) * kWaves) {
         const int64_t row = tile * 32 + m;
         uint16_t xin[8];
 #pragma unroll
@@ -778,7 +781,8 @@ extern "C" int amh_mlp_forward(void *mlp, const float *x, int64_t n, float *out,
     amh::ProfScope ps_("mlp_forward", s);
     if (n == 0) return AMH_OK;
     const int64_t tiles = (n + 31) / 32;
-    const uint32_t grid = uint32_t(std::min<int64_t>(g_cus, (tiles + kFusedThreads / 64 - 1) / (kFusedThreads / 64)));
+    // from four waves' tiles a workgroup, one per SIMD, on more CUs first
+    const uint32_t grid = uint32_t(std::min<int64_t>(g_cus, (tiles + 3) / 4));
     if (M->image_stale) stage_image(M, s);
     hipLaunchKernelGGL(k_mlp_fused, dim3(grid), dim3(kFusedThreads), kFusedLds, s, x, n, M->image, out);
     AMH_LAUNCH_CHECK("amh_mlp_forward");

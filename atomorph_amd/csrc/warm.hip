@@ -22,7 +22,6 @@
 // position of each slot, normalised the same way) from converged chains.
 #include "common.h"
 #include "../../include/atomorph_hip.h"
-#include "scan.h"
 #include "shade.h"
 
 #include <algorithm>
@@ -100,38 +99,40 @@ __global__ __launch_bounds__(kT) void k_features(amh_render R, int y, const RowS
     }
 }
 
-// Raster key of a position at 1/16 px: set bit, chain, y, x, with cb chain
-// bits and cx bits per coordinate (positions clamped to the frame's range).
-__device__ __forceinline__ uint64_t raster_key(uint64_t set, uint64_t chain, double x, double y, int cb, int cx) {
+// Raster key of a position at 1/16 px: chain, y, x, with cx bits per
+// coordinate (positions clamped to the frame's range).
+__device__ __forceinline__ uint64_t raster_key(uint64_t chain, double x, double y, int cx) {
     const double lim = double((1ull << cx) - 1);
     const uint64_t fx = uint64_t(fmin(fmax(rint(x * 16.0), 0.0), lim));
     const uint64_t fy = uint64_t(fmin(fmax(rint(y * 16.0), 0.0), lim));
-    return (set << (cb + 2 * cx)) | (chain << (2 * cx)) | (fy << cx) | fx;
+    return (chain << (2 * cx)) | (fy << cx) | fx;
 }
 
-// One sort for both lists: keys [0, n) are the predictions for row y+1
-// (set 0), keys [n, 2n) the points row y+1 holds now (set 1); values are
-// the slots.  Sorted, set 0 and set 1 each list chain by chain (each chain
-// has its width in both), so rank r of chain c sits at the same offset in
-// both halves.
+// Two lists of n keys, sorted side by side: the predictions for row y+1, then
+// the points row y+1 holds now; values are the slots.  Sorted, each lists
+// chain by chain (each chain has its width in both), so rank r of chain c sits
+// at the same place in both.  The row's points are kept in row[] for
+// k_match_apply, which overwrites them.
 __global__ __launch_bounds__(kT) void k_match_keys(amh_render R, int yn, const RowStat *__restrict__ st,
-                                                  const float *__restrict__ pred, int cb, int cx,
-                                                  uint64_t *__restrict__ key, uint32_t *__restrict__ val) {
+                                                  const float *__restrict__ pred, int cx,
+                                                  uint64_t *__restrict__ key, uint32_t *__restrict__ val,
+                                                  uint64_t *__restrict__ row) {
     const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
     const int c = block_chain(R.chain_off_dev, R.nchains, a);
     if (a >= R.wtot) return;
     const RowStat s = st[int64_t(yn) * R.nchains + c];
     const double ux = s.cx + s.s * double(pred[a * 2 + 0]), uy = s.cy + s.s * double(pred[a * 2 + 1]);
     const uint64_t q = R.pts_dev[int64_t(yn) * R.wtot + a];
-    key[a] = raster_key(0, uint64_t(c), ux, uy, cb, cx);
+    key[a] = raster_key(uint64_t(c), ux, uy, cx);
     const uint64_t lim = (1ull << cx) - 1;
-    key[R.wtot + a] = (1ull << (cb + 2 * cx)) | (uint64_t(c) << (2 * cx)) |
-                      (min(uint64_t(pt_fy(q) >> 4), lim) << cx) | min(uint64_t(pt_fx(q) >> 4), lim);
+    key[R.wtot + a] =
+        (uint64_t(c) << (2 * cx)) | (min(uint64_t(pt_fy(q) >> 4), lim) << cx) | min(uint64_t(pt_fx(q) >> 4), lim);
+    row[a] = q;
     val[a] = uint32_t(a);
     val[R.wtot + a] = uint32_t(a);
 }
 
-// Rank r of both sorted halves pairs up inside one chain: the slot with the
+// Rank r of both sorted lists pairs up inside one chain: the slot with the
 // r-th prediction takes the r-th point.
 __global__ void k_match_apply(int64_t n, const uint32_t *__restrict__ sorted, const uint64_t *__restrict__ row,
                               uint64_t *__restrict__ out) {
@@ -140,67 +141,144 @@ __global__ void k_match_apply(int64_t n, const uint32_t *__restrict__ sorted, co
 }
 
 // ------------------------------------------------------- radix sort
-// LSD radix sort of (u64 key, u32 value) pairs, 8 bits per pass; a block
-// covers kRsTile elements; the scatter is stable (rank within a round from
-// per-digit lane masks built from eight ballots).
-constexpr int kRsTile = kT * 8;
+// LSD radix sort of two lists of n (u64 key, u32 value) pairs (blockIdx.y is
+// the list, the second n after the first) in as few passes of at most
+// kRsBits bits as the keys need, their bits dealt evenly; a block covers
+// kRsTile elements.  Launches and latency bound it: a pass is three launches
+// (digit counts per block, their prefix per digit, scatter), so it takes nine
+// bits rather than eight, and the scatter scans the digits' totals itself and
+// meets two barriers, not four for each 256 elements.  2 x 229k pairs of 36
+// bits on one MI355X: 72 us, 123 us as one list with a bit to tell them apart
+// in five passes of four launches.
+constexpr int kRsBits = 9, kRsDigits = 1 << kRsBits;
+constexpr int kRsPer = 4;  // elements of a thread
+constexpr int kRsTile = kT * kRsPer;
 
-__global__ __launch_bounds__(kT) void k_rs_hist(const uint64_t *__restrict__ key, int64_t n, int shift,
+__global__ __launch_bounds__(kT) void k_rs_hist(const uint64_t *__restrict__ key, int64_t n, int shift, uint32_t mask,
                                                int nblk, int *__restrict__ hist) {
-    __shared__ int h[256];
-    h[threadIdx.x] = 0;
+    __shared__ int h[kRsDigits];
+    for (int d = threadIdx.x; d < kRsDigits; d += kT) h[d] = 0;
     __syncthreads();
     const int64_t base = int64_t(blockIdx.x) * kRsTile;
-    for (int j = 0; j < 8; ++j) {
+    key += blockIdx.y * n;
+    hist += (int64_t(blockIdx.y) * nblk + blockIdx.x) * kRsDigits;
+    for (int j = 0; j < kRsPer; ++j) {
         const int64_t e = base + j * kT + threadIdx.x;
-        if (e < n) atomicAdd(&h[int((key[e] >> shift) & 255u)], 1);
+        if (e < n) atomicAdd(&h[uint32_t(key[e] >> shift) & mask], 1);
     }
     __syncthreads();
-    hist[int64_t(threadIdx.x) * nblk + blockIdx.x] = h[threadIdx.x];
+    for (int d = threadIdx.x; d < kRsDigits; d += kT) hist[d] = h[d];
 }
 
+// kRsCols digits per block: their counts over the blocks, hist[block][digit],
+// become exclusive prefixes, and total[digit] their sums.  A thread adds up a
+// digit's counts over a share of the blocks, rows of kRsCols words at a time.
+constexpr int kRsCols = 16, kPrefixT = 1024, kRsShares = kPrefixT / kRsCols;
+
+__global__ __launch_bounds__(kPrefixT) void k_rs_prefix(int *__restrict__ hist, int nblk, int *__restrict__ total) {
+    __shared__ int part[kRsShares][kRsCols];
+    const int col = threadIdx.x % kRsCols, share = threadIdx.x / kRsCols, d = blockIdx.x * kRsCols + col;
+    hist += int64_t(blockIdx.y) * nblk * kRsDigits + d;
+    const int per = (nblk + kRsShares - 1) / kRsShares, lo = min(share * per, nblk), hi = min(lo + per, nblk);
+    int sum = 0;
+#pragma unroll 4
+    for (int b = lo; b < hi; ++b) sum += hist[int64_t(b) * kRsDigits];
+    part[share][col] = sum;
+    __syncthreads();
+    // (every share in the same steps, in place)
+    int at = 0;
+    for (int q = 0; q < kRsShares; ++q) at += q < share ? part[q][col] : 0;
+    if (share == kRsShares - 1) total[blockIdx.y * kRsDigits + d] = at + sum;
+#pragma unroll 8
+    for (int b = lo; b < hi; ++b) {
+        const int v = hist[int64_t(b) * kRsDigits];
+        hist[int64_t(b) * kRsDigits] = at;
+        at += v;
+    }
+}
+
+// Inclusive sum over the block, in thread order.
+__device__ __forceinline__ int block_inclusive(int v, int *wsum) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(v, off, 64);
+        if (lane >= off) v += u;
+    }
+    if (lane == 63) wsum[wave] = v;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) v += wsum[w];
+    return v;
+}
+
+// Stable: a wave's elements are consecutive, its digits are counted in its
+// own counters in order (ranks within 64 from per-digit lane masks built of
+// ballots), and the waves' counts are summed once at the end.
 __global__ __launch_bounds__(kT) void k_rs_scatter(const uint64_t *__restrict__ key, const uint32_t *__restrict__ val,
-                                                  int64_t n, int shift, int nblk, const int *__restrict__ off,
+                                                  int64_t n, int shift, uint32_t mask, int nblk,
+                                                  const int *__restrict__ hist, const int *__restrict__ total,
                                                   uint64_t *__restrict__ okey, uint32_t *__restrict__ oval) {
-    __shared__ int base[256];
-    __shared__ int cnt[kT / 64][256];
+    static_assert(kRsDigits == 2 * kT, "two digits per thread");
+    __shared__ int cnt[kT / 64][kRsDigits];
+    __shared__ int wsum[kT / 64];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    base[t] = off[int64_t(t) * nblk + blockIdx.x];
     const uint64_t below = (1ull << lane) - 1ull;
-    const int64_t b0 = int64_t(blockIdx.x) * kRsTile;
-    for (int j = 0; j < 8; ++j) {
-        for (int w = 0; w < kT / 64; ++w) cnt[w][t] = 0;
-        __syncthreads();
-        const int64_t e = b0 + j * kT + t;
-        const bool ok = e < n;
-        const uint64_t k = ok ? key[e] : 0;
-        const uint32_t v = ok ? val[e] : 0;
-        const int d = int((k >> shift) & 255u);
+    const int64_t e0 = int64_t(blockIdx.x) * kRsTile + wave * (64 * kRsPer) + lane;
+    key += blockIdx.y * n;
+    val += blockIdx.y * n;
+    okey += blockIdx.y * n;
+    oval += blockIdx.y * n;
+    hist += (int64_t(blockIdx.y) * nblk + blockIdx.x) * kRsDigits;
+    total += blockIdx.y * kRsDigits;
+    uint64_t k[kRsPer];
+    uint32_t v[kRsPer];
+#pragma unroll
+    for (int j = 0; j < kRsPer; ++j) {
+        const int64_t e = e0 + j * 64;
+        k[j] = e < n ? key[e] : 0;
+        v[j] = e < n ? val[e] : 0;
+    }
+    // the two digits of this thread: where this block's elements of them go
+    const int d0 = 2 * t, d1 = 2 * t + 1;
+    const int2 tot = *reinterpret_cast<const int2 *>(total + d0), h = *reinterpret_cast<const int2 *>(hist + d0);
+    for (int d = lane; d < kRsDigits; d += 64) cnt[wave][d] = 0;
+    int pos[kRsPer];
+#pragma unroll
+    for (int j = 0; j < kRsPer; ++j) {
+        const bool ok = e0 + j * 64 < n;
+        const uint32_t d = uint32_t(k[j] >> shift) & mask;
         uint64_t same = __ballot(ok);
-        for (int bit = 0; bit < 8; ++bit) {
+#pragma unroll
+        for (int bit = 0; bit < kRsBits; ++bit) {
             const uint64_t bb = __ballot((d >> bit) & 1);
             same &= ((d >> bit) & 1) ? bb : ~bb;
         }
         const int rank = int(__popcll(same & below));
-        if (ok && rank == 0) cnt[wave][d] = int(__popcll(same));
-        __syncthreads();
-        int before = 0;
-        for (int w = 0; w < wave; ++w) before += cnt[w][d];
-        if (ok) {
-            const int pos = base[d] + before + rank;
-            okey[pos] = k;
-            oval[pos] = v;
-        }
-        __syncthreads();
-        int tot = 0;
-        for (int w = 0; w < kT / 64; ++w) tot += cnt[w][t];
-        base[t] += tot;
-        __syncthreads();
+        const int before = cnt[wave][d];
+        if (ok && rank == 0) cnt[wave][d] = before + int(__popcll(same));
+        pos[j] = before + rank;
+        __builtin_amdgcn_wave_barrier();
+    }
+    const int incl = block_inclusive(tot.x + tot.y, wsum);  // (its barrier publishes cnt)
+    int b0 = incl - tot.x - tot.y + h.x, b1 = incl - tot.y + h.y;
+    for (int w = 0; w < kT / 64; ++w) {
+        const int c0 = cnt[w][d0], c1 = cnt[w][d1];
+        cnt[w][d0] = b0;
+        cnt[w][d1] = b1;
+        b0 += c0;
+        b1 += c1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kRsPer; ++j) {
+        if (e0 + j * 64 >= n) continue;
+        const int to = cnt[wave][uint32_t(k[j] >> shift) & mask] + pos[j];
+        okey[to] = k[j];
+        oval[to] = v[j];
     }
 }
 
 struct WarmLayout {
-    size_t stats, x, pred, kk, kv, k2, i2, hist, hoff, sums, offs, row, total;
+    size_t stats, x, pred, kk, kv, k2, i2, hist, sums, row, total;
     int nblk;
 };
 
@@ -209,9 +287,8 @@ WarmLayout warm_layout(int64_t wtot, int32_t nchains, int32_t nkeys) {
     size_t o = 0;
     auto al = [](size_t v) { return (v + 255) & ~size_t(255); };
     const size_t n = size_t(wtot);
-    L.nblk = int((2 * wtot + kRsTile - 1) / kRsTile);
-    const size_t hn = size_t(256) * size_t(std::max(L.nblk, 1));
-    const size_t sb = size_t(scan::blocks(int64_t(hn)));
+    L.nblk = int((wtot + kRsTile - 1) / kRsTile);
+    const size_t hn = 2 * size_t(kRsDigits) * size_t(std::max(L.nblk, 1));
     L.stats = o; o = al(o + sizeof(RowStat) * size_t(nkeys) * size_t(std::max(nchains, 1)));
     L.x = o; o = al(o + n * 8 * 4);
     L.pred = o; o = al(o + n * 2 * 4);
@@ -220,30 +297,29 @@ WarmLayout warm_layout(int64_t wtot, int32_t nchains, int32_t nkeys) {
     L.k2 = o; o = al(o + 2 * n * 8);
     L.i2 = o; o = al(o + 2 * n * 4);
     L.hist = o; o = al(o + hn * 4);
-    L.hoff = o; o = al(o + (hn + 1) * 4);
-    L.sums = o; o = al(o + sb * 4);
-    L.offs = o; o = al(o + (sb + 1) * 4);
+    L.sums = o; o = al(o + 2 * kRsDigits * 4);
     L.row = o; o = al(o + n * 8);
     L.total = o;
     return L;
 }
 
-// Sorts (k, v) by the low `bits` bits of the keys, ping-ponging through
-// (k2, v2); returns the values array that holds the result.
+// Sorts both lists of n in (k, v) by the low `bits` bits of the keys,
+// ping-ponging through (k2, v2); returns the values array that holds the result.
 uint32_t *radix_sort(uint64_t *k, uint32_t *v, uint64_t *k2, uint32_t *v2, int64_t n, int bits, char *base,
                      const WarmLayout &L, hipStream_t s) {
     int *hist = reinterpret_cast<int *>(base + L.hist);
-    int *hoff = reinterpret_cast<int *>(base + L.hoff);
-    int *sums = reinterpret_cast<int *>(base + L.sums);
-    int *offs = reinterpret_cast<int *>(base + L.offs);
-    const int64_t hn = int64_t(256) * L.nblk;
-    for (int shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_rs_hist, dim3(uint32_t(L.nblk)), dim3(kT), 0, s, k, n, shift, L.nblk, hist);
-        scan::exclusive(hist, hn, sums, offs, hoff, s);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(uint32_t(L.nblk)), dim3(kT), 0, s, k, v, n, shift, L.nblk, hoff, k2,
-                           v2);
+    int *total = reinterpret_cast<int *>(base + L.sums);
+    const int passes = (bits + kRsBits - 1) / kRsBits;
+    for (int p = 0, shift = 0; p < passes; ++p) {
+        const int digit = (bits - shift + passes - p - 1) / (passes - p);
+        const uint32_t mask = (1u << digit) - 1u;
+        hipLaunchKernelGGL(k_rs_hist, dim3(uint32_t(L.nblk), 2), dim3(kT), 0, s, k, n, shift, mask, L.nblk, hist);
+        hipLaunchKernelGGL(k_rs_prefix, dim3(kRsDigits / kRsCols, 2), dim3(kPrefixT), 0, s, hist, L.nblk, total);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(uint32_t(L.nblk), 2), dim3(kT), 0, s, k, v, n, shift, mask, L.nblk, hist,
+                           total, k2, v2);
         std::swap(k, k2);
         std::swap(v, v2);
+        shift += digit;
     }
     return v;
 }
@@ -301,19 +377,18 @@ extern "C" int amh_warm_start(void *mlp, const amh_render *R, uint64_t *pts_dev,
     uint64_t *row = reinterpret_cast<uint64_t *>(b + L.row);
     const uint32_t ga = uint32_t((R->wtot + kT - 1) / kT);
     hipLaunchKernelGGL(k_row_stats, dim3(uint32_t(R->nchains), uint32_t(R->nkeys)), dim3(kT), 0, s, *R, st);
-    // key bits: set (1), chain, and y, x at 1/16 px over the frame
+    // key bits: chain, and y, x at 1/16 px over the frame
     int cb = 0, cx = 0;
     while ((1 << cb) < R->nchains) ++cb;
     while ((int64_t(1) << cx) < int64_t(std::max(std::max(R->width, R->height), 1)) * 16) ++cx;
-    const int bits = 1 + cb + 2 * cx;
+    const int bits = cb + 2 * cx;
     for (int y = 0; y + 1 < R->nkeys; ++y) {
         hipLaunchKernelGGL(k_features, dim3(ga), dim3(kT), 0, s, *R, y, st, x, static_cast<float *>(nullptr));
         if (int r = amh_mlp_forward(mlp, x, R->wtot, pred, stream)) return r;
-        hipLaunchKernelGGL(k_match_keys, dim3(ga), dim3(kT), 0, s, *R, y + 1, st, pred, cb, cx, kk, kv);
-        const uint32_t *sorted = radix_sort(kk, kv, k2, i2, 2 * R->wtot, bits, b, L, s);
+        hipLaunchKernelGGL(k_match_keys, dim3(ga), dim3(kT), 0, s, *R, y + 1, st, pred, cx, kk, kv,
+                           row);
+        const uint32_t *sorted = radix_sort(kk, kv, k2, i2, R->wtot, bits, b, L, s);
         uint64_t *dst = pts_dev + int64_t(y + 1) * R->wtot;
-        if (int r = check_hip(hipMemcpyAsync(row, dst, size_t(R->wtot) * 8, hipMemcpyDeviceToDevice, s), "warm"))
-            return r;
         hipLaunchKernelGGL(k_match_apply, dim3(ga), dim3(kT), 0, s, R->wtot, sorted, row, dst);
     }
     AMH_LAUNCH_CHECK("amh_warm_start");
