@@ -126,6 +126,24 @@ def test_fluid_step_of_crowded_cells_matches_oracle(crowd, fill):
         assert d <= tol, (col, d)
 
 
+@pytest.mark.parametrize("n", [1, 63, 65, 32768, 32769, 70000])
+def test_fluid_particles_read_back_as_set(n):
+    """Around the rows of a workgroup and the particles read back at a time."""
+    rng = np.random.default_rng(n)
+    P = rng.uniform(0, 1, (n, 20))
+    P[:, 16:18] = rng.integers(0, 2, (n, 2))
+    lib = G.lib()
+    f = _model(n, 64, 64)
+    try:
+        G.log(f"fluid particles {n}")
+        G.check(lib.amh_fluid_set_particles(f, op.ptr(P), G.stream()), "set")
+        Q = np.full((n, 20), -7.0)
+        G.check(lib.amh_fluid_get_particles(f, op.ptr(Q), G.stream()), "get")
+    finally:
+        lib.amh_fluid_destroy(f)
+    assert (Q[:, :18] == P[:, :18]).all() and (Q[:, 18:] == -7.0).all()
+
+
 def _clustered(rng, n, lo, hi, shift=0.0):
     """Particles in runs of 256 around random centres in [lo, hi)^2 (moved by
     shift cells), with velocities, attractors and colours."""
