@@ -38,11 +38,10 @@ struct Particles {  // structure of arrays, device
     double *x, *y, *u, *v, *gx, *gy, *fr;
     double *R, *G, *B, *A, *r, *g, *b, *a;
     double *strength;
-    double *u2, *v2;  // the velocity between G2P and advection
     int32_t *active, *mature, *owner, *key;  // owner: first at its source
     int32_t *atom;  // in the cell-ordered copy: the particle (atom) in each slot
 };
-constexpr int kParticleDoubles = 18;
+constexpr int kParticleDoubles = 16;
 constexpr int kParticleInts = 5;
 
 // FP32 node fields, [gsx * gsy], node (i, j) at i * gsy + j.  FluidModel's
@@ -168,20 +167,10 @@ __device__ __forceinline__ float basis_gradient(int a, float w0, float w1, float
     return k0 * w0 + k1 * w1 + k2 * w2;
 }
 
-__device__ __forceinline__ float nd(const float *f, int i, int j, int gsx, int gsy) {
-    return node_ok(i, j, gsx, gsy) ? f[int64_t(i) * gsy + j] : 0.0f;
-}
-
 // A node's acceleration and velocity as FluidModel reads them after dividing
 // them by the node mass where it is positive (fluidmodel.cpp:359-364,
 // 437-443); the readers divide, so no pass over the grid is needed.
 __device__ __forceinline__ float per_mass(float v, float m) { return m > 0.0f ? v / m : v; }
-// f[k] / mass of node (i, j); muvw holds the mass of node k at 4k.
-__device__ __forceinline__ float nd_m(const float *f, const float *muvw, int i, int j, int gsx, int gsy) {
-    if (!node_ok(i, j, gsx, gsy)) return 0.0f;
-    const int64_t k = int64_t(i) * gsy + j;
-    return per_mass(f[k], muvw[4 * k]);
-}
 
 // pressure from the bicubic density interpolation, wall forces
 // (fluidmodel.cpp:251-357)
@@ -247,21 +236,20 @@ __device__ __forceinline__ void toward(double x1, double y1, double x2, double y
 // ------------------------------------------------------------------ tiles
 // The grid's nodes are owned by kTile x kTile tiles.  Each step every active
 // particle is binned into each tile that holds a node of its 3x3 stencil (1,
-// 2 or 4 tiles; a counting sort of slot numbers); the entry for the tile of
-// its own cell is marked as its home.  The block of a tile reads its bin,
+// 2 or 4 tiles; a counting sort of slot numbers).  The block of a tile reads
+// its bin,
 // sums what those particles add to its nodes in LDS and stores every node
 // once.  No phase of the step uses a global atomic (device-wide atomics are
 // performed past the per-XCD L2) and no phase needs the grid cleared first.
 constexpr int kTile = 8;
-constexpr int kReach = kTile + 2;       // cells per axis that reach a tile's nodes
-constexpr int kHome = int(0x80000000);  // bin entry flag: the particle's home tile
+constexpr int kReach = kTile + 2;  // cells per axis that reach a tile's nodes
 
 struct Bins {
     int32_t ntx, nty;   // tiles per axis
     int32_t *count[2];  // [tiles] per step parity; the other parity is zero
     int32_t *start;     // [tiles + 1]
     int32_t *rank;      // [4][n]: place of particle i's j-th entry in its bin
-    int32_t *list;      // [<= 4n] slot | kHome, grouped by bin
+    int32_t *list;      // [<= 4n] slots, grouped by bin
     int32_t item;         // entries of a work item at most, one per thread
     // Work items of `item` entries at most, each one workgroup (chunk NULL:
     // whole bins, one workgroup per tile, from start[]).  A dense bin is
@@ -281,7 +269,7 @@ struct Bins {
 constexpr int kLdsTiles = 4096;  // up to this many tiles the placing blocks scan the counts in LDS
 
 // The tiles holding the stencil nodes of a particle at (x, y): tx0..tx1 x
-// ty0..ty1 (nodes clamped to the grid); (tx0, ty0) is its home.
+// ty0..ty1 (nodes clamped to the grid).
 __device__ __forceinline__ void stencil_tiles(double x, double y, int gsx, int gsy, int &tx0, int &tx1, int &ty0,
                                               int &ty1) {
     const int cx = static_cast<int>(x - 0.5), cy = static_cast<int>(y - 0.5);
@@ -299,7 +287,7 @@ __device__ __forceinline__ int entry_tile(int j, int tx0, int tx1, int ty0, int 
 }
 
 // What a particle is binned by: tiles(i, tx0, tx1, ty0, ty1) gives the
-// block tx0..tx1 x ty0..ty1 of tiles it enters ((tx0, ty0) its home) and
+// block tx0..tx1 x ty0..ty1 of tiles it enters and
 // returns false for a particle that is not binned.
 struct StencilTiles {  // the step: tiles holding the 3x3 stencil nodes
     Particles P;
@@ -440,7 +428,7 @@ __global__ __launch_bounds__(kT) void k_bin_place(Tiles tiles_of, int n, Bins B,
     if (binned)
         for (int j = 0; j < 4; ++j) {
             const int t = entry_tile(j, tx0, tx1, ty0, ty1, B.nty);
-            if (t >= 0) B.list[start[t] + rank[j]] = i | (j == 0 ? kHome : 0);
+            if (t >= 0) B.list[start[t] + rank[j]] = i;
         }
     if (i < n) tail(i);
 }
@@ -516,11 +504,11 @@ __global__ __launch_bounds__(kT) void k_item_place(StencilTiles tiles_of, int n,
     if (!binned) return;
     for (int j = 0; j < 4; ++j) {
         const int t = entry_tile(j, tx0, tx1, ty0, ty1, B.nty);
-        if (t >= 0) B.list[int64_t(first[t]) * B.item + rank[j]] = i | (j == 0 ? kHome : 0);
+        if (t >= 0) B.list[int64_t(first[t]) * B.item + rank[j]] = i;
     }
 }
 
-// Calls body(slot, home, item) for the entries [s0, s1) of a whole bin (the
+// Calls body(slot, item) for the entries [s0, s1) of a whole bin (the
 // splat's pixel tiles), kT at a time (slot -1 past the end), item =
 // fetch(slot) holding the particle fields the body reads.  The next kT
 // entries and their fields are loaded before the current ones are
@@ -528,29 +516,21 @@ __global__ __launch_bounds__(kT) void k_item_place(StencilTiles tiles_of, int n,
 // uniform over the block.
 template <class Fetch, class Body>
 __device__ __forceinline__ void for_bin(const Bins &B, int s0, int s1, const Fetch &fetch, const Body &body) {
-    auto entry = [&](int base, int &slot, bool &home) {
+    auto entry = [&](int base, int &slot) {
         const int k = base + int(threadIdx.x);
-        slot = -1;
-        home = false;
-        if (k < s1) {
-            const int e = B.list[k];
-            slot = e & 0x7FFFFFFF;
-            home = e < 0;
-        }
+        slot = k < s1 ? B.list[k] : -1;
     };
     int slot, nslot = -1;
-    bool home, nhome = false;
-    entry(s0, slot, home);
+    entry(s0, slot);
     auto item = fetch(slot);
     for (int base = s0; base < s1; base += kT) {
         auto next = item;
         if (base + kT < s1) {
-            entry(base + kT, nslot, nhome);
+            entry(base + kT, nslot);
             next = fetch(nslot);
         }
-        body(slot, home, item);
+        body(slot, item);
         slot = nslot;
-        home = nhome;
         item = next;
     }
 }
@@ -573,25 +553,23 @@ __device__ __forceinline__ ItemWords load_item(const Bins &B, int b) {
 }
 // Its tile, whether it is the tile's only item (then it stores its nodes;
 // otherwise it adds them atomically), and this thread's entry (slot -1
-// past the item's entries, home: the particle's home tile).
-__device__ __forceinline__ void tile_item(const ItemWords &w, int &t, bool &single, int &slot, bool &home) {
+// past the item's entries).
+__device__ __forceinline__ void tile_item(const ItemWords &w, int &t, bool &single, int &slot) {
     t = w.c.x;
     single = w.c.z != 0;
-    const bool has = int(threadIdx.x) < w.c.y;
-    slot = has ? (w.e & 0x7FFFFFFF) : -1;
-    home = has && w.e < 0;
+    slot = int(threadIdx.x) < w.c.y ? w.e : -1;
 }
 
-// body(slot, home, item) on this thread's entry, item = fetch(slot) holding
+// body(slot, item) on this thread's entry, item = fetch(slot) holding
 // the particle fields the body reads; prologue() runs once those loads are
 // issued and before they are used, so its own memory traffic (a node halo
 // staged in LDS, with the barrier that publishes it) overlaps them.
 template <class Fetch, class Body, class Prologue>
-__device__ __forceinline__ void run_item(int slot, bool home, const Fetch &fetch, const Body &body,
+__device__ __forceinline__ void run_item(int slot, const Fetch &fetch, const Body &body,
                                          const Prologue &prologue) {
     const auto item = fetch(slot);
     prologue();
-    if (__ballot(slot >= 0)) body(slot, home, item);  // a sparse tile leaves whole waves empty
+    if (__ballot(slot >= 0)) body(slot, item);  // a sparse tile leaves whole waves empty
 }
 
 __device__ __forceinline__ void put_node(float *f, int64_t k, float v, bool single) {
@@ -607,7 +585,7 @@ __device__ __forceinline__ bool in_reach(int cx, int cy, int x0, int y0) {
 // x0-2 .. x0+kTile+1 by y0-2 .. y0+kTile+1 cover the stencil of every
 // particle in reach of the tile (origins x0-2 .. x0+kTile-1, 3 nodes) and
 // the bicubic density corners of particle_forces (int(x) <= origin + 1).
-// Nodes outside the grid hold 0, as nd() reads them.
+// Nodes outside the grid hold 0.
 constexpr int kHalo = kTile + 4;
 
 __device__ __forceinline__ int halo_index(int i, int j, int x0, int y0) {
@@ -735,8 +713,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
     if (blockIdx.x == 0 && threadIdx.x == 0) B.nchunks[B.par ^ 1] = 0;
     for (int item = int(blockIdx.x); item < nchunks; item += int(gridDim.x)) {
         int tile, slot0;
-        bool single, home0;
-        tile_item(next, tile, single, slot0, home0);
+        bool single;
+        tile_item(next, tile, single, slot0);
         next = load_item<NT>(B, item + int(gridDim.x));
         const int64_t s0 = int64_t(item) * NT;  // the item's entries in the list
         const int tx = tile / B.nty, ty = tile % B.nty;
@@ -782,12 +760,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
         };
         {
             // at most NT entries: one pass, ranks fit in 8 bits
-            run_item(slot0, home0, fetch, [&](int slot, bool home, const P2gItem &it) {
+            run_item(slot0, fetch, [&](int slot, const P2gItem &it) {
                 const int cx = static_cast<int>(it.x - 0.5), cy = static_cast<int>(it.y - 0.5);
                 const int bucket = in_reach(cx, cy, x0, y0) ? (cx - x0 + 2) * kReach + (cy - y0 + 2) : kCells;
                 if (slot >= 0) {
                     const int l = threadIdx.x;
-                    mine[l] = make_int2(slot | (home ? kHome : 0), (bucket << 8) | atomicAdd(&cellpos[bucket], 1));
+                    mine[l] = make_int2(slot, (bucket << 8) | atomicAdd(&cellpos[bucket], 1));
                     float t[5];
                     tints(it, t);
                     stage.item.x[l] = it.x;
@@ -901,8 +879,8 @@ __global__ __launch_bounds__(NT) void k_forces(Particles P, Grid Gd, int gsx, in
     const int nchunks = B.nchunks[B.par];
     for (int item = int(blockIdx.x); item < nchunks; item += int(gridDim.x)) {
         int tile, slot0;
-        bool single, home0;
-        tile_item(load_item<NT>(B, item), tile, single, slot0, home0);
+        bool single;
+        tile_item(load_item<NT>(B, item), tile, single, slot0);
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
         acc.clear();
@@ -920,7 +898,7 @@ __global__ __launch_bounds__(NT) void k_forces(Particles P, Grid Gd, int gsx, in
             const int q = slot >= 0 ? slot : 0;
             return double2{P.x[q], P.y[q]};
         };
-        run_item(slot0, home0, fetch, [&](int slot, bool, const double2 &it) {
+        run_item(slot0, fetch, [&](int slot, const double2 &it) {
             int cx, cy;
             double px[3], py[3], gx[3], gy[3];
             double pressure = 0.0, fx = 0.0, fy = 0.0;
@@ -956,8 +934,8 @@ struct G2pItem {
     int mature;
 };
 
-// Particle velocity from node accelerations plus the attractor (written by
-// the particle's home tile), then the momentum of the tile's nodes
+// Particle velocity from node accelerations plus the attractor, and from it
+// the momentum of the tile's nodes
 // (fluidmodel.cpp:359-437).
 template <int NT>
 __global__ __launch_bounds__(NT) void k_g2p(Particles P, Grid Gd, int gsx, int gsy, Bins B) {
@@ -966,8 +944,8 @@ __global__ __launch_bounds__(NT) void k_g2p(Particles P, Grid Gd, int gsx, int g
     const int nchunks = B.nchunks[B.par];
     for (int item = int(blockIdx.x); item < nchunks; item += int(gridDim.x)) {
         int tile, slot0;
-        bool single, home0;
-        tile_item(load_item<NT>(B, item), tile, single, slot0, home0);
+        bool single;
+        tile_item(load_item<NT>(B, item), tile, single, slot0);
         const int tx = tile / B.nty, ty = tile % B.nty;
         const int x0 = tx * kTile, y0 = ty * kTile;
         acc.clear();
@@ -983,7 +961,7 @@ __global__ __launch_bounds__(NT) void k_g2p(Particles P, Grid Gd, int gsx, int g
             const int q = slot >= 0 ? slot : 0;
             return G2pItem{P.x[q], P.y[q], P.gx[q], P.gy[q], P.u[q], P.v[q], P.mature[q]};
         };
-        run_item(slot0, home0, fetch, [&](int slot, bool home, const G2pItem &it) {
+        run_item(slot0, fetch, [&](int slot, const G2pItem &it) {
             int cx, cy;
             double px[3], py[3], gx[3], gy[3];
             const double x = it.x, y = it.y;
@@ -998,29 +976,12 @@ __global__ __launch_bounds__(NT) void k_g2p(Particles P, Grid Gd, int gsx, int g
                 nax[k] = accel[0][e + k / 3 * kHalo + k % 3];
                 nay[k] = accel[1][e + k / 3 * kHalo + k % 3];
             }
-            if (home && !valid) {  // a stencil that leaves the grid
-#pragma unroll 1
-                for (int k = 0; k < 9; ++k) {
-                    const float ax = nd_m(Gd.ax, Gd.muvw, cx + k / 3, cy + k % 3, gsx, gsy);
-                    const float ay = nd_m(Gd.ay, Gd.muvw, cx + k / 3, cy + k % 3, gsx, gsy);
-                    for (int q = 0; q < 9; ++q) {  // (no indexed registers)
-                        nax[q] = q == k ? ax : nax[q];
-                        nay[q] = q == k ? ay : nay[q];
-                    }
-                }
-            }
             for (int k = 0; k < 9; ++k) {
                 const double phi = px[k / 3] * py[k % 3];
                 u += phi * (nax[k] + cax);
                 v += phi * (nay[k] + cay);
             }
-            if (home) {  // other tiles still read the old velocity
-                P.u2[slot] = u;
-                P.v2[slot] = v;
-            }
-            const bool act = valid || home;
-            const double mu = act ? (it.mature ? u : u * 0.0) : 0.0;
-            const double mv = act ? (it.mature ? v : v * 0.0) : 0.0;
+            const double mu = it.mature ? u : u * 0.0, mv = it.mature ? v : v * 0.0;
             float p[18];
             for (int k = 0; k < 9; ++k) {
                 const double phi = px[k / 3] * py[k % 3];
@@ -1166,7 +1127,7 @@ __device__ __forceinline__ double2 advect_one(Particles P, int i, const Grid &Gd
     const int mature = P.mature[i];
     const double R0 = P.R[i], G0 = P.G[i], B0 = P.B[i], A0 = P.A[i];
     const double r0 = P.r[i], g0 = P.g[i], b0 = P.b[i], a0 = P.a[i];
-    const double tgx = P.gx[i], tgy = P.gy[i], fr = P.fr[i], u2 = P.u2[i], v2 = P.v2[i];
+    const double tgx = P.gx[i], tgy = P.gy[i], fr = P.fr[i];
     if (out) {
         out->s = P.strength[i];
         out->R = R0; out->G = G0; out->B = B0; out->A = A0;
@@ -1228,9 +1189,9 @@ __device__ __forceinline__ double2 advect_one(Particles P, int i, const Grid &Gd
             y += my * w;
         }
     }
-    double u = u2, v = v2;
-    u += gu - u;
-    v += gv - v;
+    // u += gu - u: the velocity becomes the grid's, so
+    // what G2P made of the old one need not be stored for here
+    double u = gu, v = gv;
     if (x < 1.0) { x = 1.0 + jitter(seed, id, 0); u = 0.0; }
     else if (x > gsx - 2) { x = gsx - 2 - jitter(seed, id, 1); u = 0.0; }
     if (y < 1.0) { y = 1.0 + jitter(seed, id, 2); v = 0.0; }
@@ -1488,7 +1449,7 @@ size_t fluid_bytes(int gsx, int gsy, int count, int W, int H, int nkeys) {
 
 void carve_particles(Particles &Q, size_t n, const std::function<char *(size_t)> &take) {
     double **d[kParticleDoubles] = {&Q.x, &Q.y, &Q.u, &Q.v, &Q.gx, &Q.gy, &Q.fr, &Q.R, &Q.G,
-                                    &Q.B, &Q.A, &Q.r, &Q.g, &Q.b, &Q.a, &Q.strength, &Q.u2, &Q.v2};
+                                    &Q.B, &Q.A, &Q.r, &Q.g, &Q.b, &Q.a, &Q.strength};
     for (double **q : d) *q = reinterpret_cast<double *>(take(n * 8));
     int32_t **ints[kParticleInts] = {&Q.active, &Q.mature, &Q.owner, &Q.key, &Q.atom};
     for (int32_t **q : ints) *q = reinterpret_cast<int32_t *>(take(n * 4));
@@ -2045,7 +2006,7 @@ __global__ __launch_bounds__(kT) void k_splat_tile(Bins B, const uint32_t *__res
         }
         return it;
     };
-    for_bin(B, B.start[blockIdx.x], B.start[blockIdx.x + 1], fetch, [&](int slot, bool, const SplatItem &it) {
+    for_bin(B, B.start[blockIdx.x], B.start[blockIdx.x + 1], fetch, [&](int slot, const SplatItem &it) {
         if (slot < 0 || it.xy == kNoTap) return;
         const int X = int(it.xy & 0xFFFFu), Y = int(it.xy >> 16);
         for (int q = 0; q < 4; ++q) {
