@@ -44,6 +44,7 @@ constexpr int kTile = 16;             // pixels per side of an image tile
 constexpr int kTilePx = kTile * kTile;  // one thread of the splat per pixel
 static_assert(kTilePx == kT, "one thread per pixel");
 constexpr int kLdsTiles = 4096;       // up to this many tiles every placing block scans the counts in LDS
+constexpr int kFewTiles = 4096;       // up to this many tiles blocks count atoms per tile in LDS
 constexpr int kNoBlob = 0x7FFFFFFF;
 
 // --------------------------------------------------------------- prepare
@@ -75,11 +76,17 @@ __device__ __forceinline__ int tile_of(uint32_t x, uint32_t y, int j, int ntx) {
 
 // What bounds it: the instructions of the PERLIN fade's 16 noise octaves per
 // atom (1.7 M atoms: 246 us with one noise at a time and selects for the
-// gradients, 108 us with both together from tables).  The taps are counted per tile with the wave's lanes grouped
-// by tile first, one atomic per distinct tile: neighbouring atoms of a chain
-// fall in few tiles.
+// gradients, 108 us with both together from tables).  The taps are counted per
+// tile.  kFew (up to kFewTiles tiles): in LDS, then one atomic per tile and
+// block: on few tiles scattered atoms would queue at the same counters.
+// Otherwise with the wave's lanes grouped by tile first, one atomic per
+// distinct tile: neighbouring atoms of a chain fall in few tiles, and the
+// counters are many.  (11,000 atoms on 70 tiles: 17.8 us
+// grouped, 4.9 in LDS; 300,000 refined ones on 3,087: 21.7 and 10.0.)
+template <bool kFew>
 __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B) {
     __shared__ PerlinTab tab;
+    __shared__ int cnt[kFew ? kFewTiles : 1];
     const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
     const bool in = a < R.wtot;
     // the points first: their loads overlap the tables' and the chain search
@@ -89,6 +96,9 @@ __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__re
     uint64_t tk[4] = {p1, p1, p2, p2};
     traj_keys(R, F, al, tk);
     if (R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
+    const int tiles = B.ntx * B.nty;
+    if (kFew)
+        for (int k = threadIdx.x; k < tiles; k += kT) cnt[k] = 0;
     __syncthreads();
     const int c = block_chain(R.chain_off_dev, R.nchains, a);
     uint32_t mask = 0, X = 0, Y = 0;
@@ -120,6 +130,16 @@ __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__re
         }
         recs[a] = rec;
     }
+    if (kFew) {
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t m = taps_in(mask, X, Y, j);
+            if (m) atomicAdd(&cnt[tile_of(X, Y, j, B.ntx)], int(__popc(m)));
+        }
+        __syncthreads();
+        for (int k = threadIdx.x; k < tiles; k += kT)
+            if (cnt[k]) atomicAdd(&B.taps[k], cnt[k]);
+        return;
+    }
     const int lane = threadIdx.x & 63;
     for (int j = 0; j < 4; ++j) {
         const uint32_t m = taps_in(mask, X, Y, j);
@@ -141,7 +161,8 @@ __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__re
 // The atoms' numbers into their tiles' lists, in no fixed order (the sums are
 // exact).  kLds: every block scans the tap counts in LDS (block 0 stores the
 // starts); otherwise B.start holds the scan already.
-template <bool kLds>
+// kFew: ranks within the block from LDS counters, as in k_prepare.
+template <bool kLds, bool kFew>
 __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int64_t n, Tiles B) {
     __shared__ int sstart[kLds ? kLdsTiles + 1 : 1];
     __shared__ int wsum[kT / 64];
@@ -155,6 +176,24 @@ __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int6
         if (blockIdx.x == 0)
             for (int k = threadIdx.x; k <= tiles; k += kT) B.start[k] = sstart[k];
         start = sstart;
+    }
+    if (kFew) {
+        __shared__ int cnt[kFew ? kFewTiles : 1];
+        const int tiles = B.ntx * B.nty;
+        for (int k = threadIdx.x; k < tiles; k += kT) cnt[k] = 0;
+        __syncthreads();
+        int t[4], rank[4];
+        for (int j = 0; j < 4; ++j) {
+            t[j] = taps_in(mask, X, Y, j) ? tile_of(X, Y, j, B.ntx) : -1;
+            rank[j] = t[j] >= 0 ? atomicAdd(&cnt[t[j]], 1) : 0;
+        }
+        __syncthreads();
+        for (int k = threadIdx.x; k < tiles; k += kT)
+            if (cnt[k]) cnt[k] = start[k] + atomicAdd(&B.entries[k], cnt[k]);
+        __syncthreads();
+        for (int j = 0; j < 4; ++j)
+            if (t[j] >= 0) B.list[cnt[t[j]] + rank[j]] = uint32_t(a);
+        return;
     }
     const int lane = threadIdx.x & 63;
     const uint64_t below = (1ull << lane) - 1ull;
@@ -751,13 +790,14 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
         amh::launch_timed(name, kernel, dim3(uint32_t((threads + kT - 1) / kT)), dim3(kT), 0, s, args...);
     };
     if (Rc.wtot > 0) {
-        launch("k_prepare", k_prepare, Rc.wtot, Rc, F, recs, B);
+        const bool few = L.tiles <= kFewTiles;
+        launch("k_prepare", few ? k_prepare<true> : k_prepare<false>, Rc.wtot, Rc, F, recs, B);
         if (L.tiles <= kLdsTiles) {
-            launch("k_place", k_place<true>, Rc.wtot, recs, Rc.wtot, B);
+            launch("k_place", few ? k_place<true, true> : k_place<true, false>, Rc.wtot, recs, Rc.wtot, B);
         } else {
             scan::exclusive(B.taps, L.tiles, reinterpret_cast<int *>(base + L.sums),
                             reinterpret_cast<int *>(base + L.offs), B.start, s);
-            launch("k_place", k_place<false>, Rc.wtot, recs, Rc.wtot, B);
+            launch("k_place", k_place<false, false>, Rc.wtot, recs, Rc.wtot, B);
         }
     }
     const bool texture = Rc.show_blobs != 1 && Rc.show_blobs != 2;
