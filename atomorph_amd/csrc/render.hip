@@ -44,7 +44,8 @@ constexpr int kTile = 16;             // pixels per side of an image tile
 constexpr int kTilePx = kTile * kTile;  // one thread of the splat per pixel
 static_assert(kTilePx == kT, "one thread per pixel");
 constexpr int kLdsTiles = 4096;       // up to this many tiles every placing block scans the counts in LDS
-constexpr int kFewTiles = 4096;       // up to this many tiles blocks count atoms per tile in LDS
+constexpr int kFewTiles = 4096;       // up to this many tiles blocks count and place atoms per tile in LDS
+constexpr int kManyTiles = 16384;     // up to this many, larger blocks count them there
 constexpr int kNoBlob = 0x7FFFFFFF;
 
 // --------------------------------------------------------------- prepare
@@ -76,18 +77,20 @@ __device__ __forceinline__ int tile_of(uint32_t x, uint32_t y, int j, int ntx) {
 
 // What bounds it: the instructions of the PERLIN fade's 16 noise octaves per
 // atom (1.7 M atoms: 246 us with one noise at a time and selects for the
-// gradients, 108 us with both together from tables).  The taps are counted per
-// tile.  kFew (up to kFewTiles tiles): in LDS, then one atomic per tile and
-// block: on few tiles scattered atoms would queue at the same counters.
-// Otherwise with the wave's lanes grouped by tile first, one atomic per
-// distinct tile: neighbouring atoms of a chain fall in few tiles, and the
-// counters are many.  (11,000 atoms on 70 tiles: 17.8 us
-// grouped, 4.9 in LDS; 300,000 refined ones on 3,087: 21.7 and 10.0.)
-template <bool kFew>
-__global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B) {
+// gradients, 90 us with both together from tables).  The taps are counted per
+// tile in the block's LDS, TILES counters of 16 bits, then one atomic per
+// tile and block: refined chains scatter, so that grouping a wave's lanes by
+// tile (TILES = 0, one atomic per distinct tile) takes up to 64 turns, and on
+// few tiles the atomics queue at the same counters.  11,000 atoms on 70
+// tiles: 17.8 us grouped, 4.9 in LDS; 300,000 on 3,087: 21.7 and 10; 1.7 M on
+// 16,384: 110 and 90, in blocks of 1,024 that share the 32 KB.  Beyond that
+// too few blocks fit a CU.
+template <int NT, int TILES>
+__global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B) {
     __shared__ PerlinTab tab;
-    __shared__ int cnt[kFew ? kFewTiles : 1];
-    const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
+    __shared__ uint4 counters[TILES ? TILES / 8 : 1];  // 16 bits per tile
+    static_assert(4 * NT < 1 << 16, "a block's taps fit 16 bits");
+    const int64_t a = int64_t(blockIdx.x) * NT + threadIdx.x;
     const bool in = a < R.wtot;
     // the points first: their loads overlap the tables' and the chain search
     const int64_t al = in ? a : 0;
@@ -95,10 +98,10 @@ __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__re
     const uint64_t p2 = R.pts_dev[int64_t(F.fnext) * R.wtot + al];
     uint64_t tk[4] = {p1, p1, p2, p2};
     traj_keys(R, F, al, tk);
-    if (R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, kT);
+    if (R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, threadIdx.x, NT);
     const int tiles = B.ntx * B.nty;
-    if (kFew)
-        for (int k = threadIdx.x; k < tiles; k += kT) cnt[k] = 0;
+    if (TILES)
+        for (int k = threadIdx.x; k < (tiles + 7) / 8; k += NT) counters[k] = uint4{0u, 0u, 0u, 0u};
     __syncthreads();
     const int c = block_chain(R.chain_off_dev, R.nchains, a);
     uint32_t mask = 0, X = 0, Y = 0;
@@ -130,14 +133,24 @@ __global__ __launch_bounds__(kT) void k_prepare(amh_render R, Frame F, Rec *__re
         }
         recs[a] = rec;
     }
-    if (kFew) {
+    if (TILES) {
+        uint32_t *cnt = reinterpret_cast<uint32_t *>(counters);
         for (int j = 0; j < 4; ++j) {
             const uint32_t m = taps_in(mask, X, Y, j);
-            if (m) atomicAdd(&cnt[tile_of(X, Y, j, B.ntx)], int(__popc(m)));
+            if (!m) continue;
+            const int t = tile_of(X, Y, j, B.ntx);
+            atomicAdd(&cnt[t / 2], uint32_t(__popc(m)) << (t % 2 * 16));
         }
         __syncthreads();
-        for (int k = threadIdx.x; k < tiles; k += kT)
-            if (cnt[k]) atomicAdd(&B.taps[k], cnt[k]);
+        for (int k = threadIdx.x; k < (tiles + 7) / 8; k += NT) {
+            const uint4 c = counters[k];
+            if ((c.x | c.y | c.z | c.w) == 0) continue;
+            const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+            for (int q = 0; q < 8; ++q) {
+                const int n = int(w[q / 2] >> (q % 2 * 16) & 0xFFFFu);
+                if (n) atomicAdd(&B.taps[8 * k + q], n);
+            }
+        }
         return;
     }
     const int lane = threadIdx.x & 63;
@@ -786,12 +799,16 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
     F.fnext = (F.fk + 1) % R->nkeys;
     const double dt = 1.0 / double(R->nkeys);
     F.tl = fmax(0.0, (F.tn - (double(F.fk) * dt)) / dt);
-    const auto launch = [&](const char *name, auto kernel, int64_t threads, auto... args) {
+    const auto launch = [&](const char *name, auto kernel, int64_t threads, auto... args) {  // workgroups of kT
         amh::launch_timed(name, kernel, dim3(uint32_t((threads + kT - 1) / kT)), dim3(kT), 0, s, args...);
     };
     if (Rc.wtot > 0) {
         const bool few = L.tiles <= kFewTiles;
-        launch("k_prepare", few ? k_prepare<true> : k_prepare<false>, Rc.wtot, Rc, F, recs, B);
+        if (few) launch("k_prepare", k_prepare<kT, kFewTiles>, Rc.wtot, Rc, F, recs, B);
+        else if (L.tiles <= kManyTiles)
+            amh::launch_timed("k_prepare", k_prepare<1024, kManyTiles>, dim3(uint32_t((Rc.wtot + 1023) / 1024)),
+                              dim3(1024), 0, s, Rc, F, recs, B);
+        else launch("k_prepare", k_prepare<kT, 0>, Rc.wtot, Rc, F, recs, B);
         if (L.tiles <= kLdsTiles) {
             launch("k_place", few ? k_place<true, true> : k_place<true, false>, Rc.wtot, recs, Rc.wtot, B);
         } else {

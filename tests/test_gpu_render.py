@@ -199,3 +199,29 @@ def test_render_tiles_of_overlapping_blobs(W, H, nchains, width, spread, feather
                                     op.ptr(order), nchains, None, t, op.ptr(want))
         assert int(np.abs(got.astype(np.int32) - want.astype(np.int32)).max()) <= 1, t
         assert (rend.frame(t) == got).all()
+
+
+@pytest.mark.parametrize("W,H", [(1024, 1024), (1040, 1024), (2048, 2048), (2064, 2048)])
+def test_render_scattered_atoms_on_many_tiles(W, H):
+    """Atoms anywhere in frames of 4,096, 4,160, 16,384 and 16,512 image tiles:
+    each way of counting and placing atoms per tile, within 1 LSB of the
+    oracle's frame."""
+    rng = np.random.default_rng(W + H)
+    widths = np.array([700, 3000, 1], np.int64)
+    wtot, h = int(widths.sum()), 2
+    off = np.concatenate([[0], np.cumsum(widths)[:-1]]).astype(np.int64)
+    x, y = rng.integers(0, W, (wtot, h)), rng.integers(0, H, (wtot, h))
+    pts = op.pack_points(x, y, rng.integers(0, 256, (wtot, h)), rng.integers(0, 256, (wtot, h)), 3).ravel()
+    keys = rng.integers(0, 256, (h, H, W, 4)).astype(np.uint8)
+    order = np.stack([rng.permutation(3) for _ in range(h)]).astype(np.int32)
+    lag, slope = op.perlin_perm(3), op.perlin_perm(4)
+    vals = {"bbox": [0, 0, W - 1, H - 1], "motion": 3, "fading": 6, "show": 0, "density": 1, "feather": 0, "keep_bg": 0}
+    rend = GpuRenderer(keys, pts, off, widths, order, np.zeros((h, 3), np.uint32), vals, lag, slope)
+    cfg = op.RenderCfg(W, H, h, 0, 0, W - 1, H - 1, 3, 6, 0, 1, 0, 0, 0, 0, op.ptr(lag), op.ptr(slope))
+    want = np.zeros((H, W, 4), np.uint8)
+    G.log(f"render {W}x{H}, scattered atoms")
+    got = rend.frame(0.21)
+    op.oracle().or_render_atoms(C.byref(cfg), op.ptr(keys), op.ptr(pts), op.ptr(off), op.ptr(widths), 3, op.ptr(order),
+                                3, None, 0.21, op.ptr(want))
+    assert int(np.abs(got.astype(np.int32) - want.astype(np.int32)).max()) <= 1
+    assert (rend.frame(0.21) == got).all()
