@@ -467,8 +467,8 @@ def main():
     #                  write, per grid node N the FP32 fields:
     #                  k_p2g    A (7x8 + 4 + 4) read, N 8x4 written
     #                  k_forces A (2x8 + 4) read, N 3x4 read + 2x4 written
-    #                  k_g2p    A (6x8 + 4 + 4) read + 2x8 written, N 3x4 + 2x4
-    #                  k_advect A (15x8 + 2x4) read + 8x8 written, N 8x4 read
+    #                  k_g2p    A (6x8 + 4 + 4) read, N 3x4 + 2x4
+    #                  k_advect A (13x8 + 2x4) read + 8x8 written, N 8x4 read
     per_attempt = 8 * 2 * (2 + (1 if h > 2 else 0))
     refine_bytes = attempts_job * per_attempt + accepted_job * 16
     rooflines = {}
@@ -482,8 +482,8 @@ def main():
         P = m.fluid_particles()
         A = int((P[:, 16] > 0).sum()) if P.size else 0
         N = (int(W * args.fluid_sparseness) + 20) * (int(H * args.fluid_sparseness) + 20)
-        per = {"k_p2g": A * 64 + N * 32, "k_forces": A * 20 + N * 20, "k_g2p": A * 72 + N * 20,
-               "k_advect": A * 192 + N * 32}
+        per = {"k_p2g": A * 64 + N * 32, "k_forces": A * 20 + N * 20, "k_g2p": A * 56 + N * 20,
+               "k_advect": A * 176 + N * 32}
         for k, b in per.items():
             if k in kernels:
                 rooflines[k] = (b, kernels[k]["avg_us"] / 1e6, kernels[k]["launches"])
