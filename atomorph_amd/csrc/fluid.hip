@@ -140,31 +140,32 @@ __device__ __forceinline__ void seg_sums(float (&c)[N], const Seg &s) {
 
 // ------------------------------------------------------------ P2G
 // Mass (= density), density gradient and strength-weighted colour
-// (fluidmodel.cpp:191-249).  A particle at e = x - cx - 1 in [-0.5, 0.5) of
-// its cell has the quadratic B-spline weights
-//   w[0] = (0.5 - e)^2 / 2,  w[1] = 0.75 - e^2,  w[2] = (0.5 + e)^2 / 2
-// (h likewise in y), whose gradients are combinations of them: with
-// 1 = w[0] + w[1] + w[2] and e = w[2] - w[0], gx[a] = sum_p kG[a][p] w[p].  So
-// the node sums of px[a] py[b], gx[a] py[b] and px[a] gy[b] over the
-// particles of one cell follow from the cell's nine sums of w[p](e) w[q](h).
-// A particle therefore adds 9 products and 5 colour sums to its one cell
-// instead of 8 values to each of 9 nodes; the nodes are assembled from the
-// 3x3 cells around them.  The products, and so the masses that the later
-// phases divide by, keep their precision however small they are (sums of the
-// powers of e and h lose it where a weight nearly vanishes).
-constexpr int kCellSums = 14;  // 9 products (p-major), then s*r, s*g, s*b, s*a, s
+// (fluidmodel.cpp:191-249).  With e = x - cx - 1 in [-0.5, 0.5) the
+// quadratic B-spline weights and their gradients are polynomials in e:
+//   px[a] = sum_p kW[a][p] e^p,   gx[a] = sum_p kD[a][p] e^p,
+// so the node sums of px[a] py[b], gx[a] py[b] and px[a] gy[b] over the
+// particles of one cell follow from the cell's nine moments
+// M[p][q] = sum e^p h^q (h likewise in y).  A particle therefore adds 9
+// moments and 5 colour sums to its one cell instead of 8 values to each of 9
+// nodes; the nodes are assembled from the 3x3 cells around them.  At a node
+// where all weights nearly vanish the mass is then FP32 rounding of the
+// moments (about 1e-8), and may be negative; per_mass reads it as it is.
+__constant__ float kW[3][3] = {{0.125f, -0.5f, 0.5f}, {0.75f, 0.0f, -1.0f}, {0.125f, 0.5f, 0.5f}};
+__constant__ float kD[3][3] = {{0.5f, -1.0f, 0.0f}, {0.0f, 2.0f, 0.0f}, {-0.5f, -1.0f, 0.0f}};
+constexpr int kCellSums = 14;  // 9 moments (p-major), then s*r, s*g, s*b, s*a, s
 
-__device__ __forceinline__ void basis(double e, double (&w)[3]) {
-    w[0] = 0.5 * (0.5 - e) * (0.5 - e);
-    w[1] = 0.75 - e * e;
-    w[2] = 0.5 * (0.5 + e) * (0.5 + e);
-}
-// The gradient of weight a from the sums w[] of the three weights.
-__device__ __forceinline__ float basis_gradient(int a, float w0, float w1, float w2) {
-    const float k0 = a == 0 ? 1.5f : a == 1 ? -2.0f : 0.5f;
-    const float k1 = a == 0 ? 0.5f : a == 1 ? 0.0f : -0.5f;
-    const float k2 = a == 0 ? -0.5f : a == 1 ? 2.0f : -1.5f;
-    return k0 * w0 + k1 * w1 + k2 * w2;
+// The 8 node values (m, gx, gy, r, g, b, a, w) that the sums c[] of cell
+// (node - (a, b)) contribute to the node.
+__device__ __forceinline__ void cell_to_node(const float *c, int a, int b, float *v) {
+    float xw[3], xd[3];  // sum_p kW[a][p] M[p][q], sum_p kD[a][p] M[p][q]
+    for (int q = 0; q < 3; ++q) {
+        xw[q] = kW[a][0] * c[q] + kW[a][1] * c[3 + q] + kW[a][2] * c[6 + q];
+        xd[q] = kD[a][0] * c[q] + kD[a][1] * c[3 + q] + kD[a][2] * c[6 + q];
+    }
+    v[0] = kW[b][0] * xw[0] + kW[b][1] * xw[1] + kW[b][2] * xw[2];
+    v[1] = kW[b][0] * xd[0] + kW[b][1] * xd[1] + kW[b][2] * xd[2];
+    v[2] = kD[b][0] * xw[0] + kD[b][1] * xw[1] + kD[b][2] * xw[2];
+    for (int k = 0; k < 5; ++k) v[3 + k] = c[9 + k];
 }
 
 // A node's acceleration and velocity as FluidModel reads them after dividing
@@ -665,7 +666,7 @@ struct P2gItem {
 };
 
 // Mass (= density), density gradient and strength-weighted colour of the
-// tile's nodes from the sums of the cells that reach them.
+// tile's nodes from the moments of the cells that reach them.
 //
 // The block first counting-sorts its chunk by cell (the kReach x
 // kReach cells in reach, then the entries out of reach) through LDS, sums
@@ -743,18 +744,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
             t[3] = tint ? float(it.s * it.a) : 0.0f;
             t[4] = tint ? float(it.s) : 0.0f;
         };
-        // The products of one particle at (x, y) and its colour terms t (valid:
+        // The moments of one particle at (x, y) and its colour terms t (valid:
         // in reach of the tile) into its cell's LDS sums; every lane of
         // the wave calls it.  Branch-free: selects instead of conditional
         // blocks, so no load is deferred into a branch.
         const auto sum_cells = [&](bool valid, double x, double y, const float (&t)[5]) {
             const int cx = static_cast<int>(x - 0.5), cy = static_cast<int>(y - 0.5);
             float c[kCellSums];
-            double ex[3], hy[3];
-            basis(x - cx - 1.0, ex);
-            basis(y - cy - 1.0, hy);
+            const double e = x - cx - 1.0, h = y - cy - 1.0;
+            const double ep[3] = {1.0, e, e * e}, hp[3] = {1.0, h, h * h};
             for (int p = 0; p < 3; ++p)
-                for (int q = 0; q < 3; ++q) c[p * 3 + q] = valid ? float(ex[p] * hy[q]) : 0.0f;
+                for (int q = 0; q < 3; ++q) c[p * 3 + q] = valid ? float(ep[p] * hp[q]) : 0.0f;
             for (int k = 0; k < 5; ++k) c[9 + k] = valid ? t[k] : 0.0f;
             sums.put(c, valid, cx, cy, x0, y0);
         };
@@ -822,11 +822,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_
                     // an empty cell's sums are zero and add nothing; no branch on
                     // it, so the three cells' LDS loads are in flight together
                     const int cell = (ni - a + 2) * kReach + (nj - b + 2);
-                    const float r0 = cs[a * 3][cell], r1 = cs[a * 3 + 1][cell], r2 = cs[a * 3 + 2][cell];
-                    acc[0] += b == 0 ? r0 : b == 1 ? r1 : r2;
-                    acc[1] += basis_gradient(a, cs[b][cell], cs[3 + b][cell], cs[6 + b][cell]);
-                    acc[2] += basis_gradient(b, r0, r1, r2);
-                    for (int k = 0; k < 5; ++k) acc[3 + k] += cs[9 + k][cell];
+                    float m[kCellSums], v[8];
+                    for (int k = 0; k < kCellSums; ++k) m[k] = cs[k][cell];
+                    cell_to_node(m, a, b, v);
+                    for (int f = 0; f < 8; ++f) acc[f] += v[f];
                 }
                 for (int f = 0; f < 8; ++f) part[a][f][node] = acc[f];
             }

@@ -126,6 +126,108 @@ def test_fluid_step_of_crowded_cells_matches_oracle(crowd, fill):
         assert d <= tol, (col, d)
 
 
+def _lone_particle_step(P):
+    """One model step of particles whose stencils meet no other's, away from
+    the walls and within their freedom radius, in the engine's arithmetic: FP32
+    node fields from the FP32 moments e^p h^q of each particle's cell, all else
+    FP64 in the oracle's order.  Returns x, y, u, v."""
+    f32 = np.float32
+    kW = np.array([[0.125, -0.5, 0.5], [0.75, 0, -1], [0.125, 0.5, 0.5]], f32)
+    kD = np.array([[0.5, -1, 0], [0, 2, 0], [-0.5, -1, 0]], f32)
+    x, y, gravity = P[:, 0], P[:, 1], P[:, 4:6]
+    cell = [(c - 0.5).astype(int) for c in (x, y)]
+    e, h = x - cell[0] - 1.0, y - cell[1] - 1.0
+    M = [[(a * b).astype(f32) for b in (np.ones_like(h), h, h * h)] for a in (np.ones_like(e), e, e * e)]
+
+    def along(k, v):  # sum_p k[p] v[p]
+        return (k[0] * v[0] + k[1] * v[1]) + k[2] * v[2]
+
+    m, mx, my = (np.zeros((3, 3, len(P)), f32) for _ in range(3))
+    for a in range(3):
+        xw = [along(kW[a], [M[p][q] for p in range(3)]) for q in range(3)]
+        xd = [along(kD[a], [M[p][q] for p in range(3)]) for q in range(3)]
+        for b in range(3):
+            m[a, b], mx[a, b], my[a, b] = along(kW[b], xw), along(kW[b], xd), along(kD[b], xw)
+
+    def weights(c, v):
+        t = c - v
+        w = [0.5 * t * t + 1.5 * t + 1.125]
+        d = [t + 1.5]
+        t = t + 1.0
+        w.append(-t * t + 0.75)
+        d.append(-2.0 * t)
+        t = t + 1.0
+        return w + [0.5 * t * t - 1.5 * t + 1.125], d + [t - 1.5]
+
+    (px, gx), (py, gy) = weights(cell[0], x), weights(cell[1], y)
+    ix, iy, n = x.astype(int), y.astype(int), np.arange(len(P))
+
+    def node(f, i, j):
+        return f[ix + i - cell[0], iy + j - cell[1], n].astype(float)
+
+    d01, d02, d11, d12 = (node(m, i, j) for i in (0, 1) for j in (0, 1))
+    x01, x02, x11, x12 = (node(mx, i, j) for i in (0, 1) for j in (0, 1))
+    y01, y02, y11, y12 = (node(my, i, j) for i in (0, 1) for j in (0, 1))
+    pdx, pdy = d11 - d01, d02 - d01
+    C20, C02 = 3.0 * pdx - x11 - 2.0 * x01, 3.0 * pdy - y02 - 2.0 * y01
+    C30, C03 = -2.0 * pdx + x11 + x01, -2.0 * pdy + y02 + y01
+    s1, s2 = d01 + y01 + C02 + C03, d01 + x01 + C20 + C30
+    C21, C31 = 3.0 * d12 - 2.0 * x02 - x12 - 3.0 * s1 - C20, -2.0 * d12 + x02 + x12 + 2.0 * s1 - C30
+    C12, C13 = 3.0 * d12 - 2.0 * y11 - y12 - 3.0 * s2 - C02, -2.0 * d12 + y11 + y12 + 2.0 * s2 - C03
+    C11 = x02 - C13 - C12 - x01
+    u, v = x - ix, y - iy
+    u2, v2 = u * u, v * v
+    density = (d01 + x01 * u + y01 * v + C20 * u2 + C02 * v2 + C30 * (u * u2) + C03 * (v * v2) + C21 * u2 * v +
+               C31 * (u * u2) * v + C12 * u * v2 + C13 * u * (v * v2) + C11 * u * v)
+    pressure = np.minimum(density - 1.0, 2.0)
+
+    def per_mass(f, a, b):
+        return np.where(m[a, b] > 0, f / np.where(m[a, b] > 0, m[a, b], f32(1)), f).astype(float)
+
+    A, B = np.abs(y - gravity[:, 1]), np.abs(x - gravity[:, 0])
+    C_ = np.sqrt(A * A + B * B)
+    dx = np.minimum(0.03, C_) * B / C_
+    dy = A * dx / B
+    cax, cay = np.where(x <= gravity[:, 0], dx, -dx), np.where(y <= gravity[:, 1], dy, -dy)
+    U, V = P[:, 2].copy(), P[:, 3].copy()
+    stencil = [(a, b, px[a] * py[b]) for a in range(3) for b in range(3)]
+    for a, b, phi in stencil:
+        U += phi * (per_mass((-((gx[a] * py[b]) * pressure)).astype(f32), a, b) + cax)
+        V += phi * (per_mass((-((px[a] * gy[b]) * pressure)).astype(f32), a, b) + cay)
+    gu, gv = np.zeros_like(U), np.zeros_like(V)
+    for a, b, phi in stencil:
+        gu += phi * per_mass((phi * U).astype(f32), a, b)
+        gv += phi * per_mass((phi * V).astype(f32), a, b)
+    return np.stack([x + gu, y + gv, gu, gv], 1)
+
+
+@pytest.mark.parametrize("spacing", [5, 8, 11])
+def test_fluid_step_where_weights_vanish(spacing):
+    """Particles near a cell's edge, whose weight at the far nodes is 1e-3 to
+    1e-13: the node masses there are the FP32 rounding of the cell's moments,
+    to the bit, and the velocities divided by them are reproduced.  1e-10 is
+    what one FP32 rounding of a node's sums may move a particle (2^-24 of
+    velocities of at most 1e-3 from such nodes); masses from the weights'
+    products would move most of them by 1e-6 to 1e-4."""
+    rng = np.random.default_rng(spacing)
+    gsx = gsy = 200
+    at = np.arange(10, gsx - 10, spacing)
+    cells = np.stack(np.meshgrid(at, at), -1).reshape(-1, 2)
+    n = len(cells)
+    P = np.zeros((n, 20))
+    near = 10.0 ** rng.uniform(-6, -1, (n, 2))  # distance of e and h from -0.5 or 0.5
+    P[:, 0:2] = cells + 0.5 + np.where(rng.integers(0, 2, (n, 2)), near, 1.0 - near)
+    P[:, 2:4] = rng.normal(0, 0.2, (n, 2))
+    P[:, 4:6] = P[:, 0:2] + rng.uniform(0.5, 3, (n, 2))
+    P[:, 6] = 1.0
+    P[:, 7:15] = rng.uniform(0, 1, (n, 8))
+    P[:, 15:18] = 1.0
+    want = _lone_particle_step(P)
+    G.log(f"fluid step, {n} lone particles {spacing} cells apart")
+    got = _step_gpu(P, gsx, gsy, 1, 20.0)[0]
+    assert np.abs(got[:, :4] - want).max() <= 1e-10
+
+
 @pytest.mark.parametrize("n", [1, 63, 65, 32768, 32769, 70000])
 def test_fluid_particles_read_back_as_set(n):
     """Around the rows of a workgroup and the particles read back at a time."""
