@@ -670,6 +670,7 @@ __global__ __launch_bounds__(256) void k_train_reduce(const float *__restrict__ 
 // ------------------------------------------------------------- handle
 struct amh_mlp_s {
     int32_t batch = 0;
+    int cus = 0;  // of the device the handle was made on
     void *buf = nullptr;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // [kParams]
     uint16_t *pb = nullptr;                                         // bfloat16 copy
@@ -681,27 +682,27 @@ struct amh_mlp_s {
 };
 
 namespace {
-int g_cus = 0;
-int g_fused = -1;  // -1 unknown, 0 no, 1 yes
-// The fused kernels' LDS (110 KB and 137 KB in one workgroup).
-bool fused_ok() {
-    if (g_fused >= 0) return g_fused == 1;
-    int dev = 0, cus = 0;
-    g_fused = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mlp_fused), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            int(kFusedLds)) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void *>(&k_train), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            int(sizeof(TrainLds))) != hipSuccess)
-        return false;
-    g_cus = cus;
-    g_fused = 1;
-    return true;
+// Readies the current device for the fused kernels (110 KB and 137 KB of LDS in
+// one workgroup) and counts its CUs.  Each handle asks for itself: handles may
+// be made from several threads at once and on several devices.
+int fused_kernels(int &cus) {
+    const char *what = "amh_mlp_create: the kernels' LDS";
+    int dev = 0;
+    int r = check_hip(hipGetDevice(&dev), what);
+    if (!r) r = check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), what);
+    if (!r)
+        r = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mlp_fused),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(kFusedLds)),
+                      what);
+    if (!r)
+        r = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_train),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(sizeof(TrainLds))),
+                      what);
+    return r;
 }
 
 // Workgroups of the training step on n rows: one per CU at most.
-int train_groups(int n) { return std::min(g_cus, (n + kTrainRows - 1) / kTrainRows); }
+int train_groups(int cus, int n) { return std::min(cus, (n + kTrainRows - 1) / kTrainRows); }
 
 int stage_image(amh_mlp_s *M, hipStream_t s) {
     hipLaunchKernelGGL(k_fused_stage, dim3(64), dim3(256), 0, s, M->pb, M->p, M->image);
@@ -715,13 +716,15 @@ extern "C" int amh_mlp_create(void **mlp, int32_t batch_max, void *stream) {
         set_error("amh_mlp_create: invalid argument");
         return AMH_E_ARG;
     }
-    if (!fused_ok()) return check_hip(hipErrorInvalidDevice, "amh_mlp_create: the kernels' LDS");
+    int cus = 0;
+    if (int r = fused_kernels(cus)) return r;
     amh_mlp_s *M = new amh_mlp_s;
     M->batch = batch_max;
+    M->cus = cus;
     const auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t vec = al(kParams * 4), half = al(kParams * 2), train = al(sizeof(TrainImage));
     const size_t held = 4 * vec + half + al(kFusedLds) + train;
-    if (int r = check_hip(hipMalloc(&M->buf, held + size_t(train_groups(batch_max)) * kPart * 4), "amh_mlp_create")) {
+    if (int r = check_hip(hipMalloc(&M->buf, held + size_t(train_groups(cus, batch_max)) * kPart * 4), "amh_mlp_create")) {
         delete M;
         return r;
     }
@@ -782,7 +785,7 @@ extern "C" int amh_mlp_forward(void *mlp, const float *x, int64_t n, float *out,
     if (n == 0) return AMH_OK;
     const int64_t tiles = (n + 31) / 32;
     // from four waves' tiles a workgroup, one per SIMD, on more CUs first
-    const uint32_t grid = uint32_t(std::min<int64_t>(g_cus, (tiles + 3) / 4));
+    const uint32_t grid = uint32_t(std::min<int64_t>(M->cus, (tiles + 3) / 4));
     if (M->image_stale) stage_image(M, s);
     hipLaunchKernelGGL(k_mlp_fused, dim3(grid), dim3(kFusedThreads), kFusedLds, s, x, n, M->image, out);
     AMH_LAUNCH_CHECK("amh_mlp_forward");
@@ -798,7 +801,7 @@ extern "C" int amh_mlp_gradients(void *mlp, const float *x, const float *t, int3
     if (!M || !x || !t || n <= 0 || n > M->batch) { set_error("amh_mlp_gradients: invalid argument"); return AMH_E_ARG; }
     hipStream_t s = static_cast<hipStream_t>(stream);
     amh::ProfScope ps_("mlp_gradients", s);
-    const int groups = train_groups(n);
+    const int groups = train_groups(M->cus, n);
     hipLaunchKernelGGL(k_train, dim3(uint32_t(groups)), dim3(kTrainThreads), sizeof(TrainLds), s, x, t, int(n),
                        M->train, M->p, M->part);
     hipLaunchKernelGGL(k_train_reduce, dim3((kPart + 63) / 64), dim3(256), 0, s, M->part, groups, M->g, grad, loss_dev);

@@ -3,6 +3,8 @@ CPU oracle, which rounds the operands of every product to bfloat16 the same
 way; tolerances cover FP32-vs-FP64 accumulation and the rare activation
 that rounds to the other bfloat16 neighbour."""
 import ctypes as C
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -178,3 +180,31 @@ def test_adam_training_reduces_loss():
         G.lib().amh_mlp_destroy(h)
     assert losses[-1] < 0.05 * losses[0], losses
     assert np.isfinite(q).all() and not np.array_equal(q, p)
+
+
+def test_first_handles_made_from_several_threads():
+    """Threads whose first calls are amh_mlp_create, at the same time, in a
+    process that has made no handle yet: every one gets a handle (a job with
+    the learned start that another job's first handle overlaps must not lose
+    its own)."""
+    code = """
+import ctypes as C, threading
+from atomorph_amd import _capi as A
+lib = A.load()
+rcs, gate = [], threading.Barrier(8)
+def make():
+    h = C.c_void_p()
+    gate.wait()
+    rc = lib.amh_mlp_create(C.byref(h), 64, None)
+    rcs.append((rc, lib.amh_last_error() if rc else b""))
+    if rc == 0:
+        lib.amh_mlp_destroy(h)
+threads = [threading.Thread(target=make) for _ in range(8)]
+for t in threads: t.start()
+for t in threads: t.join()
+assert all(rc == 0 for rc, _ in rcs), rcs
+print("made", len(rcs))
+"""
+    G.log("mlp handles from 8 threads")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
+    assert r.returncode == 0 and "made 8" in r.stdout, r.stdout + r.stderr
