@@ -661,7 +661,7 @@ __global__ __launch_bounds__(256) void k_train_reduce(const float *__restrict__ 
         g[i] = v;
         if (grad) grad[i] = v;
     } else if (loss) {
-        *loss += v;
+        atomicAdd(loss, v);  // (other handles' steps, on other streams, may add to it too)
     }
 }
 

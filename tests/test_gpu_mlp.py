@@ -208,3 +208,36 @@ print("made", len(rcs))
     G.log("mlp handles from 8 threads")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
     assert r.returncode == 0 and "made 8" in r.stdout, r.stdout + r.stderr
+
+
+def test_losses_of_several_streams_add_up():
+    """Handles on streams of their own that add their losses to one word:
+    none is lost.  FP32 rounding of 1,200 additions is at most 1,200 x 2^-24 =
+    7e-5 of the sum (1e-4 asserted); a lost loss is 8e-4 of it."""
+    rng = np.random.default_rng(21)
+    n, calls, handles = 64, 300, 4
+    lib, T = G.lib(), G.torch()
+    x, t = rng.normal(0, 1, (n, 8)).astype(np.float32), rng.normal(0, 1, (n, 2)).astype(np.float32)
+    p = _mlp_params(rng)
+    dx, dt = G.to_dev(x), G.to_dev(t)
+    hs, streams = [_mlp(n, p) for _ in range(handles)], [C.c_void_p() for _ in range(handles)]
+    try:
+        _, one = _gradients(hs[0], x, t)
+        dl = G.zeros(1, T.float32)
+        for s in streams:
+            G.check(lib.amh_stream_create(C.byref(s)), "stream")
+        G.sync()
+        G.log(f"mlp losses of {handles} streams, {calls} steps each")
+        for _ in range(calls):
+            for h, s in zip(hs, streams):
+                G.check(lib.amh_mlp_gradients(h, G.dptr(dx), G.dptr(dt), n, None, G.dptr(dl), s), "grad")
+        for s in streams:
+            G.check(lib.amh_stream_sync(s), "sync")
+        total = float(G.to_host(dl, np.float32)[0])
+    finally:
+        G.sync()
+        for h in hs:
+            lib.amh_mlp_destroy(h)
+        for s in streams:
+            lib.amh_stream_destroy(s)
+    assert abs(total - handles * calls * one) <= 1e-4 * handles * calls * one, (total, one)
