@@ -1681,7 +1681,7 @@ void bin_particles(const Tiles &tiles_of, int n, const Bins &B, int tiles, int p
         hipLaunchKernelGGL((k_bin_place<true, Tiles, Tail>), dim3(gb), dim3(kT), 0, s, tiles_of, n, B, tiles, par,
                            tail);
     } else {
-        hipLaunchKernelGGL(scan::k_scan_sums, dim3(1), dim3(1024), 0, s, B.count[par], tiles, B.start);
+        hipLaunchKernelGGL(scan::k_scan_sums<int>, dim3(1), dim3(1024), 0, s, B.count[par], tiles, B.start);
         hipLaunchKernelGGL((k_bin_place<false, Tiles, Tail>), dim3(gb), dim3(kT), 0, s, tiles_of, n, B, tiles, par,
                            tail);
     }

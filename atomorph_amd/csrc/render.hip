@@ -47,6 +47,10 @@ constexpr int kLdsTiles = 4096;       // up to this many tiles every placing blo
 constexpr int kFewTiles = 4096;       // up to this many tiles blocks count and place atoms per tile in LDS
 constexpr int kManyTiles = 16384;     // up to this many, larger blocks count them there
 constexpr int kNoBlob = 0x7FFFFFFF;
+// The tiles' lists are indexed by 32-bit sums of the atoms' taps, four of an
+// atom at most (kEnd is none of them).
+constexpr int64_t kMaxAtoms = 0x3FFFFFFF;
+constexpr uint32_t kEnd = 0xFFFFFFFFu;
 
 // --------------------------------------------------------------- prepare
 struct Rec {       // one atom's splat, 16 bytes
@@ -59,10 +63,10 @@ struct Rec {       // one atom's splat, 16 bytes
 // The image tiles and their lists.
 struct Tiles {
     int32_t ntx, nty;
-    int32_t *taps;     // [tiles] taps that fall in the tile
-    int32_t *entries;  // [tiles] atoms listed so far
-    int32_t *start;    // [tiles + 1] scan of taps: a tile lists at most one atom per tap
-    uint32_t *list;    // [<= 4 atoms] atom numbers
+    uint32_t *taps;     // [tiles] taps that fall in the tile
+    uint32_t *entries;  // [tiles] atoms listed so far
+    uint32_t *start;    // [tiles + 1] scan of taps: a tile lists at most one atom per tap
+    uint32_t *list;     // [<= 4 atoms] atom numbers
 };
 
 // The taps of `mask` (bit k: tap (k & 1, k >> 1) of the base pixel x, y) that
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__re
             if ((c.x | c.y | c.z | c.w) == 0) continue;
             const uint32_t w[4] = {c.x, c.y, c.z, c.w};
             for (int q = 0; q < 8; ++q) {
-                const int n = int(w[q / 2] >> (q % 2 * 16) & 0xFFFFu);
+                const uint32_t n = w[q / 2] >> (q % 2 * 16) & 0xFFFFu;
                 if (n) atomicAdd(&B.taps[8 * k + q], n);
             }
         }
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__re
             const int leader = __ffsll((unsigned long long)todo) - 1;
             const uint64_t same = __ballot(t == __builtin_amdgcn_readlane(t, leader));
             if (lane == leader)
-                atomicAdd(&B.taps[t], int(__popcll(same & w0) + 2 * __popcll(same & w1) + 4 * __popcll(same & w2)));
+                atomicAdd(&B.taps[t], uint32_t(__popcll(same & w0) + 2 * __popcll(same & w1) + 4 * __popcll(same & w2)));
             todo &= ~same;
         }
     }
@@ -177,12 +181,12 @@ __global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__re
 // kFew: ranks within the block from LDS counters, as in k_prepare.
 template <bool kLds, bool kFew>
 __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int64_t n, Tiles B) {
-    __shared__ int sstart[kLds ? kLdsTiles + 1 : 1];
-    __shared__ int wsum[kT / 64];
+    __shared__ uint32_t sstart[kLds ? kLdsTiles + 1 : 1];
+    __shared__ uint32_t wsum[kT / 64];
     const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
     const uint2 r = *reinterpret_cast<const uint2 *>(&recs[a < n ? a : 0]);
     const uint32_t X = r.x & 0xFFFFu, Y = r.x >> 16, mask = a < n ? r.y >> 16 : 0u;
-    const int32_t *start = B.start;
+    const uint32_t *start = B.start;
     if (kLds) {
         const int tiles = B.ntx * B.nty;
         scan::block_exclusive(tiles, [&](int k) { return B.taps[k]; }, sstart, wsum);
@@ -191,14 +195,15 @@ __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int6
         start = sstart;
     }
     if (kFew) {
-        __shared__ int cnt[kFew ? kFewTiles : 1];
+        __shared__ uint32_t cnt[kFew ? kFewTiles : 1];
         const int tiles = B.ntx * B.nty;
         for (int k = threadIdx.x; k < tiles; k += kT) cnt[k] = 0;
         __syncthreads();
-        int t[4], rank[4];
+        int t[4];
+        uint32_t rank[4];
         for (int j = 0; j < 4; ++j) {
             t[j] = taps_in(mask, X, Y, j) ? tile_of(X, Y, j, B.ntx) : -1;
-            rank[j] = t[j] >= 0 ? atomicAdd(&cnt[t[j]], 1) : 0;
+            rank[j] = t[j] >= 0 ? atomicAdd(&cnt[t[j]], 1u) : 0u;
         }
         __syncthreads();
         for (int k = threadIdx.x; k < tiles; k += kT)
@@ -210,30 +215,31 @@ __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int6
     }
     const int lane = threadIdx.x & 63;
     const uint64_t below = (1ull << lane) - 1ull;
-    int t[4], lead[4], pre[4], total[4];  // the wave's lanes grouped by tile, per neighbour tile
+    int t[4], lead[4];  // the wave's lanes grouped by tile, per neighbour tile
+    uint32_t pre[4], total[4];
     for (int j = 0; j < 4; ++j) {
         t[j] = taps_in(mask, X, Y, j) ? tile_of(X, Y, j, B.ntx) : -1;
         lead[j] = lane;
-        pre[j] = total[j] = 0;
+        pre[j] = total[j] = 0u;
         uint64_t todo = __ballot(t[j] >= 0);
         while (todo) {
             const int leader = __ffsll((unsigned long long)todo) - 1;
             const uint64_t same = __ballot(t[j] == __builtin_amdgcn_readlane(t[j], leader));
             if ((same >> lane) & 1u) {
                 lead[j] = leader;
-                pre[j] = int(__popcll(same & below));
+                pre[j] = uint32_t(__popcll(same & below));
             }
-            if (lane == leader) total[j] = int(__popcll(same));
+            if (lane == leader) total[j] = uint32_t(__popcll(same));
             todo &= ~same;
         }
     }
-    int base[4], first[4];
+    uint32_t base[4], first[4];
     for (int j = 0; j < 4; ++j) {
-        base[j] = total[j] > 0 ? atomicAdd(&B.entries[t[j]], total[j]) : 0;
+        base[j] = total[j] > 0u ? atomicAdd(&B.entries[t[j]], total[j]) : 0u;
         first[j] = start[max(t[j], 0)];
     }
     for (int j = 0; j < 4; ++j) {
-        const int b = __shfl(base[j], lead[j], 64);
+        const uint32_t b = __shfl(base[j], lead[j], 64);
         if (t[j] >= 0) B.list[first[j] + b + pre[j]] = uint32_t(a);
     }
 }
@@ -270,18 +276,18 @@ __device__ __forceinline__ Px resolve(uint32_t cnt, T sn, const T s[4], int dens
 struct Ov {
     int32_t blob;
     uint32_t col;
-    int32_t next;  // -1: last
+    uint32_t next;  // kEnd: last
 };
 struct Resolved {
     int32_t *blob;  // [npx] kNoBlob: none
     uint32_t *col;
-    int32_t *next;
+    uint32_t *next;
     Ov *ov;         // [<= 4 atoms]
 };
 
 // Is blob b among the further blobs of pixel q?
 __device__ __forceinline__ bool chained(const Resolved &V, int64_t q, int b) {
-    for (int i = V.next[q]; i >= 0; i = V.ov[i].next)
+    for (uint32_t i = V.next[q]; i != kEnd; i = V.ov[i].next)
         if (V.ov[i].blob == b) return true;
     return false;
 }
@@ -528,15 +534,17 @@ __global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *
     } acc;
     __shared__ int bcur[kTilePx], bnext[kTilePx];
     __shared__ std::conditional_t<kMode == kOver, PerlinTab, char> tab;
-    __shared__ int nov, some;
+    __shared__ uint32_t nov;
+    __shared__ int some;
     const int tile = int(blockIdx.x), tid = int(threadIdx.x);
     const int x0 = (tile % B.ntx) * kTile, y0 = (tile / B.ntx) * kTile;
     const int x = x0 + tid % kTile, y = y0 + tid / kTile;
     const bool inside = x < R.width && y < R.height;
     const int64_t p = int64_t(y) * R.width + x;
-    const int n = B.entries[tile], s0 = B.start[tile];
+    const int n = int(B.entries[tile]);
+    const uint32_t s0 = B.start[tile];
     std::conditional_t<kMode == kOver, Blend, Over> fold;
-    int last = -1;  // kFeather: the pixel's last chained Ov
+    uint32_t last = kEnd;  // kFeather: the pixel's last chained Ov
     bool first = true;
     if constexpr (kMode == kOver)
         if (R.keep_background && R.fading == kPerlin) stage_perlin(R.lag_perm_dev, R.slope_perm_dev, tab, tid, kT);
@@ -559,9 +567,9 @@ __global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *
                     V.blob[p] = b;
                     V.col[p] = c;
                 } else {
-                    const int o = s0 + atomicAdd(&nov, 1);
-                    V.ov[o] = Ov{b, c, -1};
-                    if (last < 0) V.next[p] = o;
+                    const uint32_t o = s0 + atomicAdd(&nov, 1u);
+                    V.ov[o] = Ov{b, c, kEnd};
+                    if (last == kEnd) V.next[p] = o;
                     else V.ov[last].next = o;
                     last = o;
                 }
@@ -584,7 +592,7 @@ __global__ __launch_bounds__(kT) void k_splat(amh_render R, Frame F, const Rec *
     if (!inside) return;
     if constexpr (kMode == kFeather) {
         if (first) V.blob[p] = kNoBlob;
-        if (last < 0) V.next[p] = -1;
+        if (last == kEnd) V.next[p] = kEnd;
     } else if constexpr (kMode == kOver) {
         out[p] = finish(R, fold, R.keep_background ? background(R, F, x, y, tab) : 0u);
     } else {
@@ -611,7 +619,7 @@ __global__ __launch_bounds__(kT) void k_composite(amh_render R, Frame F, Resolve
         if (d <= R.feather)
             c = (c & 0x00FFFFFFu) | (narrow8(round(double(c >> 24) * (double(d) / double(R.feather + 1)))) << 24);
         if (c >> 24) fold.add(c);
-        if (o.next < 0) break;
+        if (o.next == kEnd) break;
         o = V.ov[o.next];
     }
     out[p] = finish(R, fold, R.keep_background ? background(R, F, x, y, tab) : 0u);
@@ -657,8 +665,8 @@ Layout layout(int32_t W, int32_t H, int64_t wtot) {
 }
 
 Tiles tiles_of(char *ws, const Layout &L) {
-    return Tiles{L.ntx, L.nty, reinterpret_cast<int32_t *>(ws + L.taps), reinterpret_cast<int32_t *>(ws + L.entries),
-                 reinterpret_cast<int32_t *>(ws + L.start), reinterpret_cast<uint32_t *>(ws + L.list)};
+    return Tiles{L.ntx, L.nty, reinterpret_cast<uint32_t *>(ws + L.taps), reinterpret_cast<uint32_t *>(ws + L.entries),
+                 reinterpret_cast<uint32_t *>(ws + L.start), reinterpret_cast<uint32_t *>(ws + L.list)};
 }
 
 }  // namespace
@@ -685,7 +693,7 @@ bool render_args_ok(const amh_render *R) {
     return R && R->width > 0 && R->height > 0 && R->nkeys > 0 && R->nchains >= 0 && R->keys_dev &&
            !(R->wtot > 0 && (!R->pts_dev || !R->chain_off_dev || !R->chain_w_dev || !R->rank_dev)) &&
            !(R->fading == kPerlin && (!R->lag_perm_dev || !R->slope_perm_dev)) && R->width <= 65535 &&
-           R->height <= 65535 && R->wtot >= 0;
+           R->height <= 65535 && R->wtot >= 0 && R->wtot <= kMaxAtoms;
 }
 
 // The frame itself, on a workspace laid out by `L` whose tile counters are
@@ -746,9 +754,9 @@ int scratch_ptr(char **out) {
 }
 
 // The tile counters := 0.
-__global__ __launch_bounds__(kT) void k_ws_reset(int32_t *__restrict__ counters, int64_t n) {
+__global__ __launch_bounds__(kT) void k_ws_reset(uint32_t *__restrict__ counters, int64_t n) {
     const int64_t i = int64_t(blockIdx.x) * kT + threadIdx.x;
-    if (i < n) counters[i] = 0;
+    if (i < n) counters[i] = 0u;
 }
 
 }  // namespace
@@ -771,7 +779,7 @@ extern "C" int amh_render_frame_noalloc(const amh_render *R, double t, uint32_t 
     if (int r = scratch_ptr(&base)) return r;
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipLaunchKernelGGL(k_ws_reset, dim3(uint32_t((2 * L.tiles + kT - 1) / kT)), dim3(kT), 0, s,
-                       reinterpret_cast<int32_t *>(base + L.taps), 2 * L.tiles);
+                       reinterpret_cast<uint32_t *>(base + L.taps), 2 * L.tiles);
     AMH_LAUNCH_CHECK("amh_render_frame_noalloc");
     return render_frame_on(R, t, base, L, out, s);
 }
@@ -782,7 +790,7 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
     Rec *recs = reinterpret_cast<Rec *>(base + L.recs);
     const Tiles B = tiles_of(base, L);
     const Resolved V = {reinterpret_cast<int32_t *>(base + L.blob), reinterpret_cast<uint32_t *>(base + L.col),
-                        reinterpret_cast<int32_t *>(base + L.next), reinterpret_cast<Ov *>(base + L.ov)};
+                        reinterpret_cast<uint32_t *>(base + L.next), reinterpret_cast<Ov *>(base + L.ov)};
 
     // morph::normalize_time / get_frame_key (morph.cpp:404-450, 460-464)
     Frame F;
@@ -812,8 +820,8 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
         if (L.tiles <= kLdsTiles) {
             launch("k_place", few ? k_place<true, true> : k_place<true, false>, Rc.wtot, recs, Rc.wtot, B);
         } else {
-            scan::exclusive(B.taps, L.tiles, reinterpret_cast<int *>(base + L.sums),
-                            reinterpret_cast<int *>(base + L.offs), B.start, s);
+            scan::exclusive(B.taps, L.tiles, reinterpret_cast<uint32_t *>(base + L.sums),
+                            reinterpret_cast<uint32_t *>(base + L.offs), B.start, s);
             launch("k_place", k_place<false, false>, Rc.wtot, recs, Rc.wtot, B);
         }
     }

@@ -1,6 +1,7 @@
-// Exclusive prefix sum of int counts on the device: per-block sums, one
-// block scanning the block sums, then per-block scans with the block offset.
-// Used to turn per-pixel and per-cell counts into segment starts.
+// Exclusive prefix sum of counts (T: int, or uint32_t where the total passes
+// 2^31) on the device: per-block sums, one block scanning the block sums, then
+// per-block scans with the block offset.  Used to turn per-pixel and per-cell
+// counts into segment starts.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -14,10 +15,11 @@ inline int64_t blocks(int64_t n) { return (n + kBlock - 1) / kBlock; }
 
 namespace {
 
-__global__ __launch_bounds__(256) void k_blk_sum(const int *__restrict__ in, int64_t n, int *__restrict__ sums) {
-    __shared__ int part[4];
+template <class T>
+__global__ __launch_bounds__(256) void k_blk_sum(const T *__restrict__ in, int64_t n, T *__restrict__ sums) {
+    __shared__ T part[4];
     const int64_t base = int64_t(blockIdx.x) * kBlock;
-    int s = 0;
+    T s = 0;
     for (int l = threadIdx.x; l < kBlock; l += 256) {
         const int64_t i = base + l;
         if (i < n) s += in[i];
@@ -29,18 +31,19 @@ __global__ __launch_bounds__(256) void k_blk_sum(const int *__restrict__ in, int
 }
 
 // offs[b] = sums[0] + ... + sums[b-1]; offs[nb] = total
-__global__ __launch_bounds__(1024) void k_scan_sums(const int *__restrict__ in, int nb, int *__restrict__ out) {
-    __shared__ int buf[1024];
-    __shared__ int carry;
+template <class T>
+__global__ __launch_bounds__(1024) void k_scan_sums(const T *__restrict__ in, int nb, T *__restrict__ out) {
+    __shared__ T buf[1024];
+    __shared__ T carry;
     if (threadIdx.x == 0) carry = 0;
     __syncthreads();
     for (int base = 0; base < nb; base += 1024) {
         const int i = base + threadIdx.x;
-        const int v = i < nb ? in[i] : 0;
+        const T v = i < nb ? in[i] : 0;
         buf[threadIdx.x] = v;
         __syncthreads();
         for (int off = 1; off < 1024; off <<= 1) {
-            const int t = threadIdx.x >= off ? buf[threadIdx.x - off] : 0;
+            const T t = threadIdx.x >= off ? buf[threadIdx.x - off] : 0;
             __syncthreads();
             buf[threadIdx.x] += t;
             __syncthreads();
@@ -54,23 +57,24 @@ __global__ __launch_bounds__(1024) void k_scan_sums(const int *__restrict__ in, 
 }
 
 // exclusive scan inside each block plus the block's offset; out[n] = total
-__global__ __launch_bounds__(256) void k_blk_apply(const int *__restrict__ in, int64_t n,
-                                                   const int *__restrict__ offs, int nb, int *__restrict__ out) {
-    __shared__ int wsum[4];
+template <class T>
+__global__ __launch_bounds__(256) void k_blk_apply(const T *__restrict__ in, int64_t n, const T *__restrict__ offs,
+                                                   int nb, T *__restrict__ out) {
+    __shared__ T wsum[4];
     const int64_t base = int64_t(blockIdx.x) * kBlock;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int running = offs[blockIdx.x];
+    T running = offs[blockIdx.x];
     for (int chunk = 0; chunk < kBlock / 256; ++chunk) {
         const int64_t i = base + chunk * 256 + threadIdx.x;
-        const int v = i < n ? in[i] : 0;
-        int incl = v;
+        const T v = i < n ? in[i] : 0;
+        T incl = v;
         for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off, 64);
+            const T t = __shfl_up(incl, off, 64);
             if (lane >= off) incl += t;
         }
         if (lane == 63) wsum[wave] = incl;
         __syncthreads();
-        int before = running;
+        T before = running;
         for (int w = 0; w < wave; ++w) before += wsum[w];
         if (i < n) out[i] = before + incl - v;
         running += wsum[0] + wsum[1] + wsum[2] + wsum[3];
@@ -84,29 +88,30 @@ __global__ __launch_bounds__(256) void k_blk_apply(const int *__restrict__ in, i
 // values, 256 threads); the last block writes out[n] = total.
 constexpr int kFoldBlocks = 2048;
 
-__global__ __launch_bounds__(256) void k_blk_apply_fold(const int *__restrict__ in, int64_t n,
-                                                        const int *__restrict__ sums, int nb, int *__restrict__ out) {
-    __shared__ int wsum[4];
+template <class T>
+__global__ __launch_bounds__(256) void k_blk_apply_fold(const T *__restrict__ in, int64_t n,
+                                                        const T *__restrict__ sums, int nb, T *__restrict__ out) {
+    __shared__ T wsum[4];
     const int64_t base = int64_t(blockIdx.x) * kBlock;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int o = 0;
+    T o = 0;
     for (int j = threadIdx.x; j < int(blockIdx.x); j += 256) o += sums[j];
     for (int off = 32; off > 0; off >>= 1) o += __shfl_down(o, off, 64);
     if (lane == 0) wsum[wave] = o;
     __syncthreads();
-    int running = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    T running = wsum[0] + wsum[1] + wsum[2] + wsum[3];
     __syncthreads();  // wsum is reused below
     for (int chunk = 0; chunk < kBlock / 256; ++chunk) {
         const int64_t i = base + chunk * 256 + threadIdx.x;
-        const int v = i < n ? in[i] : 0;
-        int incl = v;
+        const T v = i < n ? in[i] : 0;
+        T incl = v;
         for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off, 64);
+            const T t = __shfl_up(incl, off, 64);
             if (lane >= off) incl += t;
         }
         if (lane == 63) wsum[wave] = incl;
         __syncthreads();
-        int before = running;
+        T before = running;
         for (int w = 0; w < wave; ++w) before += wsum[w];
         if (i < n) out[i] = before + incl - v;
         running += wsum[0] + wsum[1] + wsum[2] + wsum[3];
@@ -120,25 +125,25 @@ constexpr int kBlockT = 256;
 // Exclusive scan of value(k) over k < n into out[0..n] (out[n] = total) by the
 // whole block of kBlockT threads in LDS: thread t takes a run of k.  value is
 // called once per k, by the thread of its run, in order.
-template <class Value>
-__device__ __forceinline__ void block_exclusive(int n, const Value &value, int *out, int *wsum) {
+template <class T, class Value>
+__device__ __forceinline__ void block_exclusive(int n, const Value &value, T *out, T *wsum) {
     const int per = (n + kBlockT - 1) / kBlockT;
     const int lo = min(int(threadIdx.x) * per, n), hi = min(lo + per, n);
-    int sum = 0;
+    T sum = 0;
     for (int k = lo; k < hi; ++k) {
-        const int v = value(k);
+        const T v = value(k);
         out[k] = sum;
         sum += v;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = sum;
+    T incl = sum;
     for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(incl, off, 64);
+        const T v = __shfl_up(incl, off, 64);
         if (lane >= off) incl += v;
     }
     if (lane == 63) wsum[wave] = incl;
     __syncthreads();
-    int off = incl - sum;
+    T off = incl - sum;
     for (int w = 0; w < wave; ++w) off += wsum[w];
     for (int k = lo; k < hi; ++k) out[k] += off;
     if (threadIdx.x == kBlockT - 1) out[n] = off + sum;
@@ -150,15 +155,16 @@ __device__ __forceinline__ void block_exclusive(int n, const Value &value, int *
 // out[0..n] = exclusive scan of in[0..n) with out[n] = total.  Workspace:
 // sums[blocks(n)], offs[blocks(n) + 1].  n > 0.  Up to kFoldBlocks blocks
 // the block sums are not scanned by a launch of their own.
-inline void exclusive(const int *in, int64_t n, int *sums, int *offs, int *out, hipStream_t s) {
+template <class T>
+inline void exclusive(const T *in, int64_t n, T *sums, T *offs, T *out, hipStream_t s) {
     const int64_t nb = blocks(n);
-    hipLaunchKernelGGL(k_blk_sum, dim3(uint32_t(nb)), dim3(256), 0, s, in, n, sums);
+    hipLaunchKernelGGL(k_blk_sum<T>, dim3(uint32_t(nb)), dim3(256), 0, s, in, n, sums);
     if (nb <= kFoldBlocks) {
-        hipLaunchKernelGGL(k_blk_apply_fold, dim3(uint32_t(nb)), dim3(256), 0, s, in, n, sums, int(nb), out);
+        hipLaunchKernelGGL(k_blk_apply_fold<T>, dim3(uint32_t(nb)), dim3(256), 0, s, in, n, sums, int(nb), out);
         return;
     }
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, int(nb), offs);
-    hipLaunchKernelGGL(k_blk_apply, dim3(uint32_t(nb)), dim3(256), 0, s, in, n, offs, int(nb), out);
+    hipLaunchKernelGGL(k_scan_sums<T>, dim3(1), dim3(1024), 0, s, sums, int(nb), offs);
+    hipLaunchKernelGGL(k_blk_apply<T>, dim3(uint32_t(nb)), dim3(256), 0, s, in, n, offs, int(nb), out);
 }
 
 }  // namespace scan

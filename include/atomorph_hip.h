@@ -263,7 +263,7 @@ typedef struct amh_render {
     int32_t keep_background;
     int32_t blend_blobs;
     int32_t nchains;
-    int64_t wtot;
+    int64_t wtot;                   /* atoms, at most 2^30 - 1 in a frame    */
     const uint32_t *keys_dev;       /* [nkeys][height*width] get_pixel colour */
     const uint64_t *pts_dev;        /* [nkeys][wtot] chain points             */
     const int64_t *chain_off_dev;   /* [nchains]                              */

@@ -61,6 +61,21 @@ def test_error_path_without_device_work():
     assert lib.amh_render_graph_destroy(None) == 0
 
 
+def test_render_refuses_more_atoms_than_its_lists_index():
+    """The tiles' lists are indexed by 32-bit sums of up to four taps per atom:
+    2^30 atoms are refused before any HIP call, by every entry point that
+    draws a frame (never dereferenced: the pointers are made up)."""
+    lib = A.load()
+    made_up = 1 << 20
+    args = A.RenderArgs(64, 64, 2, 1, 0, 0, 63, 63, 3, 3, 0, 1, 0, 0, 0, 1, 1 << 30, *([made_up] * 8))
+    ws, many, g = C.c_void_p(made_up), 1 << 50, C.c_void_p()
+    for rc in (lib.amh_render_frame(C.byref(args), 0.0, ws, many, ws, None),
+               lib.amh_render_frame_noalloc(C.byref(args), 0.0, ws, None),
+               lib.amh_render_graph_create(C.byref(g), C.byref(args), ws, many, ws)):
+        assert rc == -1 and b"invalid argument" in lib.amh_last_error()
+    assert not g.value
+
+
 @pytest.mark.parametrize("gsx,gsy,w,h", [(65535, 64, 64, 64), (64, 70000, 64, 64), (64, 64, 65536, 8),
                                          (64, 64, 8, 100000), (7, 64, 64, 64)])
 def test_fluid_create_rejects_sizes_the_packing_cannot_hold(gsx, gsy, w, h):

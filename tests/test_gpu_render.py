@@ -225,3 +225,44 @@ def test_render_scattered_atoms_on_many_tiles(W, H):
                                 3, None, 0.21, op.ptr(want))
     assert int(np.abs(got.astype(np.int32) - want.astype(np.int32)).max()) <= 1
     assert (rend.frame(0.21) == got).all()
+
+
+@pytest.mark.parametrize("W,H", [(64, 64), (1040, 1024)])
+def test_render_more_taps_than_31_bits_count(W, H):
+    """2^29 + 999 atoms, each with four taps, so that the tiles' lists start
+    beyond 2^31: 131,072 or so per pixel on few tiles, 504 on many.  Every
+    pixel is the rounded mean of the up to four key pixels whose atoms reach
+    it, exactly (52 GB of device memory)."""
+    T, lib = G.torch(), G.lib()
+    wtot, h, n = (1 << 29) + 999, 2, W * H
+    rng = np.random.default_rng(W)
+    keys = rng.integers(0, 256, (h, H, W, 4)).astype(np.uint8)
+    keys[..., 3] = 255
+    a = T.arange(wtot, device="cuda") % n
+    pts = T.empty(h, wtot, dtype=T.int64, device="cuda")
+    T.remainder(a, W, out=pts[0])
+    pts[0] |= T.div(a, W, rounding_mode="floor") << 16
+    del a
+    pts[0] |= (128 << 32) | (128 << 40) | (3 << 48)
+    pts[1] = pts[0]
+    dkeys = G.to_dev(keys.view(np.uint32).reshape(-1))
+    off, width, rank = G.to_dev(np.zeros(1, np.int64)), G.to_dev(np.array([wtot], np.int32)), G.zeros(h, T.int32)
+    args = A.RenderArgs(W, H, h, 1, 0, 0, W - 1, H - 1, 3, 3, 0, 1, 0, 0, 0, 1, wtot, dkeys.data_ptr(), pts.data_ptr(),
+                        off.data_ptr(), width.data_ptr(), rank.data_ptr(), None, None, None)
+    wsb = lib.amh_render_workspace_bytes(W, H, wtot)
+    ws, out = T.empty(wsb, dtype=T.uint8, device="cuda"), G.zeros(n, T.int32)
+    G.check(lib.amh_render_workspace_init(G.dptr(ws), wsb, W, H, wtot, G.stream()), "workspace init")
+    G.sync()
+    G.log(f"render {W}x{H}, {wtot} atoms")
+    G.check(lib.amh_render_frame(C.byref(args), 0.0, G.dptr(ws), wsb, G.dptr(out), G.stream()), "amh_render_frame")
+    got = G.to_host(out, np.uint32).view(np.uint8).reshape(H, W, 4).astype(np.int64)
+    del ws, pts
+    T.cuda.empty_cache()
+    per = (wtot // n + (np.arange(n) < wtot % n)).reshape(H, W)
+    den, num = np.zeros((H, W), np.int64), np.zeros((H, W, 4), np.int64)
+    for dy in (0, 1):
+        for dx in (0, 1):
+            w = per[:H - dy, :W - dx] * (128 if dx else 127) * (128 if dy else 127)
+            den[dy:, dx:] += w
+            num[dy:, dx:] += w[..., None] * keys[0, :H - dy, :W - dx].astype(np.int64)
+    assert (got == (2 * num + den[..., None]) // (2 * den[..., None])).all()
