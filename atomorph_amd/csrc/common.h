@@ -140,6 +140,16 @@ __host__ __device__ __forceinline__ uint64_t knn_draw(uint64_t seed, uint64_t st
     return mix64(seed ^ 0x2545F4914F6CDD1Dull ^ mix64(stream ^ (uint64_t(round) << 32) ^ l));
 }
 
+// ------------------------------------------------------------- one wave
+// Between LDS accesses of one wave that meet across its lanes: what a lane
+// stored before is what another reads after.  The LDS does a wave's accesses in
+// order, so this costs no instruction; it keeps the compiler to that order.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ------------------------------------------------------------ reductions
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);

@@ -231,9 +231,8 @@ __device__ __forceinline__ void run_rounds(uint2 *P, int2 *S, uint32_t *cs, int 
             }
             pairs += npairs;
             c = __builtin_amdgcn_readfirstlane(next);
-            // (one wave: its LDS accesses are in order anyway)
             if (NT > 64) __syncthreads();
-            else __builtin_amdgcn_wave_barrier();
+            else wave_order();
         }
         att += pairs;
         acc += swaps;

@@ -721,7 +721,9 @@ __global__ __launch_bounds__(kOneT) void k_group_one(const int *__restrict__ bop
     __syncthreads();
     for (int j = 0; j < kPer; ++j) {
         s[j] = same_lanes(b[j]);
-        if (s[j].total > 0 && s[j].rank == 0) cnt[wave][b[j]] += s[j].total;  // (this wave's own counts)
+        // (this wave's own counts, by another lane in the next turn)
+        if (s[j].total > 0 && s[j].rank == 0) cnt[wave][b[j]] += s[j].total;
+        wave_order();
     }
     __syncthreads();
     {   // thread b: blob b's total, its start, and each wave's first place
@@ -755,6 +757,7 @@ __global__ __launch_bounds__(kOneT) void k_group_one(const int *__restrict__ bop
             at = cnt[wave][b[j]];
             cnt[wave][b[j]] = at + s[j].total;
         }
+        wave_order();
         at = __shfl(at, s[j].lead, 64);
         if (b[j] >= 0) list[at + s[j].rank] = w0 + 64 * j + lane;
     }

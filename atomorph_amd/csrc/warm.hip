@@ -253,10 +253,11 @@ __global__ __launch_bounds__(kT) void k_rs_scatter(const uint64_t *__restrict__ 
             same &= ((d >> bit) & 1) ? bb : ~bb;
         }
         const int rank = int(__popcll(same & below));
+        wave_order();
         const int before = cnt[wave][d];
+        wave_order();
         if (ok && rank == 0) cnt[wave][d] = before + int(__popcll(same));
         pos[j] = before + rank;
-        __builtin_amdgcn_wave_barrier();
     }
     const int incl = block_inclusive(tot.x + tot.y, wsum);  // (its barrier publishes cnt)
     int b0 = incl - tot.x - tot.y + h.x, b1 = incl - tot.y + h.y;
