@@ -43,8 +43,7 @@ constexpr int kT = 256;
 constexpr int kTile = 16;             // pixels per side of an image tile
 constexpr int kTilePx = kTile * kTile;  // one thread of the splat per pixel
 static_assert(kTilePx == kT, "one thread per pixel");
-constexpr int kLdsTiles = 4096;       // up to this many tiles every placing block scans the counts in LDS
-constexpr int kFewTiles = 4096;       // up to this many tiles blocks count and place atoms per tile in LDS
+constexpr int kFewTiles = 4096;       // up to this many tiles blocks count, scan and place atoms per tile in LDS
 constexpr int kManyTiles = 16384;     // up to this many, larger blocks count them there
 constexpr int kNoBlob = 0x7FFFFFFF;
 // The tiles' lists are indexed by 32-bit sums of the atoms' taps, four of an
@@ -176,27 +175,20 @@ __global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__re
 }
 
 // The atoms' numbers into their tiles' lists, in no fixed order (the sums are
-// exact).  kLds: every block scans the tap counts in LDS (block 0 stores the
-// starts); otherwise B.start holds the scan already.
-// kFew: ranks within the block from LDS counters, as in k_prepare.
-template <bool kLds, bool kFew>
+// exact).  kFew: every block scans the tap counts in LDS (block 0 stores the
+// starts) and takes ranks within the block from LDS counters, as in k_prepare;
+// otherwise B.start holds the scan already and a wave's lanes are grouped.
+template <bool kFew>
 __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int64_t n, Tiles B) {
-    __shared__ uint32_t sstart[kLds ? kLdsTiles + 1 : 1];
-    __shared__ uint32_t wsum[kT / 64];
     const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
     const uint2 r = *reinterpret_cast<const uint2 *>(&recs[a < n ? a : 0]);
     const uint32_t X = r.x & 0xFFFFu, Y = r.x >> 16, mask = a < n ? r.y >> 16 : 0u;
-    const uint32_t *start = B.start;
-    if (kLds) {
+    if constexpr (kFew) {
+        __shared__ uint32_t start[kFewTiles + 1], cnt[kFewTiles], wsum[kT / 64];
         const int tiles = B.ntx * B.nty;
-        scan::block_exclusive(tiles, [&](int k) { return B.taps[k]; }, sstart, wsum);
+        scan::block_exclusive(tiles, [&](int k) { return B.taps[k]; }, start, wsum);
         if (blockIdx.x == 0)
-            for (int k = threadIdx.x; k <= tiles; k += kT) B.start[k] = sstart[k];
-        start = sstart;
-    }
-    if (kFew) {
-        __shared__ uint32_t cnt[kFew ? kFewTiles : 1];
-        const int tiles = B.ntx * B.nty;
+            for (int k = threadIdx.x; k <= tiles; k += kT) B.start[k] = start[k];
         for (int k = threadIdx.x; k < tiles; k += kT) cnt[k] = 0;
         __syncthreads();
         int t[4];
@@ -236,7 +228,7 @@ __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int6
     uint32_t base[4], first[4];
     for (int j = 0; j < 4; ++j) {
         base[j] = total[j] > 0u ? atomicAdd(&B.entries[t[j]], total[j]) : 0u;
-        first[j] = start[max(t[j], 0)];
+        first[j] = B.start[max(t[j], 0)];
     }
     for (int j = 0; j < 4; ++j) {
         const uint32_t b = __shfl(base[j], lead[j], 64);
@@ -811,18 +803,17 @@ int render_frame_on(const amh_render *R, double t, char *base, const Layout &L, 
         amh::launch_timed(name, kernel, dim3(uint32_t((threads + kT - 1) / kT)), dim3(kT), 0, s, args...);
     };
     if (Rc.wtot > 0) {
-        const bool few = L.tiles <= kFewTiles;
-        if (few) launch("k_prepare", k_prepare<kT, kFewTiles>, Rc.wtot, Rc, F, recs, B);
+        if (L.tiles <= kFewTiles) launch("k_prepare", k_prepare<kT, kFewTiles>, Rc.wtot, Rc, F, recs, B);
         else if (L.tiles <= kManyTiles)
             amh::launch_timed("k_prepare", k_prepare<1024, kManyTiles>, dim3(uint32_t((Rc.wtot + 1023) / 1024)),
                               dim3(1024), 0, s, Rc, F, recs, B);
         else launch("k_prepare", k_prepare<kT, 0>, Rc.wtot, Rc, F, recs, B);
-        if (L.tiles <= kLdsTiles) {
-            launch("k_place", few ? k_place<true, true> : k_place<true, false>, Rc.wtot, recs, Rc.wtot, B);
+        if (L.tiles <= kFewTiles) {
+            launch("k_place", k_place<true>, Rc.wtot, recs, Rc.wtot, B);
         } else {
             scan::exclusive(B.taps, L.tiles, reinterpret_cast<uint32_t *>(base + L.sums),
                             reinterpret_cast<uint32_t *>(base + L.offs), B.start, s);
-            launch("k_place", k_place<false, false>, Rc.wtot, recs, Rc.wtot, B);
+            launch("k_place", k_place<false>, Rc.wtot, recs, Rc.wtot, B);
         }
     }
     const bool texture = Rc.show_blobs != 1 && Rc.show_blobs != 2;
