@@ -70,49 +70,35 @@ __device__ __forceinline__ float gelu_and_d(float z, float &d) {
     return z * cdf;
 }
 
-template <class T> __device__ __forceinline__ uint16_t load_bf16(const T *p);
-template <> __device__ __forceinline__ uint16_t load_bf16<float>(const float *p) { return to_bf16(*p); }
-template <> __device__ __forceinline__ uint16_t load_bf16<uint16_t>(const uint16_t *p) { return *p; }
-
-// ------------------------------------------------------------------ GEMM
-// Block tile 64 x 64 (2 x 2 waves of 32 x 32), K staged 32 at a time in LDS
-// as bfloat16: As[m][k] and Bs[n][k] so each lane's MFMA operand is 16
-// contiguous bytes.  MFMA 32x32x16 operands: lane l holds row/column l % 32
+// ---------------------------------------------------------- plain product
+// c[M][N] = a[M][K] b[K][N], operands rounded to bfloat16, FP32 out: for
+// amh_mlp_gemm_test alone, which pins the operand and accumulator layout of the
+// 32x32x16 instruction that k_mlp_fused rests on.  Block tile 64 x 64 (2 x 2
+// waves of 32 x 32), K staged 32 at a time in LDS as As[m][k] and Bs[n][k], so
+// each lane's operand is 16 contiguous bytes: lane l holds row/column l % 32
 // and k = 8 * (l / 32) + 0..7; the accumulator's register r of lane l is
 // row 8 * (r / 4) + 4 * (l / 32) + r % 4, column l % 32.
 constexpr int kBM = 64, kBN = 64, kBK = 32, kPadK = kBK + 8;
 
-struct Gemm {
-    int M, N, K;
-    int64_t sam, sak;  // A(m, k) = a[m * sam + k * sak]
-    int64_t sbk, sbn;  // B(k, n) = b[k * sbk + n * sbn]
-    int ksplit;        // K per blockIdx.z
-};
-
-template <class TB, class Epi>
-__global__ __launch_bounds__(256) void k_gemm(const float *__restrict__ a, const TB *__restrict__ b, Gemm g, Epi epi) {
+__global__ __launch_bounds__(256) void k_gemm(const float *__restrict__ a, const float *__restrict__ b,
+                                              float *__restrict__ c, int M, int N, int K) {
     __shared__ __attribute__((aligned(16))) uint16_t As[kBM][kPadK];
     __shared__ __attribute__((aligned(16))) uint16_t Bs[kBN][kPadK];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.x * kBM, n0 = blockIdx.y * kBN;
-    const int kb = blockIdx.z * g.ksplit, ke = min(g.K, kb + g.ksplit);
     floatx16 acc;
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    const int sr = t >> 2, sk = (t & 3) * 8;  // staging: row sr, k sk..sk+7
-    for (int k0 = kb; k0 < ke; k0 += kBK) {
-        {
-            const int m = m0 + sr;
-            alignas(16) uint16_t va[8], vb[8];
-            for (int j = 0; j < 8; ++j) {
-                const int k = k0 + sk + j;
-                va[j] = (m < g.M && k < ke) ? load_bf16(a + m * g.sam + k * g.sak) : uint16_t(0);
-                const int n = n0 + sr;
-                vb[j] = (n < g.N && k < ke) ? load_bf16(b + k * g.sbk + n * g.sbn) : uint16_t(0);
-            }
-            *reinterpret_cast<uint4 *>(&As[sr][sk]) = *reinterpret_cast<const uint4 *>(va);
-            *reinterpret_cast<uint4 *>(&Bs[sr][sk]) = *reinterpret_cast<const uint4 *>(vb);
+    const int sr = t >> 2, sk = (t & 3) * 8, m = m0 + sr, n = n0 + sr;  // staging: row sr, k sk..sk+7
+    for (int k0 = 0; k0 < K; k0 += kBK) {
+        alignas(16) uint16_t va[8], vb[8];
+        for (int j = 0; j < 8; ++j) {
+            const int k = k0 + sk + j;
+            va[j] = (m < M && k < K) ? to_bf16(a[int64_t(m) * K + k]) : uint16_t(0);
+            vb[j] = (n < N && k < K) ? to_bf16(b[int64_t(k) * N + n]) : uint16_t(0);
         }
+        *reinterpret_cast<uint4 *>(&As[sr][sk]) = *reinterpret_cast<const uint4 *>(va);
+        *reinterpret_cast<uint4 *>(&Bs[sr][sk]) = *reinterpret_cast<const uint4 *>(vb);
         __syncthreads();
         for (int ks = 0; ks < kBK; ks += 16) {
             const int kk = ks + 8 * (lane >> 5);
@@ -125,20 +111,8 @@ __global__ __launch_bounds__(256) void k_gemm(const float *__restrict__ a, const
     const int col = n0 + wn * 32 + (lane & 31);
     for (int r = 0; r < 16; ++r) {
         const int row = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row < g.M && col < g.N) epi(row, col, acc[r]);
+        if (row < M && col < N) c[int64_t(row) * N + col] = acc[r];
     }
-}
-
-// epilogues
-struct EpiStore {  // c[row][col] = v
-    float *c;
-    int ld;
-    __device__ void operator()(int row, int col, float v) const { c[int64_t(row) * ld + col] = v; }
-};
-template <class TB, class Epi>
-void gemm(const float *a, const TB *b, const Gemm &g, const Epi &epi, int splits, hipStream_t s) {
-    dim3 grid(uint32_t((g.M + kBM - 1) / kBM), uint32_t((g.N + kBN - 1) / kBN), uint32_t(splits));
-    hipLaunchKernelGGL((k_gemm<TB, Epi>), grid, dim3(256), 0, s, a, b, g, epi);
 }
 
 // ------------------------------------------------------- training images
@@ -824,13 +798,12 @@ extern "C" int amh_mlp_adam_step(void *mlp, float lr, void *stream) {
     return AMH_OK;
 }
 
-// Plain product for tests of the matrix-core kernel: c[M][N] = a[M][K] b[K][N]
-// (FP32 row-major in, bfloat16 rounding of both operands, FP32 out).
+// Plain product for the test of the matrix instruction's layouts (k_gemm).
 extern "C" int amh_mlp_gemm_test(const float *a, const float *b, float *c, int32_t M, int32_t N, int32_t K,
                                  void *stream) {
     if (!a || !b || !c || M <= 0 || N <= 0 || K <= 0) { set_error("amh_mlp_gemm_test: invalid argument"); return AMH_E_ARG; }
-    Gemm g{M, N, K, K, 1, N, 1, ((K + kBK - 1) / kBK) * kBK};
-    gemm(a, b, g, EpiStore{c, N}, 1, static_cast<hipStream_t>(stream));
+    hipLaunchKernelGGL(k_gemm, dim3(uint32_t((M + kBM - 1) / kBM), uint32_t((N + kBN - 1) / kBN)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), a, b, c, M, N, K);
     AMH_LAUNCH_CHECK("amh_mlp_gemm_test");
     return AMH_OK;
 }

@@ -405,8 +405,9 @@ int amh_mlp_gradients(void *mlp, const float *x_dev, const float *t_dev, int32_t
                       float *loss_dev, void *stream);
 /* One Adam step (beta 0.9 / 0.999, eps 1e-8) with the last gradients. */
 int amh_mlp_adam_step(void *mlp, float lr, void *stream);
-/* c_dev[M][N] = a_dev[M][K] . b_dev[K][N] through the MLP's matrix-core
- * kernel (FP32 row-major in and out, bfloat16 operands). */
+/* c_dev[M][N] = a_dev[M][K] . b_dev[K][N] on the matrix cores (FP32 row-major
+ * in and out, bfloat16 operands), for tests: training and inference have
+ * kernels of their own. */
 int amh_mlp_gemm_test(const float *a_dev, const float *b_dev, float *c_dev, int32_t M, int32_t N, int32_t K,
                       void *stream);
 

@@ -35,8 +35,10 @@ def _mlp(batch, params=None):
 @pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 50, 40), (256, 128, 128), (128, 2, 128), (33, 128, 8),
                                    (128, 128, 3000)])
 def test_gemm_matches_bf16_product(M, N, K):
-    """The matrix-core tile kernel (operand lane layout, accumulator layout,
-    edges) against numpy on bfloat16-rounded operands."""
+    """The matrix instruction's operand and accumulator layouts, which the fused
+    forward rests on, in a plain tiled product (edges too) against numpy on
+    bfloat16-rounded operands.  The engine's own products are compared with the
+    oracle below: the forward's, and the training step's layer by layer."""
     rng = np.random.default_rng(M * 7 + N + K)
     a = rng.normal(0, 1, (M, K)).astype(np.float32)
     b = rng.normal(0, 1, (K, N)).astype(np.float32)
