@@ -13,14 +13,17 @@ from tests import gpu_util as G
 pytestmark = pytest.mark.gpu
 
 
-def test_ingest_hsp_exhaustive():
-    """Every 24-bit colour through rgb_to_hsp and back (FP64 on the GPU with
-    the reference's operation order) equals the oracle, which equals the
-    compiled reference."""
+@pytest.mark.parametrize("absent", [0, 97])
+def test_ingest_hsp_exhaustive(absent):
+    """Every 24-bit colour through rgb_to_hsp and back equals the oracle, which
+    equals the compiled reference: in float where the 8-bit rounding is clear
+    and in FP64 in the reference's operation order where it is not.  Once with
+    every colour present, once with every 97th pixel absent."""
     T = G.torch()
     lib = G.lib()
     words = (np.arange(1 << 24, dtype=np.uint32) | np.uint32(0xFF000000))
-    words[::97] &= np.uint32(0x00FFFFFF)  # some absent pixels (alpha 0)
+    if absent:
+        words[::absent] &= np.uint32(0x00FFFFFF)  # (alpha 0)
     st_w, sh_w = op.ingest(words, 1)
     src = G.to_dev(words)
     st = G.zeros(words.size, T.int32)
@@ -178,6 +181,35 @@ def test_dithered_frames_around_tile_edges(w, h, cover):
     for b in range(0, nb, max(1, nb // 50)):
         m = want[idx] == b
         assert (s[b].x1, s[b].y1, s[b].x2, s[b].y2) == (x[m].min(), y[m].min(), x[m].max(), y[m].max())
+
+
+def test_blob_numbers_of_a_frame_beyond_the_summing_blocks():
+    """4096 x 2049 pixels, 8,196 blocks of 1,024: from 8,192 on the blocks'
+    counts are scanned instead of summed by every block.  Count, numbers and
+    statistics are those of the oracle's labels; the last pixel is a blob."""
+    T, lib, w, h = G.torch(), G.lib(), 4096, 2049
+    rng = np.random.default_rng(8)
+    fr = np.zeros((h, w, 4), np.uint8)
+    fr[rng.uniform(size=(h, w)) < 0.002] = (10, 200, 30, 255)
+    fr[-1, -1] = (9, 8, 7, 255)
+    G.log("blob numbers 4096x2049")
+    src, lab_d = _segment(fr)
+    lab, n = op.segment(fr)
+    assert (G.to_host(lab_d, np.int32) == lab).all()
+    ws = G.zeros(lib.amh_blob_workspace_bytes(w, h) // 4 + 1, T.int32)
+    nb = C.c_int32(0)
+    G.check(lib.amh_blob_count(G.dptr(lab_d), w, h, G.dptr(ws), C.byref(nb), G.stream()), "count")
+    roots = np.flatnonzero(lab == np.arange(lab.size))
+    assert nb.value == n == roots.size and lab[-1] >= 0
+    bop = G.zeros(h * w, T.int32)
+    st = T.zeros(n * C.sizeof(A.BlobStat), dtype=T.uint8, device="cuda")
+    G.check(lib.amh_blob_stats(G.dptr(lab_d), G.dptr(src), w, h, G.dptr(ws), n, G.dptr(bop), G.dptr(st), G.stream()),
+            "stats")
+    want = np.where(lab >= 0, np.searchsorted(roots, lab), -1)
+    assert (G.to_host(bop, np.int32) == want).all()
+    stats = (A.BlobStat * n).from_buffer_copy(st.cpu().numpy().tobytes())
+    assert [s.first for s in stats] == roots.tolist()
+    assert [s.count for s in stats] == np.bincount(want[want >= 0], minlength=n).tolist()
 
 
 def _group(bop_host, nb):
