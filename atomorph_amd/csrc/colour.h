@@ -92,10 +92,15 @@ __host__ __device__ inline uint32_t hsp_to_rgb(uint32_t c) {
 
 // The same two in float, for a colour whose channels all land further than
 // kClear from where the 8-bit rounding turns; false where one does not (about
-// 1 colour in 30, mostly exact ties), and the double-precision form above decides.  Float is off
-// by at most half of kClear: whole numbers up to 255 in, no differences of
-// rounded terms, and at most ten roundings of 2^-24 of values up to 255.  The
-// colours are few enough that all of them are compared.
+// 1 colour in 30, mostly exact ties), and the double-precision form above
+// decides.  Float has to be off by less than kClear = 2.4e-4.  Whole numbers up
+// to 255 go in and no rounded terms are subtracted; a rounding is 2^-24 of its
+// value, a reciprocal or root (v_rcp, v_rsq, v_sqrt) one ulp, 2^-23.  On the way
+// to HSP that comes to 6e-5 at most (P's root).  On the way back the middle
+// channel, through three of those and ten roundings, could reach 2.5e-4 if all
+// were at their worst and added up; so a test compares the two with the
+// double-precision form for every RGB colour and the HSP word it gives, which
+// is all that ingest converts.
 //
 // Measured on one MI355X, 2048x2048 pixels, 36% opaque, both ways: 52 -> 26 us.
 // In double precision the dozen divisions and two roots of a pixel bound it.

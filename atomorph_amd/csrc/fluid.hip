@@ -238,10 +238,11 @@ __device__ __forceinline__ void toward(double x1, double y1, double x2, double y
 // The grid's nodes are owned by kTile x kTile tiles.  Each step every active
 // particle is binned into each tile that holds a node of its 3x3 stencil (1,
 // 2 or 4 tiles; a counting sort of slot numbers).  The block of a tile reads
-// its bin,
-// sums what those particles add to its nodes in LDS and stores every node
-// once.  No phase of the step uses a global atomic (device-wide atomics are
-// performed past the per-XCD L2) and no phase needs the grid cleared first.
+// its bin, sums what those particles add to its nodes in LDS and stores every
+// node once, so that no phase needs the grid cleared first.  Device-wide
+// atomics are performed past the per-XCD L2, so they are few: one per bin
+// and wave for the counts, one per 128 tiles for the work items' places, and
+// the node sums of tiles too full for one work item.
 constexpr int kTile = 8;
 constexpr int kReach = kTile + 2;  // cells per axis that reach a tile's nodes
 
@@ -251,7 +252,7 @@ struct Bins {
     int32_t *start;     // [tiles + 1]
     int32_t *rank;      // [4][n]: place of particle i's j-th entry in its bin
     int32_t *list;      // [<= 4n] slots, grouped by bin
-    int32_t item;         // entries of a work item at most, one per thread
+    int32_t item;       // entries of a work item at most, one per thread
     // Work items of `item` entries at most, each one workgroup (chunk NULL:
     // whole bins, one workgroup per tile, from start[]).  A dense bin is
     // split over several items, which add their node sums with atomics to
@@ -676,14 +677,14 @@ struct P2gItem {
 // step; without the sort a cell would be many runs.
 //
 // Instructions and LDS bound this kernel, k_forces and k_g2p.  One MI355X,
-// 229k particles on 276^2 nodes (1044^2), us: here 18.2 -> 12.4 (37 -> 18.5),
-// k_forces 12.5 -> 10.1 (26 -> 17), k_g2p 14.7 -> 11.5 (34 -> 20), before with
+// 229k particles on 276^2 nodes (1044^2), us: here 18.2 -> 12.8 (37 -> 20),
+// k_forces 12.5 -> 10.1 (26 -> 17), k_g2p 14.7 -> 10.8 (34 -> 19), before with
 // LDS atomics per run and node, sums carried across the lanes' rows and kT
 // threads on either grid.
 //
-// Six waves per SIMD (72 VGPRs): the LDS (19 KB) allows eight blocks per
-// CU; seven waves spilled when there were more registers, which measured
-// slower.
+// Six waves per SIMD (71 VGPRs, 78 of half the threads): the LDS (19 KB)
+// allows eight blocks per CU; seven waves spilled when there were more
+// registers, which measured slower.
 template <int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_p2g(Particles P, Grid Gd, int gsx,
                                                                                    int gsy, Bins B) {
@@ -1421,6 +1422,8 @@ namespace {
 // workgroup idles at kT (229k particles on 1044^2 nodes, 13 per tile: four
 // frames 3.9 ms at kT, 3.7 at kT / 2); the denser grids fill kT and would be
 // split, and added with atomics, twice as often (276^2 nodes, 187 per tile).
+// Around the line the two are alike: of 276^2 nodes a step takes 81 us with 63
+// and 64 particles per tile, 82 with 65; of 500^2 184 and 187, and 189.
 size_t item_size(size_t tiles, size_t n) { return n > 64 * tiles ? kT : kT / 2; }
 
 // Upper bound of the chunks: every tile has at least one, and a particle
@@ -1720,8 +1723,8 @@ int fluid_step_on(amh_fluid_s *f, const Particles &Q, const int32_t *atom, int32
     const int par = f->bin_par;
     f->bin_par ^= 1;
     B.par = par;
-    // about one work item per workgroup (a bin averages under one chunk of
-    // kT entries, and empty tiles get none); a workgroup takes further items
+    // about one work item per workgroup (a bin averages under one item's
+    // entries, and empty tiles get none); a workgroup takes further items
     // when there are more
     const uint32_t grid = uint32_t(std::min(B.max_chunks, 2 * std::min(tiles, kLdsTiles)));
     {

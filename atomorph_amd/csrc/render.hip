@@ -23,8 +23,8 @@
 // the L2: with five of them per tap into per-pixel accumulators in memory
 // (and a second, scanned list for the other blobs of a pixel) a frame took
 // 1,518 us at 2048^2 with 1.7 M atoms, 261 us at 1001 x 777 with feather 2;
-// in tiles it takes 212 and 90 us (kernels at 2048^2: prepare 108, place 35,
-// splat 78 us).
+// in tiles it takes 207 and 70 us (kernels at 2048^2: prepare 88, the scan of
+// the counts 9, place 36, splat 73 us).
 #include <mutex>
 #include <type_traits>
 
@@ -43,7 +43,7 @@ constexpr int kT = 256;
 constexpr int kTile = 16;             // pixels per side of an image tile
 constexpr int kTilePx = kTile * kTile;  // one thread of the splat per pixel
 static_assert(kTilePx == kT, "one thread per pixel");
-constexpr int kFewTiles = 4096;       // up to this many tiles blocks count, scan and place atoms per tile in LDS
+constexpr int kFewTiles = 4096;       // up to this many tiles blocks count, scan and place atoms per tile in LDS (k_place)
 constexpr int kManyTiles = 16384;     // up to this many, larger blocks count them there
 constexpr int kNoBlob = 0x7FFFFFFF;
 // The tiles' lists are indexed by 32-bit sums of the atoms' taps, four of an
@@ -86,8 +86,10 @@ __device__ __forceinline__ int tile_of(uint32_t x, uint32_t y, int j, int ntx) {
 // tile (TILES = 0, one atomic per distinct tile) takes up to 64 turns, and on
 // few tiles the atomics queue at the same counters.  11,000 atoms on 70
 // tiles: 17.8 us grouped, 4.9 in LDS; 300,000 on 3,087: 21.7 and 10; 1.7 M on
-// 16,384: 110 and 90, in blocks of 1,024 that share the 32 KB.  Beyond that
-// too few blocks fit a CU.
+// 16,384: 110 and 90, in blocks of 1,024 that share the 32 KB.  A row of tiles
+// further 1.7 M atoms take 82 us grouped against 70 here where neighbours lie
+// together, 140 against 117 scattered; counters for more tiles than that in LDS
+// have not been measured.
 template <int NT, int TILES>
 __global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__restrict__ recs, Tiles B) {
     __shared__ PerlinTab tab;
@@ -178,6 +180,11 @@ __global__ __launch_bounds__(NT) void k_prepare(amh_render R, Frame F, Rec *__re
 // exact).  kFew: every block scans the tap counts in LDS (block 0 stores the
 // starts) and takes ranks within the block from LDS counters, as in k_prepare;
 // otherwise B.start holds the scan already and a wave's lanes are grouped.
+// (With the counting in LDS, eight 64^2 frames 239 -> 191 us, a frame of 3,087
+// tiles 94 -> 65.)  Every block scans all tiles, so that this loses before its
+// limit: of 4,096 tiles and of 4,225 (and two launches of 4.6 us for the scan)
+// 300,000 neighbouring atoms take 24 and 7 us, scattered ones 66 and 43; 1.7 M
+// neighbouring ones 104 and 22, scattered ones 185 and 209.
 template <bool kFew>
 __global__ __launch_bounds__(kT) void k_place(const Rec *__restrict__ recs, int64_t n, Tiles B) {
     const int64_t a = int64_t(blockIdx.x) * kT + threadIdx.x;
@@ -508,10 +515,12 @@ __device__ __forceinline__ void tile_blobs(Sums &acc, int *bcur, int *bnext, con
 // One workgroup per tile, one thread per pixel.  A tile's loads are one
 // dependent chain (counters, list, atoms), so each mode holds only the
 // registers it needs and eight workgroups fit a CU; then the LDS atomics and
-// the tap arithmetic bound it.  Hence the packed sums, and the single pass
-// over a tile whose atoms are all of one blob (most covered tiles): 109 us at
-// 2048^2 with 110 registers and five sums, 94 with 54 registers, 78 with
-// these.  Leaves the tile's counters at zero for the next frame.
+// the tap arithmetic bound it.  Hence the packed sums, and with them the single
+// pass over a tile whose atoms are all of one blob: 109 us at 2048^2 with 110
+// registers and five sums, 94 with 54 registers, 73 with these.  They serve
+// blobs' rims, sparse blobs and frames in motion; a tile filled by a blob at
+// rest holds 256 atoms and more, and takes the wide sums in two passes.
+// Leaves the tile's counters at zero for the next frame.
 enum SplatMode {
     kPlain,    // no background, no blending
     kOver,     // over the background, or blending
