@@ -232,7 +232,9 @@ __device__ __forceinline__ void run_rounds(uint2 *P, int2 *S, uint32_t *cs, int 
             pairs += npairs;
             c = __builtin_amdgcn_readfirstlane(next);
             if (NT > 64) __syncthreads();
-            else wave_order();
+            // (one wave: the compiler keeps each lane's order, since any slot may be
+            // any other; wave_order() here made visits 1 to 3% slower)
+            else __builtin_amdgcn_wave_barrier();
         }
         att += pairs;
         acc += swaps;
